@@ -13,12 +13,11 @@
 //
 // Data layout: atoms are binned into x-y columns of about one cluster width and
 // fine z bins, counting-sorted, and cut per column into clusters of 32
-// consecutive atoms (padded).  Cluster arrays (TC4 x, y, z, q and TC2 sigma/2,
-// sqrt(eps)) are cluster-major, 32 slots per cluster.  Cluster pairs within
-// the list cutoff (bounding-box test) are found per column neighbourhood; the
-// pair kernel gives each 64-lane wavefront one 32 x 32 tile at a time: lane l
-// owns i-slot l & 31 and half l >> 5 of the j-slots, which rotate through the
-// tile so that every j accumulator in LDS is written by one lane per step.
+// consecutive atoms (padded), each ordered into four compact groups of 8 slots.  Cluster arrays (TC4 x,
+// y, z, q and TC2 sigma/2, 2 sqrt(eps)) are cluster-major, 32 slots per cluster.  Per i-cluster a list of
+// the 8-atom j-groups within the cutoff of one of its groups is found per column neighbourhood; the
+// pair kernel gives each 64-lane wavefront a share of one cluster's list, four entries at a time, one
+// lane per pair of an 8 x 8 block.
 // Forces and energies accumulate as int64 fixed point (bitwise independent of
 // the order of summation); the reciprocal-space energy is a float64 k-space sum.
 // TC = float is the mixed-precision mode, TC = double the all-float64 mode.
@@ -42,9 +41,15 @@ using namespace tffpme;
 constexpr int CL = 32;          // atoms per cluster
 constexpr int MAXEX = 8;        // exclusion partners per atom kept for the tile masks
 constexpr int FB = 256;         // block size of the per-atom kernels
-constexpr int TILE_BLOCK = 256; // 4 waves
-constexpr int TILE_WAVES = TILE_BLOCK / TFF_WAVE;
-constexpr int E_SLOTS = 64;  // fixed-point energy slots per term
+// Fixed-point sums over a whole call go to up to E_SLOTS slots of one 64-byte line each (words: Lennard-Jones,
+// Coulomb, listed cluster pairs), added up by the last kernel: same-line atomics serialise at about
+// 6 ns each, so a few shared lines cost more than the waves that add to them compute.
+constexpr int E_SLOTS = 512;
+struct ESlots {
+  unsigned long long* p;
+  int n;
+  __device__ __forceinline__ unsigned long long* line(int k) const { return p + 8 * (long long)(k % n); }
+};
 constexpr double F_SCALE = 4294967296.0;        // 2^32: forces and energies (kJ/mol, nm)
 constexpr double Q_SCALE = 1099511627776.0;     // 2^40: PME charge grid
 // padding slots sit at x = PAD_STEP (1 + slot), y = z = PAD_STEP: every padding slot is more
@@ -209,12 +214,13 @@ __device__ __forceinline__ int column_bucket(unsigned long long key, float scale
 template <typename TI>
 __global__ __launch_bounds__(SORT_THREADS) void k_sort_columns(const TI* __restrict__ coords, Geo g,
                                                                const int* __restrict__ col_start,
-                                                               int* __restrict__ sorted_orig) {
+                                                               int* __restrict__ sorted_orig, ESlots es) {
   static_assert(COL_BUCKETS <= 8 * SORT_THREADS, "column sort: eight buckets per thread at most");
   __shared__ unsigned long long s_k[COL_SORT_MAX];
   __shared__ int s_c[COL_BUCKETS];
   __shared__ int s_tot[SORT_THREADS / TFF_WAVE], s_max[SORT_THREADS / TFF_WAVE];
   const int col = blockIdx.x;
+  for (int k = col * SORT_THREADS + threadIdx.x; k < 8 * es.n; k += gridDim.x * SORT_THREADS) es.p[k] = 0ull;
   const int cs = col_start[col], m = col_start[col + 1] - cs;
   if (m <= 1 || m > COL_SORT_MAX) return;
   const int t = threadIdx.x, lane = t & (TFF_WAVE - 1), wv = t / TFF_WAVE;
@@ -457,58 +463,131 @@ __global__ __launch_bounds__(FB) void k_fill_exclusions(const int* __restrict__ 
   for (; k < MAXEX; ++k) excl_part[sl * MAXEX + k] = -1;
 }
 
-// ---------------------------------------------------------------- 3. cluster pairs
-// Cluster-pair entries are (ci, cj, info) with cj >= ci; info packs
-//   bits  0..15  sub-tile mask: bit gi * 4 + gj set when groups gi of ci and gj of cj have
-//                bounding boxes within the list cutoff (diagonal tiles: gj >= gi only)
-//   bits 16..21  periodic shift k_a + 1 (2 bits per axis): x_j + k L is the image of cluster
+// ---------------------------------------------------------------- 3. pair list
+// Per i-cluster ci a list of entries, one per 8-atom j-group that has at least one group of ci within
+// the cutoff: eg = the j-group (cj * 4 + gj, cj >= ci) and ei =
+//   bits  0..3   bit gi set when groups gi of ci and gj of cj have bounding boxes within the
+//                interaction cutoff (diagonal tiles: gi <= gj only)
+//   bits  4..9   periodic shift k_a + 1 (2 bits per axis): x_j + k L is the image of cluster
 //                cj closest to cluster ci
-//   bit  22      the tile holds excluded pairs
-//   bit  23      the shift is not the minimum image of every atom pair of the tile (small
-//                boxes): the pair kernel then takes the minimum image per pair
-//   bit  24      always set
-// The sub-tile masks are filled in by k_compact_pairs; entries whose mask stays empty are
-// skipped by the pair kernel.
-constexpr unsigned INFO_EXCL = 1u << 22;
-constexpr unsigned INFO_MINIMG = 1u << 23;
-constexpr unsigned INFO_LISTED = 1u << 24;  // set for every entry (so that info != 0)
+//   bit  10      the j-group holds exclusion partners of ci, or belongs to ci itself
+//   bit  11      the shift is not the minimum image of every atom pair of the two clusters (small
+//                boxes): the pair kernels then take the minimum image per pair
+// The 4 * maxn entries of a cluster are filled from both ends: cluster pairs without bits 10 and 11 from
+// the front (cnt.x entries, the pair's non-empty j-groups), the others from the back (cnt.y quads, the
+// pair's four j-groups each, info 0 where empty).  The pair kernels sum a cluster pair's energies in
+// TC before they go on in double; a quad of its own keeps a pair with (large) exclusion terms, or of
+// a small box, in one piece, whatever the share of the list that a wave takes.
+constexpr unsigned ENT_EXCL = 1u << 10;
+constexpr unsigned ENT_MINIMG = 1u << 11;
 
-// One wave per i-cluster; lanes sweep the clusters of the neighbouring columns in a fixed
-// order and write the accepted j-clusters into the i-cluster's own segment.
-__global__ __launch_bounds__(FB) void k_cluster_pairs(const int* __restrict__ ncl_ptr, const int* __restrict__ cl_col,
-                                                      const int* __restrict__ col_cl_start,
-                                                      const float4* __restrict__ bb_c,
-                                                      const float4* __restrict__ bb_h, Geo g, float rlist2,
-                                                      const int* __restrict__ excl_part,
-                                                      int2* __restrict__ seg, int* __restrict__ seg_count,
-                                                      int* __restrict__ status) {
+struct PairList {
+  int* g;             // j-groups, 4 * maxn per i-cluster
+  unsigned short* i;  // their info
+  int2* cnt;          // per i-cluster
+  int cap;            // 4 * maxn
+};
+
+// One wave per i-cluster.  The lanes sweep the clusters of the neighbouring columns in a fixed order;
+// clusters within the list cutoff collect in LDS, and whenever 64 are waiting (and at the end) each
+// lane takes one of them, tests its 16 pairs of groups and the wave appends the entries (one ballot
+// per j-group).  The order is fixed, so the list is the same on every call.
+__global__ __launch_bounds__(FB) void k_pair_list(const int* __restrict__ ncl_ptr, const int* __restrict__ cl_col,
+                                                  const int* __restrict__ col_cl_start,
+                                                  const float4* __restrict__ bb_c, const float4* __restrict__ bb_h,
+                                                  const float4* __restrict__ sb_c, const float4* __restrict__ sb_h,
+                                                  Geo g, float rlist2, float cut2, const int* __restrict__ excl_part,
+                                                  PairList pl, ESlots es,
+                                                  int* __restrict__ status) {
   __shared__ int s_xp[FB / TFF_WAVE][CL * MAXEX];
   __shared__ int s_off[FB / TFF_WAVE][2 * TFF_WAVE], s_cs[FB / TFF_WAVE][2 * TFF_WAVE];
+  __shared__ int2 s_tile[FB / TFF_WAVE][2 * TFF_WAVE];
   const int lane = threadIdx.x & (TFF_WAVE - 1);
   const int w = threadIdx.x / TFF_WAVE;
-  const int ci = blockIdx.x * (FB / TFF_WAVE) + w;
+  const int ci = __builtin_amdgcn_readfirstlane(blockIdx.x * (FB / TFF_WAVE) + w);
   const int ncl = *ncl_ptr;
   if (ci >= ncl) return;
-  // clusters (other than ci) holding an exclusion partner of an atom of ci, compacted in LDS
+  const unsigned long long below = (1ull << lane) - 1ull;
+  // j-groups (of clusters other than ci) holding an exclusion partner of an atom of ci, compacted in LDS
   int nxp = 0;
   for (int k = 0; k < MAXEX; ++k) {
-    int v = lane < CL ? excl_part[(ci * CL + lane) * MAXEX + k] : -1;
-    int pc = v >= 0 ? (v >> 5) : -1;
-    bool keep = pc >= 0 && pc != ci;
-    unsigned long long m = __ballot(keep);
-    if (keep) s_xp[w][nxp + __popcll(m & ((1ull << lane) - 1ull))] = pc;
+    const int v = lane < CL ? excl_part[(ci * CL + lane) * MAXEX + k] : -1;
+    const bool keep = v >= 0 && (v >> 5) != ci;
+    const unsigned long long m = __ballot(keep);
+    if (keep) s_xp[w][nxp + __popcll(m & below)] = v >> 3;
     nxp += __popcll(m);
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  tff_wave_sync_lds();
   const int col = cl_col[ci];
   const int cx = col / g.ncol[1], cy = col % g.ncol[1];
   const float4 c0v = bb_c[ci], h0 = bb_h[ci];
+  float4 gc[4], gh[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    gc[k] = sb_c[ci * 4 + k];
+    gh[k] = sb_h[ci * 4 + k];
+  }
   const float Lv[3] = {(float)g.L[0], (float)g.L[1], (float)g.L[2]};
   const float iLv[3] = {(float)g.invL[0], (float)g.invL[1], (float)g.invL[2]};
-  int nseg = 0;
-  int2* my = seg + (long long)ci * g.maxn;
+  int nseg = 0;                    // clusters within the list cutoff
+  int nwait = 0;                   // of them in s_tile
+  int nfront = 0, nback = 0;       // entries from the front, quads from the back
+  const long long ebase = (long long)ci * pl.cap;
+  // the first n waiting clusters -> entries
+  auto emit = [&](int n) {
+    int cj = 0;
+    unsigned info = 0, bits = 0;
+    if (lane < n) {
+      const int2 e = s_tile[w][lane];
+      cj = e.x;
+      info = (unsigned)e.y;
+#pragma unroll
+      for (int gj = 0; gj < 4; ++gj) {
+        const float4 c1 = sb_c[cj * 4 + gj], h1 = sb_h[cj * 4 + gj];
+#pragma unroll
+        for (int gi = 0; gi < 4; ++gi) {
+          float dx = gc[gi].x - c1.x, dy = gc[gi].y - c1.y, dz = gc[gi].z - c1.z;
+          // minimum image of the group centres: a lower bound on the distance of every image
+          dx -= Lv[0] * rintf(dx * iLv[0]);
+          dy -= Lv[1] * rintf(dy * iLv[1]);
+          dz -= Lv[2] * rintf(dz * iLv[2]);
+          const float gx = fmaxf(fabsf(dx) - gh[gi].x - h1.x, 0.f);
+          const float gy = fmaxf(fabsf(dy) - gh[gi].y - h1.y, 0.f);
+          const float gz = fmaxf(fabsf(dz) - gh[gi].z - h1.z, 0.f);
+          if (gh[gi].x >= 0.f && h1.x >= 0.f && (ci != cj || gj >= gi) && gx * gx + gy * gy + gz * gz <= cut2)
+            bits |= 1u << (gj * 4 + gi);
+        }
+      }
+    }
+    unsigned xg = cj == ci ? 15u : 0u;  // j-groups that need the exclusion tests
+    for (int t = 0; t < nxp; ++t) {
+      const int p = s_xp[w][t];
+      xg |= (p >> 2) == cj ? 1u << (p & 3) : 0u;
+    }
+    unsigned nib_any = 0;
+#pragma unroll
+    for (int gj = 0; gj < 4; ++gj) nib_any |= (bits >> (4 * gj)) & 15u ? 1u << gj : 0u;
+    const bool back = nib_any && (xg || (info & ENT_MINIMG));
+    const int nf = back ? 0 : __popc(nib_any);
+    int kf = nfront;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const unsigned long long mf = __ballot((nf >> p) & 1);
+      kf += __popcll(mf & below) << p;
+      nfront += __popcll(mf) << p;
+    }
+    const unsigned long long mb = __ballot(back);
+    const int kb = pl.cap - 4 * (nback + __popcll(mb & below)) - 4;
+    nback += __popcll(mb);
+#pragma unroll
+    for (int gj = 0; gj < 4; ++gj) {
+      if (!back && !((nib_any >> gj) & 1u)) continue;  // (back: the empty ones too, with info 0)
+      const int k = back ? kb + gj : kf++;
+      const unsigned nib = (bits >> (4 * gj)) & 15u;
+      pl.g[ebase + k] = cj * 4 + gj;
+      pl.i[ebase + k] = (unsigned short)(nib ? info | ((xg >> gj) & 1u ? ENT_EXCL : 0u) | nib : 0u);
+    }
+  };
   const int nx = 2 * g.reach[0] + 1 >= g.ncol[0] ? g.ncol[0] : 2 * g.reach[0] + 1;
   const int ny = 2 * g.reach[1] + 1 >= g.ncol[1] ? g.ncol[1] : 2 * g.reach[1] + 1;
   const int x0 = nx == g.ncol[0] ? 0 : cx - g.reach[0];
@@ -592,14 +671,13 @@ __global__ __launch_bounds__(FB) void k_cluster_pairs(const int* __restrict__ nc
     s_cs[w][2 * lane] = r0s;
     s_off[w][2 * lane + 1] = incl - cnt + r0n;
     s_cs[w][2 * lane + 1] = r1s;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    tff_wave_sync_lds();
     const int nvalid = 2 * (ncc - c0 < TFF_WAVE ? ncc - c0 : TFF_WAVE);
     for (int b = 0; b < total; b += TFF_WAVE) {
       const int k = b + lane;
       unsigned info = 0;
       int cj = -1;
+      bool ok = false;
       if (k < total) {
         // last range whose offset is <= k (offsets are non-decreasing; an empty range shares its
         // offset with the next one, which then holds k)
@@ -622,143 +700,122 @@ __global__ __launch_bounds__(FB) void k_cluster_pairs(const int* __restrict__ nc
           const float gp = fmaxf(fabsf(dm) - hs[a], 0.f);
           gap2 += gp * gp;
           minimg = minimg || !(fabsf(dm) + hs[a] <= 0.49999f * Lv[a]);
-          shift |= (unsigned)((int)kk + 1) << (16 + 2 * a);
+          shift |= (unsigned)((int)kk + 1) << (4 + 2 * a);
         }
-        if (gap2 <= rlist2) info = shift | (minimg ? INFO_MINIMG : 0u) | INFO_LISTED;
+        ok = gap2 <= rlist2;
+        info = shift | (minimg ? ENT_MINIMG : 0u);
       }
-      const bool ok = info != 0;
-      unsigned long long bm = __ballot(ok);
-      if (ok) {
-        bool xf = cj == ci;
-        for (int t = 0; t < nxp; ++t) xf = xf || s_xp[w][t] == cj;
-        int kk = nseg + __popcll(bm & ((1ull << lane) - 1ull));
-        if (kk < g.maxn) my[kk] = make_int2(cj, (int)(info | (xf ? INFO_EXCL : 0u)));
+      const unsigned long long bm = __ballot(ok);
+      const int r = __popcll(bm & below);
+      // over the capacity (flagged below) the rest is dropped
+      if (ok && nseg + r < g.maxn) s_tile[w][nwait + r] = make_int2(cj, (int)info);
+      const int room = g.maxn - nseg, got = __popcll(bm);
+      nwait += got < room ? got : (room > 0 ? room : 0);
+      nseg += got;
+      tff_wave_sync_lds();
+      if (nwait >= TFF_WAVE) {
+        emit(TFF_WAVE);
+        nwait -= TFF_WAVE;
+        const int2 tail = s_tile[w][TFF_WAVE + lane];
+        tff_wave_sync_lds();
+        s_tile[w][lane] = tail;
+        tff_wave_sync_lds();
       }
-      nseg += __popcll(bm);
     }
     // the next group of columns rewrites s_off / s_cs
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    tff_wave_sync_lds();
   }
+  if (nwait > 0) emit(nwait);
   if (lane == 0) {
     if (nseg > g.maxn) atomicOr(status, TFF_FUSED_PAIR_OVERFLOW);
-    seg_count[ci] = nseg < g.maxn ? nseg : g.maxn;
+    atomicAdd(es.line(ci) + 2, (unsigned long long)(nseg < g.maxn ? nseg : g.maxn));
+    pl.cnt[ci] = make_int2(nfront, nback);
   }
 }
 
-// exclusive scan of the per-cluster pair counts (single workgroup), total into *ncp
-__global__ __launch_bounds__(1024) void k_scan_counts(const int* __restrict__ ncl_ptr, const int* __restrict__ cnt,
-                                                      int* __restrict__ start, int* __restrict__ ncp,
-                                                      int* __restrict__ status) {
-  const int total = tff_block_scan_1024(cnt, *ncl_ptr, start, false);  // start holds ncl entries
-  if (threadIdx.x == 0) {
-    *ncp = total;
-    status[1] = total;
-  }
-}
-
-// Segments -> one compact cluster-pair list in (ci, segment order) (deterministic), with the
-// sub-tile masks: bit gi * 4 + gj is set when the bounding boxes of group gi of ci and group
-// gj of cj are within cut2 (minimum image of the group centres: a lower bound on the distance
-// of every image of every atom pair of the two groups).  One wave per i-cluster, one lane per
-// tile (64 tiles per step): a lane loads its tile's entry, then the four group boxes of cj, and
-// forms all 16 bits itself (ci's group boxes are the same for every lane).
-__global__ __launch_bounds__(FB) void k_compact_pairs(const int* __restrict__ ncl_ptr, const int2* __restrict__ seg,
-                                                      const int* __restrict__ seg_count,
-                                                      const int* __restrict__ seg_start, int maxn,
-                                                      const float4* __restrict__ sb_c, const float4* __restrict__ sb_h,
-                                                      Geo g, float cut2, int4* __restrict__ pairs) {
-  const int lane = threadIdx.x & (TFF_WAVE - 1);
-  const int ci = (blockIdx.x * FB + threadIdx.x) / TFF_WAVE;
-  if (ci >= *ncl_ptr) return;
-  const int n = seg_count[ci], o = seg_start[ci];
-  float4 c0[4], h0[4];
-#pragma unroll
-  for (int gi = 0; gi < 4; ++gi) {
-    c0[gi] = sb_c[ci * 4 + gi];
-    h0[gi] = sb_h[ci * 4 + gi];
-  }
-  const float L0 = (float)g.L[0], L1 = (float)g.L[1], L2 = (float)g.L[2];
-  const float i0 = (float)g.invL[0], i1 = (float)g.invL[1], i2 = (float)g.invL[2];
-  for (int k = lane; k < n; k += TFF_WAVE) {
-    const int2 e = seg[(long long)ci * maxn + k];
-    const int cj = e.x;
-    unsigned bits = 0;
-#pragma unroll
-    for (int gj = 0; gj < 4; ++gj) {
-      const float4 c1 = sb_c[cj * 4 + gj], h1 = sb_h[cj * 4 + gj];
-#pragma unroll
-      for (int gi = 0; gi < 4; ++gi) {
-        if (h0[gi].x >= 0.f && h1.x >= 0.f && (ci != cj || gj >= gi)) {
-          float dx = c0[gi].x - c1.x, dy = c0[gi].y - c1.y, dz = c0[gi].z - c1.z;
-          dx -= L0 * rintf(dx * i0);
-          dy -= L1 * rintf(dy * i1);
-          dz -= L2 * rintf(dz * i2);
-          const float gx = fmaxf(fabsf(dx) - h0[gi].x - h1.x, 0.f);
-          const float gy = fmaxf(fabsf(dy) - h0[gi].y - h1.y, 0.f);
-          const float gz = fmaxf(fabsf(dz) - h0[gi].z - h1.z, 0.f);
-          if (gx * gx + gy * gy + gz * gz <= cut2) bits |= 1u << (gi * 4 + gj);
-        }
-      }
-    }
-    pairs[o + k] = make_int4(ci, cj, (int)((unsigned)e.y | bits), 0);
-  }
-}
-
-// ---------------------------------------------------------------- 4. tile kernel
-
-// sum over the 8 lanes sharing lane >> 3 (the result lands in all 8 lanes)
+// ---------------------------------------------------------------- 4. pair kernels
+// Lane maps: lane = 8 ii + jj evaluates i-slot ii of a group of ci against j-slot jj of the j-group.
+// Sums over jj (contiguous octets) are DPP adds; sums over ii (stride 8) halve with the gfx950
+// half-wave and row swaps: swapping the upper half of one value with the lower half of another and
+// adding the two leaves each half with the sum of one of them, so every exchange also scatters.
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
-__device__ __forceinline__ float octet_sum(float v) {
-  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f<0x141>(v);  // row_half_mirror
-  return v;
-}
-// float64: the same lane permutations on both 32-bit halves (VALU moves, no LDS crossbar round trip)
 template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
+__device__ __forceinline__ double dpp_f(double v) {
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
-__device__ __forceinline__ double octet_sum(double v) {
-  v += dpp_d<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_d<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_d<0x141>(v);  // row_half_mirror (every lane of a quad holds the quad's sum by now)
+// sum over the 8 lanes sharing lane >> 3 (the result lands in all 8 lanes)
+template <typename T>
+__device__ __forceinline__ T octet_sum(T v) {
+  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_f<0x141>(v);  // row_half_mirror (every lane of a quad holds the quad's sum by now)
   return v;
 }
-// sum over the 8 lanes sharing lane & 7
+// lanes 0..31: a summed over the lane pair (l, l + 32); lanes 32..63: b summed over (l - 32, l)
+__device__ __forceinline__ float half_add(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// even rows of 16 lanes: a summed over the row pair; odd rows: b summed over it
+__device__ __forceinline__ float row_add(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double join_d(unsigned lo, unsigned hi) {
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ double half_add(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  const auto l = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return join_d(l[0], h[0]) + join_d(l[1], h[1]);
+}
+__device__ __forceinline__ double row_add(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  const auto l = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return join_d(l[0], h[0]) + join_d(l[1], h[1]);
+}
+// one value of each of four entries summed over the 8 lanes sharing lane & 7: the lane gets entry
+// 2 (lane >> 5) + ((lane >> 4) & 1)'s sum (both lanes that differ in bit 3 hold it)
 template <typename T>
-__device__ __forceinline__ T stride8_sum(T v) {
-  v += __shfl_xor(v, 8, TFF_WAVE);
-  v += __shfl_xor(v, 16, TFF_WAVE);
-  v += __shfl_xor(v, 32, TFF_WAVE);
-  return v;
+__device__ __forceinline__ T quad_reduce(T f0, T f1, T f2, T f3) {
+  const T h = row_add(half_add(f0, f2), half_add(f1, f3));
+  return h + dpp_f<0x128>(h);  // row_ror:8
+}
+template <typename T>
+__device__ __forceinline__ T wave_sum_t(T v) {
+  v = octet_sum(v);
+  v += dpp_f<0x128>(v);
+  v = row_add(v, v);
+  return half_add(v, v);
 }
 
-// The 12 force components f[g][a] (k = 3 g + a) of one slot column are summed over the 8 lanes
-// that share the column (RED) and written by those 8 lanes: lane r of the eight takes values
-// r and r + 8.  The selects act on the reduced values, so the arrays stay in registers.
-template <typename T, typename RED>
-__device__ __forceinline__ void reduce_pick2(const T (&f)[4][3], int r, RED red, T& v0, T& v1) {
-  const T k0 = red(f[0][0]), k1 = red(f[0][1]), k2 = red(f[0][2]), k3 = red(f[1][0]);
-  const T k4 = red(f[1][1]), k5 = red(f[1][2]), k6 = red(f[2][0]), k7 = red(f[2][1]);
-  const T k8 = red(f[2][2]), k9 = red(f[3][0]), k10 = red(f[3][1]), k11 = red(f[3][2]);
-  const bool b0 = r & 1, b1 = r & 2, b2 = r & 4;
-  const T s0 = b0 ? k1 : k0, s1 = b0 ? k3 : k2, s2 = b0 ? k5 : k4, s3 = b0 ? k7 : k6;
-  const T t0 = b1 ? s1 : s0, t1 = b1 ? s3 : s2;
-  v0 = b2 ? t1 : t0;
-  const T w0 = b0 ? k9 : k8, w1 = b0 ? k11 : k10;
-  v1 = b1 ? w1 : w0;
+// v added to an int64 fixed-point accumulator, rounded to the nearest multiple of 2^-32: below 2^19
+// the integer is read off the mantissa of v 2^32 + 1.5 2^52 (one fma and one integer subtraction;
+// the general double-to-int64 conversion takes about ten float64 instructions); larger values (and
+// NaN) take the conversion.  Both round to nearest even.
+template <typename T>
+__device__ __forceinline__ void acc_add(unsigned long long* p, T v) {
+  unsigned long long x;
+  if (__builtin_expect(fabs((double)v) < 524288.0, 1))
+    x = (unsigned long long)(__double_as_longlong(fma((double)v, F_SCALE, 6755399441055744.0)) - 0x4338000000000000LL);
+  else
+    x = (unsigned long long)to_fx((double)v, F_SCALE);
+  if (v != (T)0) atomicAdd(p, x);
 }
-// offset of value k of a slot column within its cluster's 96 accumulators (slot = g * 8 + col)
-__device__ __forceinline__ int acc_offset(int k, int col) { return 24 * (k / 3) + 3 * col + k % 3; }
+
+// The pair kernels' force accumulators: per group of 8 slots three (backward: GN) lines of 64 bytes, one per
+// component.  Memory-side atomics cost one operation per 64-byte line an instruction touches (about
+// 24 G lines/s), so an entry costs three line operations; with x, y, z interleaved per slot it cost
+// six, and the line rate, not the arithmetic, set the kernel's time.
+__device__ __forceinline__ long long acc_slot(int sl, int a) { return (long long)(sl >> 3) * 24 + 8 * a + (sl & 7); }
 
 template <typename TC>
 struct TileArgs {
@@ -769,207 +826,258 @@ struct TileArgs {
   TC c2alpha;  // (2 / sqrt(pi)) alpha
 };
 
-// Up to 16 sub-tiles of 8 x 8 atoms of one cluster-pair tile.  Lane (ii = lane & 7, jj = lane >> 3)
-// evaluates pair (slot gi * 8 + ii of ci, slot gj * 8 + jj of cj) of sub-tile b = gi * 4 + gj.
-// MINIMG: minimum image per pair and explicit slot validity (else pj is already shifted to
-// the nearest image and padding slots sit far away); EXCL: the tile holds excluded pairs.
-template <typename TC, bool MINIMG, bool EXCL>
-__device__ __forceinline__ void tile_steps(unsigned mask, bool upper, const V4<TC> (&pi)[4], const V2<TC> (&li)[4],
-                                           const V4<TC> (&pj)[4], const V2<TC> (&lJ)[4], const unsigned (&exm)[4],
-                                           int jj, const TileArgs<TC>& ta, TC (&fi)[4][3], TC (&fj)[4][3], TC& e_c,
-                                           TC& e_lj) {
-  // j-group major, so that the first steps wait only for the first j-group's loads
-#pragma unroll
-  for (int b = 0; b < 16; ++b) {
-    const int gj = b >> 2, gi = b & 3;
-    if (!((mask >> (gi * 4 + gj)) & 1u)) continue;
-    TC dx = pi[gi].x - pj[gj].x, dy = pi[gi].y - pj[gj].y, dz = pi[gi].z - pj[gj].z;
-    if (MINIMG) {
+template <typename T> struct V3 { T x, y, z; };
+
+// the periodic shift of an entry along one axis (selected as bits, on the scalar unit)
+__device__ __forceinline__ float entry_shift(unsigned info, int axis, float L) {
+  const unsigned k = (info >> (4 + 2 * axis)) & 3u;
+  const unsigned b = __float_as_uint(L) ^ (k == 0u ? 0x80000000u : 0u);
+  return __uint_as_float(k == 1u ? 0u : b);
+}
+__device__ __forceinline__ double entry_shift(unsigned info, int axis, double L) {
+  const unsigned k = (info >> (4 + 2 * axis)) & 3u;
+  const unsigned long long b = (unsigned long long)__double_as_longlong(L);
+  const unsigned hi = (unsigned)(b >> 32) ^ (k == 0u ? 0x80000000u : 0u);
+  return join_d(k == 1u ? 0u : (unsigned)b, k == 1u ? 0u : hi);
+}
+
+// exclusion partners of the lane's i atom against j slot sj
+__device__ __forceinline__ bool is_partner(const int* __restrict__ excl_part, int sli, int sj) {
+  const int4* xp = reinterpret_cast<const int4*>(excl_part + (long long)sli * MAXEX);
+  const int4 x0 = xp[0], x1 = xp[1];
+  return x0.x == sj || x0.y == sj || x0.z == sj || x0.w == sj || x1.x == sj || x1.y == sj || x1.z == sj || x1.w == sj;
+}
+
+// A wave's share of an i-cluster's list: quads [q0, q1) of the nq quads, the first nfq of them from the
+// front (unflagged entries), the rest from the back.
+struct QuadRange {
+  int nfq, q0, q1;
+  int2 cnt;
+};
+__device__ __forceinline__ QuadRange quad_range(const PairList& pl, int ci, int part, int parts) {
+  QuadRange r;
+  r.cnt = pl.cnt[ci];
+  r.nfq = (r.cnt.x + 3) >> 2;
+  const int nq = r.nfq + r.cnt.y;
+  const int per = (nq + parts - 1) / parts;
+  r.q0 = part * per;
+  r.q1 = r.q0 + per < nq ? r.q0 + per : nq;
+  return r;
+}
+// four entries: j-groups and infos (past the list's end: info 0 and a valid entry's j-group, so that its
+// atoms can be loaded all the same)
+struct Quad {
+  int g0, g1, g2, g3;
+  unsigned i0, i1, i2, i3;
+};
+__device__ __forceinline__ Quad load_quad(const PairList& pl, int ci, const QuadRange& r, int q) {
+  const bool front = q < r.nfq;
+  const int k = front ? 4 * q : pl.cap - 4 * (q - r.nfq) - 4;
+  const long long b = (long long)ci * pl.cap + k;
+  const int4 g = *reinterpret_cast<const int4*>(pl.g + b);
+  const uint2 i = *reinterpret_cast<const uint2*>(pl.i + b);
+  const int nv = front ? r.cnt.x - k : 4;  // valid entries (at least one)
+  return {g.x, nv > 1 ? g.y : g.x, nv > 2 ? g.z : g.x, nv > 3 ? g.w : g.x,
+          i.x & 0xffffu, nv > 1 ? i.x >> 16 : 0u, nv > 2 ? i.y & 0xffffu : 0u, nv > 3 ? i.y >> 16 : 0u};
+}
+
+// the lane's atom of a j-group
+template <typename TC>
+struct JAtom {
+  V4<TC> p;
+  V2<TC> l;
+};
+template <typename TC>
+__device__ __forceinline__ JAtom<TC> load_j(const V4<TC>* __restrict__ xyzq, const V2<TC>* __restrict__ lj, int jg,
+                                            unsigned jj) {
+  return {(xyzq + (long long)jg * 8)[jj], (lj + (long long)jg * 8)[jj]};
+}
+
+template <typename TC>
+struct PairSums {
+  V3<TC> f0, f1, f2, f3;  // F of the lane's i atoms (groups 0..3)
+  TC e_lj, e_c;           // over the consecutive entries of one j-cluster
+};
+
+// One entry: the lane's j atom (shifted here) against the groups of ci in the entry's mask; F_j into fj.
+// CHECKED: the entry may hold exclusions, lie on the diagonal or need the minimum image per pair
+// (tested at run time; uniform over the wave).  The i atoms come from LDS (pi, li: slot ii of group 0):
+// kept in registers they cost two waves per SIMD (float64) for two LDS reads per group pair.
+template <typename TC, bool CHECKED>
+__device__ __forceinline__ V3<TC> entry_steps(unsigned info, int ci, int jg, const V4<TC>* pis, const V2<TC>* lis,
+                                              JAtom<TC> j, const int* __restrict__ excl_part, int ii, int jj,
+                                              const TileArgs<TC>& ta, PairSums<TC>& s) {
+  const bool minimg = CHECKED && (info & ENT_MINIMG) != 0u;
+  if (!minimg) {
+    j.p.x += entry_shift(info, 0, ta.L[0]);
+    j.p.y += entry_shift(info, 1, ta.L[1]);
+    j.p.z += entry_shift(info, 2, ta.L[2]);
+  }
+  V3<TC> fj{(TC)0, (TC)0, (TC)0};
+  auto step = [&](int gi, V3<TC>& fi) {
+    const V4<TC> pi = pis[gi * 8];
+    TC dx = pi.x - j.p.x, dy = pi.y - j.p.y, dz = pi.z - j.p.z;
+    if (minimg) {
       dx -= ta.L[0] * rint(dx * ta.invL[0]);
       dy -= ta.L[1] * rint(dy * ta.invL[1]);
       dz -= ta.L[2] * rint(dz * ta.invL[2]);
     }
-    TC r2 = dx * dx + dy * dy + dz * dz;
+    // (one order of the products in every variant: rigid molecules repeat its rounding)
+    TC r2 = fma(dz, dz, fma(dx, dx, dy * dy));
     bool ok = r2 <= ta.rc2;
-    if (MINIMG) ok = ok && pi[gi].x < (TC)PAD_LIMIT && pj[gj].x < (TC)PAD_LIMIT;
-    if (gi == gj) ok = ok && upper;
-    // about a fifth of the sub-tiles kept by the bounding-box test hold no pair within the
+    if (minimg) ok = ok && pi.x < (TC)PAD_LIMIT && j.p.x < (TC)PAD_LIMIT;
+    if (CHECKED && jg == ci * 4 + gi) ok = ok && jj > ii;
+    // about a fifth of the group pairs kept by the bounding-box test hold no pair within the
     // cutoff: the wave skips them (uniform branch)
-    if (__builtin_amdgcn_ballot_w64(ok) == 0) continue;
+    if (__builtin_amdgcn_ballot_w64(ok) == 0) return;
     bool excl = false;
-    if (EXCL) excl = (exm[gi] >> (gj * 8 + jj)) & 1u;
+    if (CHECKED && (info & ENT_EXCL)) excl = is_partner(excl_part, ci * CL + gi * 8 + ii, jg * 8 + jj);
     // pairs that do not count are moved far away: every term below is then exactly zero
     // (exp underflows, s^6 flushes), except (erfc - 1)/r of an excluded pair beyond the
-    // cutoff, which is below 1e-12 q_i q_j (and dropped with its sub-tile when no pair of the
-    // sub-tile is in range)
+    // cutoff, which is below 1e-12 q_i q_j (and dropped with its group pair when no pair of it is in
+    // range)
     r2 = ok ? r2 : (TC)1e30;
     const TC rinv = rsqrt_t(r2);
     const TC rinv2 = rinv * rinv;
     const TC r = r2 * rinv;
     TC ec, em;
-    erfc_exp(ta.alpha * r, ec, em);
-    if (EXCL) ec = excl ? ec - (TC)1 : ec;
-    const TC qr = pi[gi].w * pj[gj].w * rinv;
-    TC ep4 = li[gi].y * lJ[gj].y;
-    if (EXCL) ep4 = excl ? (TC)0 : ep4;
-    const TC sg = li[gi].x + lJ[gj].x;
+    if (CHECKED)
+      erfc_exp_excl(ta.alpha * r, excl, ec, em);
+    else
+      erfc_exp(ta.alpha * r, ec, em);
+    const V2<TC> li = lis[gi * 8];
+    const TC qr = pi.w * j.p.w * rinv;
+    TC ep4 = li.y * j.l.y;
+    if (CHECKED) ep4 = excl ? (TC)0 : ep4;
+    const TC sg = li.x + j.l.x;
     const TC s2 = sg * sg * rinv2;
     const TC s6 = s2 * s2 * s2;
     const TC a6 = ep4 * s6;  // 4 eps s^6
     // -dE/dr / r = [k q_i q_j / r (erfc + (2/sqrt pi) a r e^{-a^2 r^2}) + 4 eps s^6 (12 s^6 - 6)] / r^2
     const TC fs = fma(qr, fma(ta.c2alpha * r, em, ec), a6 * fma((TC)12, s6, (TC)-6)) * rinv2;
-    e_c = fma(qr, ec, e_c);
-    e_lj += fma(a6, s6, -a6);
+    s.e_c = fma(qr, ec, s.e_c);
+    s.e_lj += fma(a6, s6, -a6);
     // F_i += fs d, F_j -= fs d   (fs = -dE/dr / r)
-    fi[gi][0] = fma(fs, dx, fi[gi][0]);
-    fi[gi][1] = fma(fs, dy, fi[gi][1]);
-    fi[gi][2] = fma(fs, dz, fi[gi][2]);
-    fj[gj][0] = fma(-fs, dx, fj[gj][0]);
-    fj[gj][1] = fma(-fs, dy, fj[gj][1]);
-    fj[gj][2] = fma(-fs, dz, fj[gj][2]);
-  }
-}
-
-// One wave per workgroup walks a contiguous run of the (ci-ordered) tile list (the dispatcher
-// starts a new wave as soon as one finishes, which balances the uneven tiles).  F_i stays in
-// registers while ci repeats; F_j of every tile is summed over the 8 lanes sharing jj and added
-// to the int64 fixed-point accumulators.  The wave's energies go to its own slot of a partial
-// array, summed in a fixed order afterwards, so the results are bitwise reproducible.  Charges
-// are pre-multiplied by the Coulomb constant on the i side; lj holds (sigma / 2, 2 sqrt(eps))
-// so that li.y * lJ.y = 4 eps_ij.
-template <typename T>
-__device__ __forceinline__ T wave_sum_t(T v) {
-  v = octet_sum(v);
-  return stride8_sum(v);
-}
-
-template <typename TC>
-__device__ __forceinline__ void tiles_body(const int4* __restrict__ cpairs, const int* __restrict__ ncp_ptr,
-                                           long long cap, const V4<TC>* __restrict__ xyzq,
-                                           const V2<TC>* __restrict__ lj, const int* __restrict__ excl_part,
-                                           const TileArgs<TC>& ta, unsigned long long* __restrict__ facc,
-                                           unsigned long long* __restrict__ eacc) {
-  const int lane = threadIdx.x & (TFF_WAVE - 1);
-  const int ii = lane & 7, jj = lane >> 3;
-  long long ncp = *ncp_ptr;
-  if (ncp > cap) ncp = cap;
-  const long long nw = gridDim.x;
-  const long long gw = blockIdx.x;
-  const long long per = (ncp + nw - 1) / nw;
-  const long long t0 = gw * per;
-  const long long t1 = t0 + per < ncp ? t0 + per : ncp;
-  // accumulator offsets of the two values this lane writes for a j column (jj) / an i column (ii)
-  const int oj0 = acc_offset(ii, jj), oj1 = acc_offset(ii + 8 < 12 ? ii + 8 : 11, jj);
-  const int oi0 = acc_offset(jj, ii), oi1 = acc_offset(jj + 8 < 12 ? jj + 8 : 11, ii);
-  TC fi[4][3];
-  V4<TC> pi[4];
-  V2<TC> li[4];
-  auto flush_i = [&](int c) {
-    TC v0, v1;
-    reduce_pick2(fi, jj, [](TC v) { return stride8_sum(v); }, v0, v1);
-    unsigned long long* base = facc + (long long)c * (3 * CL);
-    if (v0 != (TC)0) atomicAdd(base + oi0, (unsigned long long)to_fx((double)v0, F_SCALE));
-    if (jj < 4 && v1 != (TC)0) atomicAdd(base + oi1, (unsigned long long)to_fx((double)v1, F_SCALE));
+    fi.x = fma(fs, dx, fi.x);
+    fi.y = fma(fs, dy, fi.y);
+    fi.z = fma(fs, dz, fi.z);
+    fj.x = fma(-fs, dx, fj.x);
+    fj.y = fma(-fs, dy, fj.y);
+    fj.z = fma(-fs, dz, fj.z);
   };
-  // energies: float within a tile (at most 16 terms per lane), then double across tiles
-  double e_lj = 0.0, e_c = 0.0;
-  int cur_i = -1;
-  {
-    for (long long t = t0; t < t1; ++t) {
-      const int4 cp = cpairs[t];
-      const int ci = cp.x, cj = cp.y;
-      const unsigned info = (unsigned)cp.z;
-      const unsigned mask = info & 0xffffu;
-      if (mask == 0) continue;
-      if (ci != cur_i) {
-        if (cur_i >= 0) flush_i(cur_i);
-        cur_i = ci;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int sl = ci * CL + g * 8 + ii;
-          pi[g] = xyzq[sl];
-          pi[g].w *= ta.coul;
-          li[g] = lj[sl];
-          fi[g][0] = fi[g][1] = fi[g][2] = 0;
-        }
-      }
-      const bool upper = ci != cj || jj > ii;
-      V4<TC> pj[4];
-      V2<TC> lJ[4];
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int sl = cj * CL + g * 8 + jj;
-        pj[g] = xyzq[sl];
-        lJ[g] = lj[sl];
-      }
-      unsigned exm[4] = {0u, 0u, 0u, 0u};
-      if (info & INFO_EXCL) {
-        // exclusion bit masks of this lane's four i-slots against the slots of cj
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int sl = ci * CL + g * 8 + ii;
-#pragma unroll
-          for (int k = 0; k < MAXEX; ++k) {
-            const int pv = excl_part[sl * MAXEX + k];
-            if (pv >= 0 && (pv >> 5) == cj) exm[g] |= 1u << (pv & 31);
-          }
-        }
-      }
-      TC fj[4][3];
-#pragma unroll
-      for (int g = 0; g < 4; ++g) fj[g][0] = fj[g][1] = fj[g][2] = 0;
-      TC t_lj = 0, t_c = 0;
-      if (info & INFO_MINIMG) {
-        tile_steps<TC, true, true>(mask, upper, pi, li, pj, lJ, exm, jj, ta, fi, fj, t_c, t_lj);
-      } else {
-        const TC sx = ta.L[0] * (TC)((int)((info >> 16) & 3u) - 1);
-        const TC sy = ta.L[1] * (TC)((int)((info >> 18) & 3u) - 1);
-        const TC sz = ta.L[2] * (TC)((int)((info >> 20) & 3u) - 1);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          pj[g].x += sx;
-          pj[g].y += sy;
-          pj[g].z += sz;
-        }
-        if (info & INFO_EXCL)
-          tile_steps<TC, false, true>(mask, upper, pi, li, pj, lJ, exm, jj, ta, fi, fj, t_c, t_lj);
-        else
-          tile_steps<TC, false, false>(mask, upper, pi, li, pj, lJ, exm, jj, ta, fi, fj, t_c, t_lj);
-      }
-      e_lj += (double)t_lj;
-      e_c += (double)t_c;
-      TC v0, v1;
-      reduce_pick2(fj, ii, [](TC v) { return octet_sum(v); }, v0, v1);
-      unsigned long long* base = facc + (long long)cj * (3 * CL);
-      if (v0 != (TC)0) atomicAdd(base + oj0, (unsigned long long)to_fx((double)v0, F_SCALE));
-      if (ii < 4 && v1 != (TC)0) atomicAdd(base + oj1, (unsigned long long)to_fx((double)v1, F_SCALE));
-    }
-    if (cur_i >= 0) flush_i(cur_i);
+  if (info & 1u) step(0, s.f0);
+  if (info & 2u) step(1, s.f1);
+  if (info & 4u) step(2, s.f2);
+  if (info & 8u) step(3, s.f3);
+  return fj;
+}
+
+// One wave per workgroup takes one of `parts` equal shares of an i-cluster's list, four entries at a
+// time.  The list holds only the j-groups with a partner (2.9 of the 4 of a listed cluster on average in
+// water), so the per-entry work - loads, shift, the sums of F_j, their conversion and the atomics - is
+// not spent on the empty ones; what bounds the kernel is vector issue (about 50 instructions per 8 x 8
+// block with a pair in range, 38 % of whose lanes are).  Measured at 96k atoms, alone: float 143 -> 121 us
+// (5 waves per SIMD), float64 396 -> 256 us (216 registers instead of 310: two waves per SIMD, not one),
+// against one 32 x 32 tile at a time with all 12 F_j components of it reduced in every lane; F_i stays in registers for the whole share, F_j of a quad is summed over the 8 lanes sharing
+// jj and added to the int64 fixed-point accumulators (entry 2 (lane >> 5) + ((lane >> 4) & 1), slot jj;
+// bit 3 picks the components).  Integer sums do not depend on their order and each share is summed
+// in a fixed order, so the results are bitwise reproducible.  Charges are pre-multiplied by the
+// Coulomb constant on the i side; lj holds (sigma / 2, 2 sqrt(eps)) so that li.y * lJ.y = 4 eps_ij.
+template <typename TC>
+__device__ __forceinline__ void pairs_body(const int* __restrict__ ncl_ptr, const PairList& pl, int parts,
+                                           const V4<TC>* __restrict__ xyzq, const V2<TC>* __restrict__ lj,
+                                           const int* __restrict__ excl_part, const TileArgs<TC>& ta,
+                                           unsigned long long* __restrict__ facc, ESlots es) {
+  __shared__ V4<TC> s_p[CL];
+  __shared__ V2<TC> s_l[CL];
+  const int lane = threadIdx.x & (TFF_WAVE - 1);
+  const int jj = lane & 7, ii = lane >> 3;
+  const int ci = blockIdx.x / parts;
+  if (ci >= *ncl_ptr) return;
+  const QuadRange qr = quad_range(pl, ci, blockIdx.x % parts, parts);
+  if (qr.q0 >= qr.q1) return;
+  if (lane < CL) {
+    V4<TC> p = xyzq[ci * CL + lane];
+    p.w *= ta.coul;
+    s_p[lane] = p;
+    s_l[lane] = lj[ci * CL + lane];
   }
-  // the wave's energies go to one of E_SLOTS fixed-point slots per term (spread to keep the
-  // atomics uncontended; integer sums do not depend on their order)
+  tff_wave_sync_lds();
+  const V4<TC>* pi = s_p + ii;
+  const V2<TC>* li = s_l + ii;
+  const bool b3 = lane & 8, b4 = lane & 16, b5 = lane & 32;
+  PairSums<TC> s{};
+  double e_lj = 0.0, e_c = 0.0;
+  int cj = -1;
+  auto flush_energy = [&](int c) {
+    if (c == cj) return;
+    cj = c;
+    e_lj += (double)s.e_lj;
+    e_c += (double)s.e_c;
+    s.e_lj = s.e_c = 0;
+  };
+  for (int q = qr.q0; q < qr.q1; ++q) {
+    const Quad d = load_quad(pl, ci, qr, q);
+    auto steps = [&](unsigned info, int jg, const JAtom<TC>& j) {
+      flush_energy(jg >> 2);
+      return info & (ENT_EXCL | ENT_MINIMG)
+                 ? entry_steps<TC, true>(info, ci, jg, pi, li, j, excl_part, ii, jj, ta, s)
+                 : entry_steps<TC, false>(info, ci, jg, pi, li, j, excl_part, ii, jj, ta, s);
+    };
+    // the next entry's atoms are loaded while the current one is evaluated
+    JAtom<TC> a = load_j(xyzq, lj, d.g0, jj), b = load_j(xyzq, lj, d.g1, jj);
+    const V3<TC> f0 = steps(d.i0, d.g0, a);
+    a = load_j(xyzq, lj, d.g2, jj);
+    const V3<TC> f1 = steps(d.i1, d.g1, b);
+    b = load_j(xyzq, lj, d.g3, jj);
+    const V3<TC> f2 = steps(d.i2, d.g2, a);
+    const V3<TC> f3 = steps(d.i3, d.g3, b);
+    const TC hx = quad_reduce(f0.x, f1.x, f2.x, f3.x), hy = quad_reduce(f0.y, f1.y, f2.y, f3.y),
+             hz = quad_reduce(f0.z, f1.z, f2.z, f3.z);
+    const int g0 = b4 ? d.g1 : d.g0, g1 = b4 ? d.g3 : d.g2;
+    unsigned long long* p = facc + (long long)(b5 ? g1 : g0) * 24 + jj;
+    acc_add(p + (b3 ? 8 : 0), b3 ? hy : hx);
+    if (!b3) acc_add(p + 16, hz);
+  }
+  flush_energy(-1);
+  {
+    // F_i: 12 sums over jj; lane (ii, jj) adds values jj and jj + 8 (value 3 g + a: slot g * 8 + ii)
+    const TC k0 = octet_sum(s.f0.x), k1 = octet_sum(s.f0.y), k2 = octet_sum(s.f0.z), k3 = octet_sum(s.f1.x);
+    const TC k4 = octet_sum(s.f1.y), k5 = octet_sum(s.f1.z), k6 = octet_sum(s.f2.x), k7 = octet_sum(s.f2.y);
+    const TC k8 = octet_sum(s.f2.z), k9 = octet_sum(s.f3.x), k10 = octet_sum(s.f3.y), k11 = octet_sum(s.f3.z);
+    const bool c0 = jj & 1, c1 = jj & 2, c2 = jj & 4;
+    const TC s0 = c0 ? k1 : k0, s1 = c0 ? k3 : k2, s2 = c0 ? k5 : k4, s3 = c0 ? k7 : k6;
+    const TC t0 = c1 ? s1 : s0, t1 = c1 ? s3 : s2;
+    const TC w0 = c0 ? k9 : k8, w1 = c0 ? k11 : k10;
+    unsigned long long* p = facc + (long long)ci * (3 * CL);
+    acc_add(p + 8 * jj + ii, c2 ? t1 : t0);
+    if (jj < 4) acc_add(p + 8 * (jj + 8) + ii, c1 ? w1 : w0);
+  }
+  // the wave's energies (integer sums do not depend on their order)
   const double el = wave_sum_t(e_lj), ecl = wave_sum_t(e_c);
-  if (lane == 0 && t1 > t0) {
-    atomicAdd(&eacc[gw % E_SLOTS], (unsigned long long)to_fx(el, F_SCALE));
-    atomicAdd(&eacc[E_SLOTS + gw % E_SLOTS], (unsigned long long)to_fx(ecl, F_SCALE));
+  if (lane == 0) {
+    unsigned long long* e = es.line(blockIdx.x);
+    atomicAdd(e, (unsigned long long)to_fx(el, F_SCALE));
+    atomicAdd(e + 1, (unsigned long long)to_fx(ecl, F_SCALE));
   }
 }
 
-// float: registers capped for 4 waves per SIMD; float64 keeps its full register set
 __global__ __launch_bounds__(TFF_WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_tiles_f32(
-    const int4* __restrict__ cpairs, const int* __restrict__ ncp_ptr, long long cap, const V4<float>* __restrict__ xyzq,
+    const int* __restrict__ ncl_ptr, PairList pl, int parts, const V4<float>* __restrict__ xyzq,
     const V2<float>* __restrict__ lj, const int* __restrict__ excl_part, TileArgs<float> ta,
-    unsigned long long* __restrict__ facc, unsigned long long* __restrict__ eacc) {
-  tiles_body<float>(cpairs, ncp_ptr, cap, xyzq, lj, excl_part, ta, facc, eacc);
+    unsigned long long* __restrict__ facc, ESlots es) {
+  // The body needs 89 registers, i.e. 5 waves per SIMD; naming v103 holds it at 4 (104 each) and leaves
+  // 96 per SIMD free, so that the workgroups of the reciprocal-space chain find room beside the pair
+  // kernel.  Alone the kernel takes 121 us with 5 waves and 129 with 4 (96k atoms), the whole
+  // evaluation 256 and 243 us; 999k atoms 2.02 and 2.00 ms.
+  asm volatile("" ::: "v103");
+  pairs_body<float>(ncl_ptr, pl, parts, xyzq, lj, excl_part, ta, facc, es);
 }
-__global__ __launch_bounds__(TFF_WAVE) void k_tiles_f64(const int4* __restrict__ cpairs,
-                                                       const int* __restrict__ ncp_ptr, long long cap,
-                                                       const V4<double>* __restrict__ xyzq,
-                                                       const V2<double>* __restrict__ lj,
-                                                       const int* __restrict__ excl_part, TileArgs<double> ta,
-                                                       unsigned long long* __restrict__ facc,
-                                                       unsigned long long* __restrict__ eacc) {
-  tiles_body<double>(cpairs, ncp_ptr, cap, xyzq, lj, excl_part, ta, facc, eacc);
+__global__ __launch_bounds__(TFF_WAVE) __attribute__((amdgpu_waves_per_eu(2))) void k_tiles_f64(
+    const int* __restrict__ ncl_ptr, PairList pl, int parts, const V4<double>* __restrict__ xyzq,
+    const V2<double>* __restrict__ lj, const int* __restrict__ excl_part, TileArgs<double> ta,
+    unsigned long long* __restrict__ facc, ESlots es) {
+  pairs_body<double>(ncl_ptr, pl, parts, xyzq, lj, excl_part, ta, facc, es);
 }
 
 // ---------------------------------------------------------------- 4b. force-matching backward
@@ -987,7 +1095,7 @@ constexpr int GN = 6;
 static_assert(4 * GN == 24, "a cluster column holds 24 backward sums per lane");
 
 // per slot: the upstream force v (x, y, z) and 1 / (2 eps) (w; 0 where eps = 0), from lj's 2 sqrt(eps);
-// with status_from set, thread 0 also starts the call's status words from those of the forward call
+// with status_from set, thread 0 also starts the call's flags from those of the forward call
 // whose cluster arrays and pair list are reused
 template <typename TI, typename TC>
 __global__ __launch_bounds__(FB) void k_fill_vslots(const int* __restrict__ ncl_ptr, const int* __restrict__ slot_orig,
@@ -997,7 +1105,6 @@ __global__ __launch_bounds__(FB) void k_fill_vslots(const int* __restrict__ ncl_
   const int sl = blockIdx.x * FB + threadIdx.x;
   if (status_from && sl == 0) {
     status[0] = status_from[0];
-    status[1] = status_from[1];
   }
   if (sl >= *ncl_ptr * CL) return;
   const int i = slot_orig[sl];
@@ -1007,217 +1114,167 @@ __global__ __launch_bounds__(FB) void k_fill_vslots(const int* __restrict__ ncl_
                           : V4<TC>{(TC)0, (TC)0, (TC)0, ehalf_inv};
 }
 
-// the value of the lane whose index within its eight differs in bit B (the partner for B = 2 is the
-// mirrored lane, whose lower bits differ too: only the opposite bit 2 matters below)
-template <int B>
-__device__ __forceinline__ float octet_xchg(float v) {
-  return dpp_f<B == 2 ? 0x141 : B == 1 ? 0x4E : 0xB1>(v);
-}
-template <int B>
-__device__ __forceinline__ double octet_xchg(double v) {
-  return dpp_d<B == 2 ? 0x141 : B == 1 ? 0x4E : 0xB1>(v);
-}
-template <bool STRIDE8, int B, typename T>
-__device__ __forceinline__ T xchg8(T v) {
-  if constexpr (STRIDE8)
-    return __shfl_xor(v, 8 << B, TFF_WAVE);
-  else
-    return octet_xchg<B>(v);
-}
-// Reduce-scatter of 24 values over eight lanes (contiguous lanes, or lanes at stride 8): lane m of
-// the eight ends with the sums of values m, m + 8 and m + 16.  Each of the three exchange steps
-// halves what a lane keeps: 21 exchanges where summing every value in every lane takes 72.
-template <bool STRIDE8, typename T>
-__device__ __forceinline__ void reduce_scatter24(const T (&a)[24], int m, T (&out)[3]) {
-  const bool b2 = (m >> 2) & 1, b1 = (m >> 1) & 1, b0 = m & 1;
-  T h[12];  // h[4 r + c]: value 8 r + 4 b2 + c
-#pragma unroll
-  for (int r = 0; r < 3; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const T lo = a[8 * r + c], hi = a[8 * r + 4 + c];
-      h[4 * r + c] = (b2 ? hi : lo) + xchg8<STRIDE8, 2>(b2 ? lo : hi);
-    }
-  T q[6];  // q[2 r + c]: value 8 r + 4 b2 + 2 b1 + c
-#pragma unroll
-  for (int r = 0; r < 3; ++r)
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const T lo = h[4 * r + c], hi = h[4 * r + 2 + c];
-      q[2 * r + c] = (b1 ? hi : lo) + xchg8<STRIDE8, 1>(b1 ? lo : hi);
-    }
-#pragma unroll
-  for (int r = 0; r < 3; ++r) {
-    const T lo = q[2 * r], hi = q[2 * r + 1];
-    out[r] = (b0 ? hi : lo) + xchg8<STRIDE8, 0>(b0 ? lo : hi);
-  }
-}
+template <typename T> struct GradSums { T x, y, z, q, s, e; };
 
-// One wave per workgroup over a contiguous run of the tile list (as the forward pair kernel);
-// one i-group at a time (lane = (ii, jj) holds i-slot gi * 8 + ii against j-slot gj * 8 + jj),
-// the tile's periodic shift (minimum image per pair on the tiles flagged for it).
+// One wave per workgroup over a share of an i-cluster's list, as the forward pair kernel (the tile's
+// periodic shift, minimum image per pair on the entries flagged for it); the i-side data of ci's four
+// groups stays in LDS, its sums in registers.
 // Per pair, in factored form without divisions (Q = q_i q_j, s6 = (sigma_ij / r)^6):
 //   f = -k Q g / r^3 - 4 eps s6 (12 s6 - 6) / r^2
 //   h =  k Q (3 g / r^3 + (4/sqrt pi) a^3 e^{-a^2 r^2}) / r^2 + 4 eps s6 (168 s6 - 48) / r^4
 //   d phi / d sigma_ij = 4 eps (s6 / sigma_ij) (12 s6 - 6),  s6 / sigma_ij = s^4 sigma_ij / r^2,
 //   d (f s) / d sigma_ij = -4 eps (s6 / sigma_ij) (144 s6 - 36) s / r^2,
 // and 1 / (2 eps) of every slot precomputed (the w component of the per-slot upstream force).
-// The i-side sums stay in registers while ci repeats (the list is ci-ordered) and are flushed once
-// per run of tiles; the j-side sums once per tile.  Value q = 6 g + k of a cluster's 24 per lane
-// column is component k of slot g * 8 + column.
 template <typename TC>
-__global__ __launch_bounds__(TFF_WAVE) void k_tiles_grad(const int4* __restrict__ cpairs,
-                                                         const int* __restrict__ ncp_ptr, long long cap,
-                                                         const V4<TC>* __restrict__ xyzq,
-                                                         const V2<TC>* __restrict__ lj,
-                                                         const V4<TC>* __restrict__ vsl,
-                                                         const int* __restrict__ excl_part, TileArgs<TC> ta,
-                                                         const double* __restrict__ gE_ptr,
-                                                         unsigned long long* __restrict__ gacc) {
+__device__ __forceinline__ void grad_body(const int* __restrict__ ncl_ptr, const PairList& pl, int parts,
+                                          const V4<TC>* __restrict__ xyzq, const V2<TC>* __restrict__ lj,
+                                          const V4<TC>* __restrict__ vsl, const int* __restrict__ excl_part,
+                                          const TileArgs<TC>& ta, const double* __restrict__ gE_ptr,
+                                          unsigned long long* __restrict__ gacc) {
+  __shared__ V4<TC> s_p[CL], s_v[CL];
+  __shared__ V2<TC> s_l[CL];
   const int lane = threadIdx.x & (TFF_WAVE - 1);
-  const int ii = lane & 7, jj = lane >> 3;
-  long long ncp = *ncp_ptr;
-  if (ncp > cap) ncp = cap;
-  const long long nw = gridDim.x, gw = blockIdx.x;
-  const long long per = (ncp + nw - 1) / nw;
-  const long long t0 = gw * per;
-  const long long t1 = t0 + per < ncp ? t0 + per : ncp;
+  const int jj = lane & 7, ii = lane >> 3;
+  const int ci = blockIdx.x / parts;
+  if (ci >= *ncl_ptr) return;
+  const QuadRange qr = quad_range(pl, ci, blockIdx.x % parts, parts);
+  if (qr.q0 >= qr.q1) return;
+  if (lane < CL) {
+    s_p[lane] = xyzq[ci * CL + lane];
+    s_v[lane] = vsl[ci * CL + lane];
+    s_l[lane] = lj[ci * CL + lane];
+  }
+  tff_wave_sync_lds();
   const TC gE = gE_ptr ? (TC)gE_ptr[0] : (TC)0;
   const TC c2 = (TC)1.1283791670955126;                     // 2 / sqrt(pi)
   const TC ch = (TC)2 * c2 * ta.alpha * ta.alpha * ta.alpha;  // (4 / sqrt pi) a^3
-  TC ai[4][GN];
-  int cur_i = -1;
-  // the 24 sums of a cluster's lane column over the eight lanes sharing it, added to the
-  // accumulators of slot (q / GN) * 8 + col (value q = col8 + 8 r of the lane at col8)
-  auto flush = [&](const TC (&a)[4][GN], int c, int col, int col8, auto stride8) {
-    TC v[3];
-    reduce_scatter24<decltype(stride8)::value>(reinterpret_cast<const TC(&)[24]>(a), col8, v);
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      const int q = col8 + 8 * r;
-      if (v[r] != (TC)0) {
-        const long long sl = (long long)c * CL + (q / GN) * 8 + col;
-        atomicAdd(&gacc[GN * sl + q % GN], (unsigned long long)to_fx((double)v[r], F_SCALE));
+  const bool b3 = lane & 8, b4 = lane & 16, b5 = lane & 32;
+  GradSums<TC> a0{}, a1{}, a2{}, a3{};
+  // one entry: the lane's j atom against the groups of ci in the entry's mask (see entry_steps)
+  auto entry = [&](auto chk, unsigned info, int jg) {
+    constexpr bool CHECKED = decltype(chk)::value;
+    const bool minimg = CHECKED && (info & ENT_MINIMG) != 0u;
+    JAtom<TC> j = load_j(xyzq, lj, jg, jj);
+    const V4<TC> vj = (vsl + (long long)jg * 8)[(unsigned)jj];
+    if (!minimg) {
+      j.p.x += entry_shift(info, 0, ta.L[0]);
+      j.p.y += entry_shift(info, 1, ta.L[1]);
+      j.p.z += entry_shift(info, 2, ta.L[2]);
+    }
+    const TC kqj = ta.coul * j.p.w;
+    GradSums<TC> b{};
+    auto step = [&](int gi, GradSums<TC>& a) {
+      const V4<TC> pi = s_p[gi * 8 + ii];
+      TC dx = pi.x - j.p.x, dy = pi.y - j.p.y, dz = pi.z - j.p.z;
+      if (minimg) {  // uniform over the wave
+        dx -= ta.L[0] * rint(dx * ta.invL[0]);
+        dy -= ta.L[1] * rint(dy * ta.invL[1]);
+        dz -= ta.L[2] * rint(dz * ta.invL[2]);
       }
-    }
-  };
-  for (long long t = t0; t < t1; ++t) {
-    const int4 cp = cpairs[t];
-    const int ci = cp.x, cj = cp.y;
-    const unsigned info = (unsigned)cp.z;
-    const unsigned mask = info & 0xffffu;
-    if (mask == 0) continue;
-    if (ci != cur_i) {
-      if (cur_i >= 0) flush(ai, cur_i, ii, jj, std::true_type{});
-      cur_i = ci;
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int k = 0; k < GN; ++k) ai[g][k] = 0;
-    }
-    const bool upper = ci != cj || jj > ii;
-    // tiles flagged for per-pair minimum image keep it; the others take the tile's periodic shift
-    const bool minimg = (info & INFO_MINIMG) != 0u;
-    const TC shx = minimg ? (TC)0 : ta.L[0] * (TC)((int)((info >> 16) & 3u) - 1);
-    const TC shy = minimg ? (TC)0 : ta.L[1] * (TC)((int)((info >> 18) & 3u) - 1);
-    const TC shz = minimg ? (TC)0 : ta.L[2] * (TC)((int)((info >> 20) & 3u) - 1);
-    V4<TC> pj[4], vj[4];
-    V2<TC> lJ[4];
-    TC kqj[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int sl = cj * CL + g * 8 + jj;
-      pj[g] = xyzq[sl];
-      pj[g].x += shx;
-      pj[g].y += shy;
-      pj[g].z += shz;
-      lJ[g] = lj[sl];
-      vj[g] = vsl[sl];
-      kqj[g] = ta.coul * pj[g].w;
-    }
-    TC aj[4][GN];
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int k = 0; k < GN; ++k) aj[g][k] = 0;
-#pragma unroll
-    for (int gi = 0; gi < 4; ++gi) {
-      if (!((mask >> (gi * 4)) & 0xfu)) continue;
-      const int sli = ci * CL + gi * 8 + ii;
-      const V4<TC> pi = xyzq[sli];
-      const V2<TC> li = lj[sli];
-      const V4<TC> vi = vsl[sli];
-      unsigned exm = 0u;
-      if (info & INFO_EXCL) {
-#pragma unroll
-        for (int k = 0; k < MAXEX; ++k) {
-          const int pv = excl_part[sli * MAXEX + k];
-          if (pv >= 0 && (pv >> 5) == cj) exm |= 1u << (pv & 31);
-        }
-      }
-      TC (&a)[GN] = ai[gi];
+      TC r2 = dx * dx + dy * dy + dz * dz;
+      // padding slots are out of range of everything, unless wrapped by the per-pair minimum image
+      bool ok = r2 <= ta.rc2;
+      if (minimg) ok = ok && pi.x < (TC)PAD_LIMIT && j.p.x < (TC)PAD_LIMIT;
+      if (CHECKED && jg == ci * 4 + gi) ok = ok && jj > ii;
+      if (__builtin_amdgcn_ballot_w64(ok) == 0) return;  // no pair of the two groups in range
+      bool excl = false;
+      if (CHECKED && (info & ENT_EXCL)) excl = is_partner(excl_part, ci * CL + gi * 8 + ii, jg * 8 + jj);
+      const V2<TC> li = s_l[gi * 8 + ii];
+      const V4<TC> vi = s_v[gi * 8 + ii];
       const TC kqi = ta.coul * pi.w;
-#pragma unroll
-      for (int gj = 0; gj < 4; ++gj) {
-        if (!((mask >> (gi * 4 + gj)) & 1u)) continue;
-        TC dx = pi.x - pj[gj].x, dy = pi.y - pj[gj].y, dz = pi.z - pj[gj].z;
-        if (minimg) {  // uniform over the wave
-          dx -= ta.L[0] * rint(dx * ta.invL[0]);
-          dy -= ta.L[1] * rint(dy * ta.invL[1]);
-          dz -= ta.L[2] * rint(dz * ta.invL[2]);
-        }
-        TC r2 = dx * dx + dy * dy + dz * dz;
-        bool ok = r2 <= ta.rc2 && pi.x < (TC)PAD_LIMIT && pj[gj].x < (TC)PAD_LIMIT;
-        if (gi == gj) ok = ok && upper;
-        if (__builtin_amdgcn_ballot_w64(ok) == 0) continue;  // no pair of the sub-tile in range
-        const bool excl = (exm >> (gj * 8 + jj)) & 1u;
-        r2 = ok ? r2 : (TC)1e30;
-        const TC rinv = rsqrt_t(r2);
-        const TC rinv2 = rinv * rinv;
-        const TC u = ta.alpha * (r2 * rinv);
-        TC ec, em;
+      r2 = ok ? r2 : (TC)1e30;
+      const TC rinv = rsqrt_t(r2);
+      const TC rinv2 = rinv * rinv;
+      const TC u = ta.alpha * (r2 * rinv);
+      TC ec, em;
+      if (CHECKED)
+        erfc_exp_excl(u, excl, ec, em);                      // c = erfc - [excluded]
+      else
         erfc_exp(u, ec, em);
-        ec = excl ? ec - (TC)1 : ec;                       // c = erfc - [excluded]
-        const TC grinv3 = fma(c2 * u, em, ec) * rinv * rinv2;  // g / r^3
-        const TC kQ = kqi * pj[gj].w;
-        const TC eps4 = excl ? (TC)0 : li.y * lJ[gj].y;
-        const TC sg = li.x + lJ[gj].x;
-        const TC tq = sg * rinv2;  // s^2 / sigma_ij
-        const TC s2 = sg * tq;
-        const TC s4 = s2 * s2;
-        const TC s6 = s4 * s2;
-        const TC ps = s4 * tq;     // s6 / sigma_ij
-        const TC a12 = fma((TC)12, s6, (TC)-6);
-        const TC e6 = eps4 * s6;
-        const TC f = fma(-kQ, grinv3, -e6 * a12 * rinv2);
-        const TC h = fma(kQ * rinv2, fma((TC)3, grinv3, ch * em), e6 * fma((TC)168, s6, (TC)-48) * (rinv2 * rinv2));
-        const TC okf = ok ? (TC)1 : (TC)0;
-        const TC dvx = vi.x - vj[gj].x, dvy = vi.y - vj[gj].y, dvz = vi.z - vj[gj].z;
-        const TC sdv = dx * dvx + dy * dvy + dz * dvz;
-        const TC cd = okf * fma(gE, f, -sdv * h), cv = okf * f;
-        const TC gx = cd * dx - cv * dvx, gy = cd * dy - cv * dvy, gz = cd * dz - cv * dvz;
-        a[0] += gx;
-        a[1] += gy;
-        a[2] += gz;
-        aj[gj][0] -= gx;
-        aj[gj][1] -= gy;
-        aj[gj][2] -= gz;
-        // d/dq_i = k q_j (gE c / r + (s.dv) g / r^3), d/dq_j alike with k q_i
-        const TC gq = okf * fma(gE, ec * rinv, sdv * grinv3);
-        a[3] = fma(kqj[gj], gq, a[3]);
-        aj[gj][3] = fma(kqi, gq, aj[gj][3]);
-        const TC rs = sdv * rinv2;
-        const TC ts = okf * (TC)0.5 * eps4 * ps * fma(gE, a12, rs * fma((TC)144, s6, (TC)-36));
-        a[4] += ts;
-        aj[gj][4] += ts;
-        const TC te = okf * e6 * fma(gE, s6 - (TC)1, rs * a12);
-        a[5] = fma(te, vi.w, a[5]);
-        aj[gj][5] = fma(te, vj[gj].w, aj[gj][5]);
-      }
-    }
-    flush(aj, cj, jj, ii, std::false_type{});
+      const TC grinv3 = fma(c2 * u, em, ec) * rinv * rinv2;  // g / r^3
+      const TC kQ = kqi * j.p.w;
+      const TC eps4 = CHECKED && excl ? (TC)0 : li.y * j.l.y;
+      const TC sg = li.x + j.l.x;
+      const TC tq = sg * rinv2;  // s^2 / sigma_ij
+      const TC s2 = sg * tq;
+      const TC s4 = s2 * s2;
+      const TC s6 = s4 * s2;
+      const TC ps = s4 * tq;     // s6 / sigma_ij
+      const TC a12 = fma((TC)12, s6, (TC)-6);
+      const TC e6 = eps4 * s6;
+      const TC f = fma(-kQ, grinv3, -e6 * a12 * rinv2);
+      const TC h = fma(kQ * rinv2, fma((TC)3, grinv3, ch * em), e6 * fma((TC)168, s6, (TC)-48) * (rinv2 * rinv2));
+      const TC okf = ok ? (TC)1 : (TC)0;
+      const TC dvx = vi.x - vj.x, dvy = vi.y - vj.y, dvz = vi.z - vj.z;
+      const TC sdv = dx * dvx + dy * dvy + dz * dvz;
+      const TC cd = okf * fma(gE, f, -sdv * h), cv = okf * f;
+      const TC gx = cd * dx - cv * dvx, gy = cd * dy - cv * dvy, gz = cd * dz - cv * dvz;
+      a.x += gx;
+      a.y += gy;
+      a.z += gz;
+      b.x -= gx;
+      b.y -= gy;
+      b.z -= gz;
+      // d/dq_i = k q_j (gE c / r + (s.dv) g / r^3), d/dq_j alike with k q_i
+      const TC gq = okf * fma(gE, ec * rinv, sdv * grinv3);
+      a.q = fma(kqj, gq, a.q);
+      b.q = fma(kqi, gq, b.q);
+      const TC rs = sdv * rinv2;
+      const TC ts = okf * (TC)0.5 * eps4 * ps * fma(gE, a12, rs * fma((TC)144, s6, (TC)-36));
+      a.s += ts;
+      b.s += ts;
+      const TC te = okf * e6 * fma(gE, s6 - (TC)1, rs * a12);
+      a.e = fma(te, vi.w, a.e);
+      b.e = fma(te, vj.w, b.e);
+    };
+    if (info & 1u) step(0, a0);
+    if (info & 2u) step(1, a1);
+    if (info & 4u) step(2, a2);
+    if (info & 8u) step(3, a3);
+    return b;
+  };
+  for (int q = qr.q0; q < qr.q1; ++q) {
+    const Quad d = load_quad(pl, ci, qr, q);
+    auto steps = [&](unsigned info, int jg) {
+      return info & (ENT_EXCL | ENT_MINIMG) ? entry(std::true_type{}, info, jg) : entry(std::false_type{}, info, jg);
+    };
+    const GradSums<TC> f0 = steps(d.i0, d.g0), f1 = steps(d.i1, d.g1), f2 = steps(d.i2, d.g2), f3 = steps(d.i3, d.g3);
+    const TC h0 = quad_reduce(f0.x, f1.x, f2.x, f3.x), h1 = quad_reduce(f0.y, f1.y, f2.y, f3.y),
+             h2 = quad_reduce(f0.z, f1.z, f2.z, f3.z), h3 = quad_reduce(f0.q, f1.q, f2.q, f3.q),
+             h4 = quad_reduce(f0.s, f1.s, f2.s, f3.s), h5 = quad_reduce(f0.e, f1.e, f2.e, f3.e);
+    const int g0 = b4 ? d.g1 : d.g0, g1 = b4 ? d.g3 : d.g2;
+    unsigned long long* p = gacc + (long long)(b5 ? g1 : g0) * (8 * GN) + (b3 ? 24 : 0) + jj;
+    acc_add(p, b3 ? h3 : h0);
+    acc_add(p + 8, b3 ? h4 : h1);
+    acc_add(p + 16, b3 ? h5 : h2);
   }
-  if (cur_i >= 0) flush(ai, cur_i, ii, jj, std::true_type{});
+  // the i side: 24 sums over jj; lane (ii, jj) adds values jj, jj + 8, jj + 16 (value 6 g + k: slot g * 8 + ii)
+  const TC all[24] = {a0.x, a0.y, a0.z, a0.q, a0.s, a0.e, a1.x, a1.y, a1.z, a1.q, a1.s, a1.e,
+                      a2.x, a2.y, a2.z, a2.q, a2.s, a2.e, a3.x, a3.y, a3.z, a3.q, a3.s, a3.e};
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    TC v = 0;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const TC t = octet_sum(all[8 * r + m]);
+      v = jj == m ? t : v;
+    }
+    const int k = jj + 8 * r;
+    acc_add(gacc + (long long)ci * (CL * GN) + 8 * k + ii, v);
+  }
+}
+
+__global__ __launch_bounds__(TFF_WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_tiles_grad_f32(
+    const int* __restrict__ ncl_ptr, PairList pl, int parts, const V4<float>* __restrict__ xyzq,
+    const V2<float>* __restrict__ lj, const V4<float>* __restrict__ vsl, const int* __restrict__ excl_part,
+    TileArgs<float> ta, const double* __restrict__ gE_ptr, unsigned long long* __restrict__ gacc) {
+  grad_body<float>(ncl_ptr, pl, parts, xyzq, lj, vsl, excl_part, ta, gE_ptr, gacc);
+}
+__global__ __launch_bounds__(TFF_WAVE) void k_tiles_grad_f64(
+    const int* __restrict__ ncl_ptr, PairList pl, int parts, const V4<double>* __restrict__ xyzq,
+    const V2<double>* __restrict__ lj, const V4<double>* __restrict__ vsl, const int* __restrict__ excl_part,
+    TileArgs<double> ta, const double* __restrict__ gE_ptr, unsigned long long* __restrict__ gacc) {
+  grad_body<double>(ncl_ptr, pl, parts, xyzq, lj, vsl, excl_part, ta, gE_ptr, gacc);
 }
 
 // ---------------------------------------------------------------- 5. PME on cluster slots
@@ -1944,6 +2001,16 @@ __global__ __launch_bounds__(FB) void k_gather_grad(const int* __restrict__ ncl_
   gpme[4 * (long long)sl + 3] = (unsigned long long)to_fx(dq, F_SCALE);
 }
 
+// word k of the slots, summed by the first wave of a workgroup (the result is valid there)
+__device__ __forceinline__ long long slot_sum(const ESlots& es, int k) {
+  long long v = 0;
+  if (threadIdx.x < TFF_WAVE) {
+    for (int j = threadIdx.x; j < es.n; j += TFF_WAVE) v += (long long)es.p[8 * j + k];
+    for (int o = TFF_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, TFF_WAVE);
+  }
+  return v;
+}
+
 // gradients back in the caller's atom order (pair + reciprocal accumulators; self energy
 // -k alpha / sqrt(pi) sum q^2 contributes gE * (-2 k alpha / sqrt(pi)) q_i to dL/dq_i)
 template <typename TI>
@@ -1953,28 +2020,33 @@ __global__ __launch_bounds__(FB) void k_finalize_grad(const int* __restrict__ nc
                                                       const TI* __restrict__ q, double coul, double alpha,
                                                       const double* __restrict__ gE_ptr, TI* __restrict__ dr,
                                                       TI* __restrict__ dq, TI* __restrict__ dsig, TI* __restrict__ deps,
-                                                      const int* __restrict__ status, int* __restrict__ status_host) {
+                                                      ESlots es,
+                                                      int* __restrict__ status, int* __restrict__ status_host) {
   const int sl = blockIdx.x * FB + threadIdx.x;
-  if (status_host && sl == 0) {
+  const int s1 = blockIdx.x == 0 ? (int)slot_sum(es, 2) : 0;
+  if (sl == 0) {
     // every kernel that sets a flag ran before this one on the stream; word 0 last, after a
     // system-scope fence: a host that sees it sees word 1
-    status_host[1] = status[1];
-    __threadfence_system();
-    status_host[0] = status[0];
+    status[1] = s1;
+    if (status_host) {
+      status_host[1] = s1;
+      __threadfence_system();
+      status_host[0] = status[0];
+    }
   }
   if (sl >= *ncl_ptr * CL) return;
   const int i = slot_orig[sl];
   if (i < 0) return;
-  const long long b6 = (long long)GN * sl, b4 = 4 * (long long)sl;
+  const long long b6 = (long long)(sl >> 3) * (8 * GN) + (sl & 7), b4 = 4 * (long long)sl;
   if (dr)
-    for (int a = 0; a < 3; ++a) dr[3 * i + a] = (TI)((double)(long long)(gacc[b6 + a] + gpme[b4 + a]) / F_SCALE);
+    for (int a = 0; a < 3; ++a) dr[3 * i + a] = (TI)((double)(long long)(gacc[b6 + 8 * a] + gpme[b4 + a]) / F_SCALE);
   if (dq) {
     const double gE = gE_ptr ? gE_ptr[0] : 0.0;
-    dq[i] = (TI)((double)(long long)(gacc[b6 + 3] + gpme[b4 + 3]) / F_SCALE -
+    dq[i] = (TI)((double)(long long)(gacc[b6 + 24] + gpme[b4 + 3]) / F_SCALE -
                  gE * 2.0 * coul * alpha * 0.5641895835477563 * (double)q[i]);
   }
-  if (dsig) dsig[i] = (TI)((double)(long long)gacc[b6 + 4] / F_SCALE);
-  if (deps) deps[i] = (TI)((double)(long long)gacc[b6 + 5] / F_SCALE);
+  if (dsig) dsig[i] = (TI)((double)(long long)gacc[b6 + 32] / F_SCALE);
+  if (deps) deps[i] = (TI)((double)(long long)gacc[b6 + 40] / F_SCALE);
 }
 
 // ---------------------------------------------------------------- 6. finalize
@@ -1985,15 +2057,16 @@ template <typename TI>
 __global__ __launch_bounds__(FB) void k_finalize(const int* __restrict__ ncl_ptr, const int* __restrict__ slot_orig,
                                                  const unsigned long long* __restrict__ facc,
                                                  const unsigned long long* __restrict__ facc_pme, TI* __restrict__ forces,
-                                                 const unsigned long long* __restrict__ eacc,
+                                                 ESlots es,
                                                  const double* __restrict__ kparts, int nk,
                                                  const double* __restrict__ qparts, int nq, double coul,
                                                  double alpha, double* __restrict__ out, const int* __restrict__ status,
                                                  int* __restrict__ status_out, int* __restrict__ status_host) {
   const int sl = blockIdx.x * FB + threadIdx.x;
+  const int s1 = blockIdx.x == 0 ? (int)slot_sum(es, 2) : 0;
   if (sl == 0) {
     // every kernel that sets a flag ran before this one on the stream (after the join)
-    const int s0 = status[0], s1 = status[1];
+    const int s0 = status[0];
     status_out[0] = s0;
     status_out[1] = s1;
     if (status_host) {
@@ -2007,17 +2080,13 @@ __global__ __launch_bounds__(FB) void k_finalize(const int* __restrict__ ncl_ptr
     const int i = slot_orig[sl];
     if (i >= 0)
       for (int a = 0; a < 3; ++a)
-        forces[3 * i + a] = (TI)((double)(long long)(facc[3 * sl + a] + facc_pme[3 * sl + a]) / F_SCALE);
+        forces[3 * i + a] = (TI)((double)(long long)(facc[acc_slot(sl, a)] + facc_pme[3 * sl + a]) / F_SCALE);
   }
   if (blockIdx.x != 0) return;
   const double ek = tff_sum_partials(kparts, nk);
   const double q2 = tff_sum_partials(qparts, nq);
+  const long long sl_lj = slot_sum(es, 0), sl_c = slot_sum(es, 1);
   if (threadIdx.x != 0) return;
-  long long sl_lj = 0, sl_c = 0;
-  for (int k = 0; k < E_SLOTS; ++k) {
-    sl_lj += (long long)eacc[k];
-    sl_c += (long long)eacc[E_SLOTS + k];
-  }
   out[0] = (double)sl_lj / F_SCALE;
   out[1] = (double)sl_c / F_SCALE;
   out[2] = coul * ek;
@@ -2061,12 +2130,14 @@ bool make_geo(const TffBox& box, long long n, double list_cutoff, Geo& g) {
   return true;
 }
 
-// waves of the pair kernel: about 16 tile-list slots each (some 6 listed tiles at water density)
-int tile_waves(const Geo& g) {
-  long long w = (g.pair_cap + 15) / 16;
-  if (w < 256) w = 256;
-  if (w > (1 << 20)) w = 1 << 20;
-  return (int)w;
+// Waves per i-cluster of the pair kernels: about 9000 waves in all (two rounds of the device's 4096 resident
+// ones), so that a small system still spreads over the device; one wave per cluster where the clusters
+// alone are enough.  Every further wave pays its start, the i atoms and the F_i sums again.  Measured
+// (pair kernel, float): 96k atoms 131 us at 3 waves per cluster, 138 at 6, 150 at 11; 999k atoms
+// 1.45 ms at 1, 1.54 at 4.
+int pair_parts(const Geo& g) {
+  const int p = (9000 + g.ncl_max - 1) / g.ncl_max;
+  return p > 32 ? 32 : p;
 }
 
 // z extent of the reciprocal-space array: even K2 uses the real-input half spectrum
@@ -2074,16 +2145,15 @@ int spectrum_nz(const int K[3]) { return K[2] % 2 == 0 ? K[2] / 2 + 1 : K[2]; }
 
 struct FusedWs {
   int *col_of, *off_in_col, *col_count, *col_start, *sorted_orig, *col_cl_start, *ncl, *cl_col, *slot_orig,
-      *excl_part, *ncp, *seg_count, *seg_start, *slot_of_orig;
+      *excl_part, *slot_of_orig;
   int* st;  // the forward call's status words while it runs (copied out by k_finalize)
-  int2* seg;
+  PairList pl;
   void *xyzq, *lj;
   float4 *bb_c, *bb_h, *sb_c, *sb_h;
-  int4* cpairs;
   unsigned long long *facc, *facc_pme, *grid;
   void* work;
   double *kparts, *qparts;
-  unsigned long long* eacc;
+  ESlots es;
   // float compute only: per-slot spline tables and home-brick lists of the charge spread
   float* wts;
   int* bcount;
@@ -2093,7 +2163,7 @@ struct FusedWs {
   void* vsl;
   unsigned long long *gacc, *gpme, *grid_d;
   size_t bytes;
-  int nk, nw_tiles, nq;
+  int nk, parts, nq;
 };
 
 FusedWs carve(void* base, long long n, const Geo& g, const int K[3], size_t tc, bool grad = false) {
@@ -2111,13 +2181,15 @@ FusedWs carve(void* base, long long n, const Geo& g, const int K[3], size_t tc, 
   int ncols = g.ncol[0] * g.ncol[1];
   w.col_of = (int*)take(4 * nn);
   w.off_in_col = (int*)take(4 * nn);
+  // dead after the scatter; the column sort clears the slots
+  w.es.p = (unsigned long long*)w.off_in_col;
+  w.es.n = (int)(tff_align(4 * nn) / 64 < (size_t)E_SLOTS ? tff_align(4 * nn) / 64 : (size_t)E_SLOTS);
   w.col_count = (int*)take(4 * (size_t)(ncols + 1));
   w.col_start = (int*)take(4 * (size_t)(ncols + 1));
   w.sorted_orig = (int*)take(4 * nn);
   w.col_cl_start = (int*)take(4 * (size_t)(ncols + 1));
-  w.ncl = (int*)take(16);
-  w.ncp = (int*)take(16);
-  w.st = (int*)take(16);
+  w.ncl = (int*)take(32);
+  w.st = w.ncl ? w.ncl + 4 : nullptr;
   w.cl_col = (int*)take(4 * (size_t)g.ncl_max);
   w.slot_orig = (int*)take(4 * slots);
   w.excl_part = (int*)take(4 * slots * MAXEX);
@@ -2128,14 +2200,13 @@ FusedWs carve(void* base, long long n, const Geo& g, const int K[3], size_t tc, 
   w.sb_c = (float4*)take(16 * 4 * (size_t)g.ncl_max);
   w.sb_h = (float4*)take(16 * 4 * (size_t)g.ncl_max);
   w.slot_of_orig = (int*)take(4 * nn);
-  w.cpairs = (int4*)take(16 * (size_t)g.pair_cap);
-  w.seg = (int2*)take(8 * (size_t)g.pair_cap);
-  w.seg_count = (int*)take(4 * (size_t)g.ncl_max);
-  w.seg_start = (int*)take(4 * (size_t)g.ncl_max);
+  w.pl.cap = 4 * g.maxn;  // 4 j-groups per listed cluster pair
+  w.pl.g = (int*)take(4 * 4 * (size_t)g.pair_cap);
+  w.pl.i = (unsigned short*)take(2 * 4 * (size_t)g.pair_cap);
+  w.pl.cnt = (int2*)take(8 * (size_t)g.ncl_max);
   w.facc = (unsigned long long*)take(8 * 3 * slots);
   w.facc_pme = (unsigned long long*)take(8 * 3 * slots);
-  w.nw_tiles = tile_waves(g);
-  w.eacc = (unsigned long long*)take(8 * 2 * E_SLOTS);
+  w.parts = pair_parts(g);
   w.grid = (unsigned long long*)take(8 * ng);
   w.work = take(2 * tc * ng);
   PassCfg px = pass_cfg(1, K[0], K[1] * spectrum_nz(K), 2 * tc);
@@ -2334,11 +2405,9 @@ int run_fused_core(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
       ++cl.count;
     };
     add(w.col_count, ncols + 1);
-    add(w.ncp, 4);
     add(status, 2);
     add(w.facc, 6LL * nslots);
     add(w.slot_orig, nslots);
-    add(w.eacc, 4 * E_SLOTS);
     if (w.bcount) add(w.bcount, (long long)w.bg.nb[0] * w.bg.nb[1] * w.bg.nb[2]);
     hipLaunchKernelGGL(k_clear, dim3(1024), dim3(256), 0, st, cl);
   }
@@ -2349,7 +2418,7 @@ int run_fused_core(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
                      w.ncl, status);
   hipLaunchKernelGGL(k_scatter_atoms, dim3(nbA), dim3(FB), 0, st, n, w.col_of, w.off_in_col, w.col_start,
                      w.sorted_orig);
-  hipLaunchKernelGGL(k_sort_columns<TI>, dim3(ncols), dim3(SORT_THREADS), 0, st, coords, g, w.col_start, w.sorted_orig);
+  hipLaunchKernelGGL(k_sort_columns<TI>, dim3(ncols), dim3(SORT_THREADS), 0, st, coords, g, w.col_start, w.sorted_orig, w.es);
   // 2. cluster arrays
   const unsigned nbW = (unsigned)(((long long)g.ncl_max * TFF_WAVE + FB - 1) / FB);
   const unsigned nbB = (unsigned)(((long long)g.ncl_max * CL + FB - 1) / FB);  // two clusters per wave
@@ -2406,13 +2475,11 @@ int run_fused_core(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
   {
     void* tok = tff_prof_begin("fused_cluster_pairs", st);
     float rl2 = (float)(list_cutoff * list_cutoff);
-    hipLaunchKernelGGL(k_cluster_pairs, dim3(nbW), dim3(FB), 0, st, w.ncl, w.cl_col, w.col_cl_start, w.bb_c,
-                       w.bb_h, g, rl2, w.excl_part, w.seg, w.seg_count, status);
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, w.ncl, w.seg_count, w.seg_start, w.ncp, status);
-    // sub-tiles are pruned at the interaction cutoff itself: pairs between rc and the list
+    // group pairs are pruned at the interaction cutoff itself: pairs between rc and the list
     // cutoff contribute nothing to this evaluation
-    hipLaunchKernelGGL(k_compact_pairs, dim3(nbW), dim3(FB), 0, st, w.ncl, w.seg, w.seg_count, w.seg_start, g.maxn,
-                       w.sb_c, w.sb_h, g, (float)(cutoff * cutoff), w.cpairs);
+    hipLaunchKernelGGL(k_pair_list, dim3(nbW), dim3(FB), 0, st, w.ncl, w.cl_col, w.col_cl_start, w.bb_c, w.bb_h,
+                       w.sb_c, w.sb_h, g, rl2, (float)(cutoff * cutoff), w.excl_part, w.pl,
+                       w.es, status);
     tff_prof_end(tok, st);
   }
   // 5. tiles
@@ -2427,14 +2494,13 @@ int run_fused_core(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
     ta.coul = (TC)coul;
     ta.c2alpha = (TC)(1.1283791670955126 * alpha);
     void* tok = tff_prof_begin("fused_tiles", st);
+    const dim3 nw((unsigned)((long long)g.ncl_max * w.parts));
     if constexpr (sizeof(TC) == 4)
-      hipLaunchKernelGGL(k_tiles_f32, dim3((unsigned)w.nw_tiles), dim3(TFF_WAVE), 0, st, w.cpairs, w.ncp,
-                         g.pair_cap, (const V4<float>*)w.xyzq, (const V2<float>*)w.lj, w.excl_part, ta, w.facc,
-                         w.eacc);
+      hipLaunchKernelGGL(k_tiles_f32, nw, dim3(TFF_WAVE), 0, st, w.ncl, w.pl, w.parts, (const V4<float>*)w.xyzq,
+                         (const V2<float>*)w.lj, w.excl_part, ta, w.facc, w.es);
     else
-      hipLaunchKernelGGL(k_tiles_f64, dim3((unsigned)w.nw_tiles), dim3(TFF_WAVE), 0, st, w.cpairs, w.ncp,
-                         g.pair_cap, (const V4<double>*)w.xyzq, (const V2<double>*)w.lj, w.excl_part, ta, w.facc,
-                         w.eacc);
+      hipLaunchKernelGGL(k_tiles_f64, nw, dim3(TFF_WAVE), 0, st, w.ncl, w.pl, w.parts, (const V4<double>*)w.xyzq,
+                         (const V2<double>*)w.lj, w.excl_part, ta, w.facc, w.es);
     tff_prof_end(tok, st);
   }
   aux_stream_join(st, sp);
@@ -2447,7 +2513,7 @@ template <typename TI>
 int launch_fused_finalize(const FusedWs& w, const Geo& g, double coul, double alpha, double* energies, TI* forces,
                           int* status_out, int* status_host, hipStream_t st) {
   const unsigned nbS = (unsigned)(((long long)g.ncl_max * CL + FB - 1) / FB);
-  hipLaunchKernelGGL(k_finalize<TI>, dim3(nbS), dim3(FB), 0, st, w.ncl, w.slot_orig, w.facc, w.facc_pme, forces, w.eacc,
+  hipLaunchKernelGGL(k_finalize<TI>, dim3(nbS), dim3(FB), 0, st, w.ncl, w.slot_orig, w.facc, w.facc_pme, forces, w.es,
                      w.kparts, w.nk, w.qparts, w.nq, coul, alpha, energies, w.st, status_out, status_host);
   TFF_CHECK_LAUNCH("fused energy+forces");
   return TFF_OK;
@@ -2478,8 +2544,7 @@ int run_fused_grad(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
     };
     if (!reuse) {
       add(w.col_count, ncols + 1);
-      add(w.ncp, 4);
-      add(status, 2);
+        add(status, 2);
       add(w.slot_orig, nslots);
       // the brick counters of the charge spread (float: the forward's list spread runs again)
       if (w.bcount) add(w.bcount, (long long)w.bg.nb[0] * w.bg.nb[1] * w.bg.nb[2]);
@@ -2498,7 +2563,7 @@ int run_fused_grad(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
     hipLaunchKernelGGL(k_scatter_atoms, dim3(nbA), dim3(FB), 0, st, n, w.col_of, w.off_in_col, w.col_start,
                        w.sorted_orig);
     hipLaunchKernelGGL(k_sort_columns<TI>, dim3(ncols), dim3(SORT_THREADS), 0, st, coords, g, w.col_start,
-                       w.sorted_orig);
+                       w.sorted_orig, w.es);
     const unsigned nbB = (unsigned)(((long long)g.ncl_max * CL + FB - 1) / FB);  // two clusters per wave
     hipLaunchKernelGGL((k_build_clusters<TI, TC>), dim3(nbB), dim3(FB), 0, st, coords, q, sig, eps, g, w.ncl,
                        w.col_cl_start, w.col_start, w.sorted_orig, (V4<TC>*)w.xyzq, (V2<TC>*)w.lj, w.slot_orig,
@@ -2519,11 +2584,9 @@ int run_fused_grad(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
   if (!reuse) {
     hipLaunchKernelGGL(k_fill_exclusions, dim3(nbS), dim3(FB), 0, st, w.ncl, w.slot_orig, w.slot_of_orig, n,
                        row_ptr, col, w.excl_part, status);
-    hipLaunchKernelGGL(k_cluster_pairs, dim3(nbW), dim3(FB), 0, st, w.ncl, w.cl_col, w.col_cl_start, w.bb_c,
-                       w.bb_h, g, (float)(list_cutoff * list_cutoff), w.excl_part, w.seg, w.seg_count, status);
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, w.ncl, w.seg_count, w.seg_start, w.ncp, status);
-    hipLaunchKernelGGL(k_compact_pairs, dim3(nbW), dim3(FB), 0, st, w.ncl, w.seg, w.seg_count, w.seg_start, g.maxn,
-                       w.sb_c, w.sb_h, g, (float)(cutoff * cutoff), w.cpairs);
+    hipLaunchKernelGGL(k_pair_list, dim3(nbW), dim3(FB), 0, st, w.ncl, w.cl_col, w.col_cl_start, w.bb_c, w.bb_h,
+                       w.sb_c, w.sb_h, g, (float)(list_cutoff * list_cutoff), (float)(cutoff * cutoff), w.excl_part,
+                       w.pl, w.es, status);
   }
   {
     TileArgs<TC> ta;
@@ -2536,9 +2599,13 @@ int run_fused_grad(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
     ta.coul = (TC)coul;
     ta.c2alpha = (TC)(1.1283791670955126 * alpha);
     void* tok = tff_prof_begin("fused_grad_tiles", st);
-    hipLaunchKernelGGL(k_tiles_grad<TC>, dim3((unsigned)w.nw_tiles), dim3(TFF_WAVE), 0, st, w.cpairs, w.ncp,
-                       g.pair_cap, (const V4<TC>*)w.xyzq, (const V2<TC>*)w.lj, (const V4<TC>*)w.vsl, w.excl_part, ta,
-                       gE, w.gacc);
+    const dim3 nw((unsigned)((long long)g.ncl_max * w.parts));
+    if constexpr (sizeof(TC) == 4)
+      hipLaunchKernelGGL(k_tiles_grad_f32, nw, dim3(TFF_WAVE), 0, st, w.ncl, w.pl, w.parts, (const V4<float>*)w.xyzq,
+                         (const V2<float>*)w.lj, (const V4<float>*)w.vsl, w.excl_part, ta, gE, w.gacc);
+    else
+      hipLaunchKernelGGL(k_tiles_grad_f64, nw, dim3(TFF_WAVE), 0, st, w.ncl, w.pl, w.parts, (const V4<double>*)w.xyzq,
+                         (const V2<double>*)w.lj, (const V4<double>*)w.vsl, w.excl_part, ta, gE, w.gacc);
     tff_prof_end(tok, st);
   }
   PmeGeom pg = make_geom(box, K, order, alpha);
@@ -2581,7 +2648,7 @@ int run_fused_grad(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
 #undef TFF_GRAD_PME
   aux_stream_join(st, sp);
   hipLaunchKernelGGL(k_finalize_grad<TI>, dim3(nbS), dim3(FB), 0, st, w.ncl, w.slot_orig, w.gacc, w.gpme, q, coul,
-                     alpha, gE, dr, dq, dsig, deps, status, status_host);
+                     alpha, gE, dr, dq, dsig, deps, w.es, status, status_host);
   TFF_CHECK_LAUNCH("fused energy+forces backward");
   return TFF_OK;
 }
