@@ -24,13 +24,13 @@
 // bit for bit on every run of the same pair list.  Global atomics cost one
 // memory-side operation per 64-byte line an instruction touches, whatever the
 // number of lanes on that line, so an atom's words sit in one line (x, y, z, q:
-// four high and four low words) plus a 32-byte record for sigma and epsilon,
-// and a wave issues them transposed: it compacts the atoms it updates into LDS
-// and eight adjacent lanes write one atom's line.  Consecutive rows that share
-// an atom (the i side of a cell-list pair list) are summed first by a
-// segmented scan, so such a run costs one line; the j side goes through a
-// per-wave LDS hash of atoms (exact integer words), so each distinct atom of a
-// wave step costs one line.  The integer sums hold up to
+// four high and four low words) plus a 32-byte record for sigma and epsilon.
+// Calls for coordinate and charge gradients (k_pair_xyzq) sum a chunk of rows in
+// an LDS table of atoms first; calls that also want sigma / epsilon gradients
+// (k_pair_terms) sum per wave: consecutive rows that share an atom (the i side of a
+// cell-list pair list) by a segmented scan, the j side through a per-wave LDS hash
+// (exact integer words), then issue the words transposed, eight adjacent lanes
+// per line.  The integer sums hold up to
 // 2^39 per atom; contributions (run sums) of magnitude 2^30 or more
 // (near-overlapping atoms) go to float64 atomics instead, so an atom's integer
 // sum would need 512 such contributions to overflow.  The
@@ -41,6 +41,8 @@
 // ones take float64 atomics).  eps-gradient of a pair
 // whose mixed epsilon is zero (e.g. TIP3P hydrogens) is defined as zero; the
 // exact derivative of sqrt(eps_i eps_j) is unbounded there.
+
+#include <atomic>
 
 #include "tff_common.h"
 #include "torchff_hip.h"
@@ -275,7 +277,111 @@ __device__ __forceinline__ void wave_accum_table(bool act, long long key, const 
   }
 }
 
-// chmask bits: channels of the per-atom accumulator to fill; tmask: sigma / epsilon gradients
+// One listed pair within the cutoff: energy, dE/dr / r (so grad_i = dedr_over_r * d), the charge
+// derivatives and (LJG) the Lennard-Jones parameter derivatives.
+template <typename T>
+struct PairEval {
+  T e, dedr_over_r, dq_i, dq_j;
+  T dsig, deps;       // dE/dsigma_ij, dE/deps_ij
+  T deps_i, deps_j;   // per-atom epsilon (Lorentz-Berthelot modes)
+};
+
+template <typename T, int MODE, bool LJG>
+__device__ __forceinline__ PairEval<T> eval_pair(T r2, long long i, long long j, long long idx, long long tix,
+                                                 bool is_excl, const PairArgs& a, const T* __restrict__ q,
+                                                 const T* __restrict__ sig, const T* __restrict__ eps) {
+  PairEval<T> o{};
+  const T rinv = (T)1 / sqrt(r2);
+  const T rinv2 = rinv * rinv;
+  // ---- Coulomb part
+  if (MODE == TFF_PAIR_NONBONDED) {
+    const T qq = q[i] * q[j] * (T)a.coul;
+    const T shift = a.do_shift ? (T)(1.0 / a.cutoff) : (T)0;
+    o.e += qq * (rinv - shift);
+    o.dedr_over_r += -qq * rinv * rinv2;
+    const T tmp = (rinv - shift) * (T)a.coul;
+    o.dq_i = q[j] * tmp;
+    o.dq_j = q[i] * tmp;
+  } else if (MODE == TFF_PAIR_EWALD_LJ || MODE == TFF_PAIR_COUL_EWALD || MODE == TFF_PAIR_COUL_EWALD_SYM) {
+    const T two_over_sqrt_pi = (T)1.1283791670955126;
+    T d0, d1;
+    if (a.alpha >= 0) {
+      const T r = r2 * rinv;
+      const T u = (T)a.alpha * r;
+      const T ec = erfc(u);
+      const T ex = exp(-u * u) * two_over_sqrt_pi * u;
+      d0 = ec;
+      d1 = ec + ex;
+      if (is_excl) {
+        d0 -= (T)1;
+        d1 -= (T)1;
+      }
+    } else {
+      d0 = 1;
+      d1 = 1;
+    }
+    // COUL_EWALD_SYM: the symmetric product of the charges q and the second array (sig)
+    const T qq = (MODE == TFF_PAIR_COUL_EWALD_SYM ? (T)0.5 * (q[i] * sig[j] + sig[i] * q[j]) : q[i] * q[j]) *
+                 (T)a.coul;
+    o.e += qq * d0 * rinv;
+    o.dedr_over_r += -qq * d1 * rinv * rinv2;
+    if (MODE != TFF_PAIR_COUL_EWALD_SYM) {
+      const T tmp = d0 * rinv * (T)a.coul;
+      o.dq_i = q[j] * tmp;
+      o.dq_j = q[i] * tmp;
+    }
+  }
+  // ---- Lennard-Jones part (never on exclusion-correction pairs)
+  if (MODE != TFF_PAIR_COUL_EWALD && MODE != TFF_PAIR_COUL_EWALD_SYM && !is_excl) {
+    T sij, eij;
+    if (MODE == TFF_PAIR_LJ_TYPES) {
+      sij = sig[tix];
+      eij = eps[tix];
+    } else if (MODE == TFF_PAIR_LJ_PAIRS) {
+      sij = sig[idx];
+      eij = eps[idx];
+    } else {
+      sij = (sig[i] + sig[j]) * (T)0.5;
+      eij = sqrt(eps[i] * eps[j]);
+    }
+    const T sr2 = sij * sij * rinv2;
+    const T s6 = sr2 * sr2 * sr2;
+    o.e += (T)4 * eij * s6 * (s6 - (T)1);
+    o.dedr_over_r += -(T)24 * eij * s6 * ((T)2 * s6 - (T)1) * rinv2;
+    if (LJG) {
+      o.dsig = (T)24 * eij * s6 * ((T)2 * s6 - (T)1) / sij;
+      o.deps = (T)4 * s6 * (s6 - (T)1);
+      if (MODE != TFF_PAIR_LJ_TYPES && MODE != TFF_PAIR_LJ_PAIRS && eij > (T)0) {
+        const T h = o.deps * (T)0.5 / eij;
+        o.deps_i = h * eps[j];
+        o.deps_j = h * eps[i];
+      }
+    }
+  }
+  return o;
+}
+
+// Row idx of the pair list followed by the exclusion list: its atoms (negative rows are padding; indices
+// past natoms are ignored rather than dereferenced)
+struct PairRow {
+  long long i, j;
+  bool is_excl, valid;
+};
+__device__ __forceinline__ PairRow load_row(const long long* __restrict__ pairs, long long P,
+                                            const long long* __restrict__ pexcl, long long total, long long idx,
+                                            long long natoms) {
+  PairRow r{-1, -1, idx >= P, false};
+  if (idx < total) {
+    const long long* pr = r.is_excl ? pexcl + 2 * (idx - P) : pairs + 2 * idx;
+    r.i = pr[0];
+    r.j = pr[1];
+  }
+  r.valid = idx < total && r.i >= 0 && r.j >= 0 && r.i < natoms && r.j < natoms;
+  return r;
+}
+
+// The general kernel (sigma / epsilon gradients).  chmask bits: channels of the per-atom accumulator to
+// fill; tmask: sigma / epsilon gradients
 // of the type table (LJ_TYPES), per-workgroup partials in tab_part (or float64 atomics into
 // tab_ovf for tables above TAB_MAX entries); b: the second charge array of COUL_EWALD_SYM.
 template <typename T, int MODE>
@@ -301,24 +407,15 @@ __global__ __launch_bounds__(PB) void k_pair_terms(const T* __restrict__ coords,
   double e_acc = 0.0;
   const long long total = P + PE;
   const T rc2 = (T)a.cutoff2;
-  const T inv_rc = (T)(1.0 / a.cutoff);
-  const T two_over_sqrt_pi = (T)1.1283791670955126;
   const int lane = threadIdx.x & (TFF_WAVE - 1);
   const long long wave_base = blockIdx.x * (long long)PB + (threadIdx.x - lane);
   const long long stride = (long long)gridDim.x * PB;
   // every lane of a wave runs the same iterations (the accumulation is a wave-wide step)
   for (long long base = wave_base; base < total; base += stride) {
     const long long idx = base + lane;
-    const bool is_excl = idx >= P;
-    long long i = -1, j = -1;
-    if (idx < total) {
-      const long long* pr = is_excl ? pexcl + 2 * (idx - P) : pairs + 2 * idx;
-      i = pr[0];
-      j = pr[1];
-    }
-    // negative rows are padding; indices past natoms are ignored rather than dereferenced
-    const bool valid = idx < total && i >= 0 && j >= 0 && i < natoms && j < natoms;
-    bool act = valid;
+    const PairRow r = load_row(pairs, P, pexcl, total, idx, natoms);
+    const long long i = r.i, j = r.j;
+    bool act = r.valid;
     double vi[NCH] = {0, 0, 0, 0, 0, 0}, vj[NCH] = {0, 0, 0, 0, 0, 0}, vt[2] = {0, 0};
     long long tix = 0;
     if (act) {
@@ -334,101 +431,39 @@ __global__ __launch_bounds__(PB) void k_pair_terms(const T* __restrict__ coords,
         tix = act ? ti * a.ntypes + tj : 0;
       }
       if (act) {
-        const T rinv = (T)1 / sqrt(r2);
-        const T rinv2 = rinv * rinv;
-        T e = 0, dedr_over_r = 0;  // dE/dr / r, so grad_i = dedr_over_r * d
-        // ---- Coulomb part
-        if (MODE == TFF_PAIR_NONBONDED) {
-          const T qq = q[i] * q[j] * (T)a.coul;
-          const T shift = a.do_shift ? inv_rc : (T)0;
-          e += qq * (rinv - shift);
-          dedr_over_r += -qq * rinv * rinv2;
-          const T tmp = (rinv - shift) * (T)a.coul;
-          vi[3] = (double)(q[j] * tmp);
-          vj[3] = (double)(q[i] * tmp);
-        } else if (MODE == TFF_PAIR_EWALD_LJ || MODE == TFF_PAIR_COUL_EWALD || MODE == TFF_PAIR_COUL_EWALD_SYM) {
-          T d0, d1;
-          if (a.alpha >= 0) {
-            const T r = r2 * rinv;
-            const T u = (T)a.alpha * r;
-            const T ec = erfc(u);
-            const T ex = exp(-u * u) * two_over_sqrt_pi * u;
-            d0 = ec;
-            d1 = ec + ex;
-            if (is_excl) {
-              d0 -= (T)1;
-              d1 -= (T)1;
-            }
-          } else {
-            d0 = 1;
-            d1 = 1;
-          }
-          // COUL_EWALD_SYM: the symmetric product of the charges q and the second array (sig)
-          const T qq = (MODE == TFF_PAIR_COUL_EWALD_SYM ? (T)0.5 * (q[i] * sig[j] + sig[i] * q[j]) : q[i] * q[j]) *
-                       (T)a.coul;
-          e += qq * d0 * rinv;
-          dedr_over_r += -qq * d1 * rinv * rinv2;
-          if (MODE != TFF_PAIR_COUL_EWALD_SYM) {
-            const T tmp = d0 * rinv * (T)a.coul;
-            vi[3] = (double)(q[j] * tmp);
-            vj[3] = (double)(q[i] * tmp);
-          }
+        const PairEval<T> o = eval_pair<T, MODE, true>(r2, i, j, idx, tix, r.is_excl, a, q, sig, eps);
+        e_acc += (double)o.e;
+        vi[3] = (double)o.dq_i;
+        vj[3] = (double)o.dq_j;
+        vt[0] = (double)o.dsig;
+        vt[1] = (double)o.deps;
+        if (MODE == TFF_PAIR_LJ_PAIRS) {
+          if (g_sig_pairs) g_sig_pairs[idx] = o.dsig;
+          if (g_eps_pairs) g_eps_pairs[idx] = o.deps;
+        } else if (MODE != TFF_PAIR_LJ_TYPES) {
+          vi[4] = vj[4] = (double)(o.dsig * (T)0.5);
+          vi[5] = (double)o.deps_i;
+          vj[5] = (double)o.deps_j;
         }
-        // ---- Lennard-Jones part (never on exclusion-correction pairs)
-        if (MODE != TFF_PAIR_COUL_EWALD && MODE != TFF_PAIR_COUL_EWALD_SYM && !is_excl) {
-          T sij, eij;
-          if (MODE == TFF_PAIR_LJ_TYPES) {
-            sij = sig[tix];
-            eij = eps[tix];
-          } else if (MODE == TFF_PAIR_LJ_PAIRS) {
-            sij = sig[idx];
-            eij = eps[idx];
-          } else {
-            sij = (sig[i] + sig[j]) * (T)0.5;
-            eij = sqrt(eps[i] * eps[j]);
-          }
-          const T sr2 = sij * sij * rinv2;
-          const T s6 = sr2 * sr2 * sr2;
-          e += (T)4 * eij * s6 * (s6 - (T)1);
-          dedr_over_r += -(T)24 * eij * s6 * ((T)2 * s6 - (T)1) * rinv2;
-          const T dsig = (T)24 * eij * s6 * ((T)2 * s6 - (T)1) / sij;  // dE/dsigma_ij
-          const T deps = (T)4 * s6 * (s6 - (T)1);                        // dE/deps_ij
-          if (MODE == TFF_PAIR_LJ_TYPES) {
-            vt[0] = (double)dsig;
-            vt[1] = (double)deps;
-          } else if (MODE == TFF_PAIR_LJ_PAIRS) {
-            if (g_sig_pairs) g_sig_pairs[idx] = dsig;
-            if (g_eps_pairs) g_eps_pairs[idx] = deps;
-          } else {
-            vi[4] = vj[4] = (double)(dsig * (T)0.5);
-            if (eij > (T)0) {
-              const T h = deps * (T)0.5 / eij;
-              vi[5] = (double)(h * eps[j]);
-              vj[5] = (double)(h * eps[i]);
-            }
-          }
-        }
-        e_acc += (double)e;
-        const double gx = (double)(dedr_over_r * dx), gy = (double)(dedr_over_r * dy), gz = (double)(dedr_over_r * dz);
-        vi[0] = gx;
-        vi[1] = gy;
-        vi[2] = gz;
-        vj[0] = -gx;
-        vj[1] = -gy;
-        vj[2] = -gz;
+        vi[0] = (double)(o.dedr_over_r * dx);
+        vi[1] = (double)(o.dedr_over_r * dy);
+        vi[2] = (double)(o.dedr_over_r * dz);
+        vj[0] = -vi[0];
+        vj[1] = -vi[1];
+        vj[2] = -vi[2];
       }
     }
     if (chmask) {
       // i side: runs of one atom summed by a segmented scan, flushed directly; j side: through the
       // wave's hash (both use the hash memory in turn)
       const WaveHash wh{s_hash_k[threadIdx.x / TFF_WAVE], s_hash_w[threadIdx.x / TFF_WAVE]};
-      wave_accum<NCH>(act, valid ? i : -1, vi, chmask, atoms, wh.w, wh.key);
+      wave_accum<NCH>(act, r.valid ? i : -1, vi, chmask, atoms, wh.w, wh.key);
       if (chmask & 15u) {
         hash_clear(wh);
-        hash_add<NCH>(wh, act && valid, (int)j, vj, chmask, atoms);
+        hash_add<NCH>(wh, act && r.valid, (int)j, vj, chmask, atoms);
         hash_flush(wh, chmask, atoms);
       }
-      if (chmask & 48u) wave_accum<NCH>(act, valid ? j : -1, vj, chmask & 48u, atoms, wh.w, wh.key);
+      if (chmask & 48u) wave_accum<NCH>(act, r.valid ? j : -1, vj, chmask & 48u, atoms, wh.w, wh.key);
     }
     if (MODE == TFF_PAIR_LJ_TYPES && tmask)
       wave_accum_table(act, tix, vt, tmask, tab_lds ? s_tab[threadIdx.x / TFF_WAVE] : nullptr, tab_ovf);
@@ -443,6 +478,154 @@ __global__ __launch_bounds__(PB) void k_pair_terms(const T* __restrict__ coords,
       tab_part[(long long)blockIdx.x * 2 * ntab + k] = v;
     }
   }
+}
+
+// Coordinate and charge gradients (the common calls).  A workgroup takes chunks of CHUNK_STEPS * XB
+// consecutive rows and sums both atoms of every pair in an LDS table of atoms (open addressing; two int64
+// words per channel, so the sums do not depend on the order of the adds), then adds each atom's
+// words to its 64-byte line once per chunk.  Consecutive rows of a cell list share their atoms (about
+// four rows per distinct atom in 2048 rows); adding per wave step instead cost 22 M memory-side line
+// operations at 96k atoms (26.6 M rows), which at about 20 G/s bounded the kernel (1389 us in float64
+// against 602 us this way, 2.5 M operations, bound by vector issue).  A row whose atom finds no slot in
+// PROBES steps (a list in random order) goes to the line directly.  Measured: 1024 threads and 2048
+// slots 637 us, 256 and 512 609 us, twice the slots per thread 856 us (one workgroup per CU).
+constexpr int XB = 512;              // threads
+constexpr int XLOG = 10;
+constexpr int XSLOTS = 1 << XLOG;    // atoms per table
+constexpr int XSTRIDE = XSLOTS + 1;  // int64 words per channel word (padded for the flush: 8 words of a slot at a time)
+constexpr int CHUNK_STEPS = 4;       // rows per thread and chunk
+constexpr int XROWS = 8;             // the lanes of a wave take rows this far apart: a run of rows of one atom then
+                                     // falls to several waves instead of colliding in one instruction (685 us at 1)
+constexpr int XBLOCKS = 512;
+constexpr int PROBES = 12;
+
+// v -> words as split_words, by adding 1.5 2^52 (the integer is then the low mantissa bits): three fma and an
+// addition instead of two double-to-int64 conversions
+__device__ __forceinline__ bool split_fast(double v, long long& h, long long& l) {
+  if (!(fabs(v) < 134217728.0)) return split_words(v, h, l);  // 2^27: h 2^24 fits the mantissa
+  constexpr double M = 6755399441055744.0;
+  constexpr long long MB = 0x4338000000000000LL;
+  const double t = fma(v, HI_SCALE, M);
+  h = __double_as_longlong(t) - MB;
+  const double rem = fma(t - M, -1.0 / HI_SCALE, v);  // exact, |.| <= 2^-25
+  l = __double_as_longlong(fma(rem, LO_SCALE, M)) - MB;
+  return true;
+}
+
+struct AtomTable {
+  int* key;        // XSLOTS atom indices, -1 empty
+  long long* w;    // word c of slot s at w[c * XSTRIDE + s]
+};
+
+template <int NC>
+__device__ __forceinline__ void table_add(const AtomTable& t, int atom, const double (&v)[NC], const Acc& acc) {
+  unsigned p = ((unsigned)atom * 2654435761u) >> (32 - XLOG);
+  int slot = -1;
+  for (int k = 0; k < PROBES; ++k) {
+    int old = t.key[p];
+    if (old != atom) old = old == -1 ? atomicCAS(&t.key[p], -1, atom) : old;
+    if (old == -1 || old == atom) {
+      slot = (int)p;
+      break;
+    }
+    p = (p + 1) & (XSLOTS - 1);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    long long hi, lo;
+    if (!split_fast(v[c], hi, lo)) {
+      atomicAdd(acc.ovf + (long long)atom * NCH + c, v[c]);
+    } else if (slot >= 0) {
+      atomicAdd((unsigned long long*)(t.w + c * XSTRIDE + slot), (unsigned long long)hi);
+      atomicAdd((unsigned long long*)(t.w + (NC + c) * XSTRIDE + slot), (unsigned long long)lo);
+    } else {
+      atomicAdd((unsigned long long*)(acc.a + 8LL * atom + c), (unsigned long long)hi);
+      atomicAdd((unsigned long long*)(acc.a + 8LL * atom + 4 + c), (unsigned long long)lo);
+    }
+  }
+}
+
+// NC: channels summed (0: energy only, 3: x, y, z, 4: and the charge)
+template <typename T, int MODE, int NC>
+__global__ __launch_bounds__(XB) void k_pair_xyzq(const T* __restrict__ coords, const long long* __restrict__ pairs,
+                                                  long long P, const long long* __restrict__ pexcl, long long PE,
+                                                  TffBox box, PairArgs a, const T* __restrict__ q,
+                                                  const T* __restrict__ sig, const T* __restrict__ eps,
+                                                  const long long* __restrict__ types, long long natoms,
+                                                  double* __restrict__ e_part, Acc acc, int steps) {
+  extern __shared__ __align__(16) long long s_tab[];
+  const AtomTable tab{reinterpret_cast<int*>(s_tab + 2 * NC * XSTRIDE), s_tab};
+  const int t = threadIdx.x, lane = t & (TFF_WAVE - 1), wv = t / TFF_WAVE;
+  const int row = (wv / XROWS) * TFF_WAVE * XROWS + lane * XROWS + wv % XROWS;
+  if (NC) {
+    for (int k = t; k < XSLOTS; k += XB) {
+      tab.key[k] = -1;
+#pragma unroll
+      for (int c = 0; c < 2 * NC; ++c) tab.w[c * XSTRIDE + k] = 0;
+    }
+    __syncthreads();
+  }
+  double e_acc = 0.0;
+  const long long total = P + PE;
+  const T rc2 = (T)a.cutoff2;
+  const long long chunk = (long long)steps * XB;
+  for (long long c0 = blockIdx.x * chunk; c0 < total; c0 += gridDim.x * chunk) {
+    bool any = false;
+    for (int s = 0; s < steps; ++s) {
+      const long long idx = c0 + (long long)s * XB + row;
+      const PairRow r = load_row(pairs, P, pexcl, total, idx, natoms);
+      if (!r.valid) continue;
+      const long long i = r.i, j = r.j;
+      T dx = coords[3 * i] - coords[3 * j];
+      T dy = coords[3 * i + 1] - coords[3 * j + 1];
+      T dz = coords[3 * i + 2] - coords[3 * j + 2];
+      tff_min_image<T>(box, dx, dy, dz);
+      const T r2 = dx * dx + dy * dy + dz * dz;
+      bool act = r2 <= rc2;
+      long long tix = 0;
+      if (MODE == TFF_PAIR_LJ_TYPES && act) {
+        const long long ti = types[i], tj = types[j];
+        act = ti >= 0 && tj >= 0 && ti < a.ntypes && tj < a.ntypes;
+        tix = act ? ti * a.ntypes + tj : 0;
+      }
+      if (!act) continue;
+      const PairEval<T> o = eval_pair<T, MODE, false>(r2, i, j, idx, tix, r.is_excl, a, q, sig, eps);
+      e_acc += (double)o.e;
+      if constexpr (NC > 0) {
+        any = true;
+        double v[NC];
+        v[0] = (double)(o.dedr_over_r * dx);
+        v[1] = (double)(o.dedr_over_r * dy);
+        v[2] = (double)(o.dedr_over_r * dz);
+        if constexpr (NC > 3) v[3] = (double)o.dq_i;
+        table_add<NC>(tab, (int)i, v, acc);
+        v[0] = -v[0];
+        v[1] = -v[1];
+        v[2] = -v[2];
+        if constexpr (NC > 3) v[3] = (double)o.dq_j;
+        table_add<NC>(tab, (int)j, v, acc);
+      }
+    }
+    if constexpr (NC > 0) {
+      // every filled slot's words to its atom's line (8 lanes a slot: one line each), and the table cleared
+      if (!__syncthreads_or(any)) continue;
+      for (int k = t; k < XSLOTS * 8; k += XB) {
+        const int slot = k >> 3, c = k & 7, cc = c & 3;  // line words: hi x, y, z, q, lo x, y, z, q
+        const int atom = tab.key[slot];
+        if (atom >= 0 && cc < NC) {
+          long long* w = tab.w + ((c >> 2) * NC + cc) * XSTRIDE + slot;
+          const long long v = *w;
+          *w = 0;
+          if (v != 0) atomicAdd((unsigned long long*)(acc.a + 8LL * atom + c), (unsigned long long)v);
+        }
+      }
+      __syncthreads();
+      for (int k = t; k < XSLOTS; k += XB) tab.key[k] = -1;
+      __syncthreads();
+    }
+  }
+  const double tot = tff_block_sum(e_acc);
+  if (t == 0) e_part[blockIdx.x] = tot;
 }
 
 // type-table gradient entry k (of n = 2 ntab): the workgroup partials summed in workgroup order
@@ -532,6 +715,22 @@ PairWs carve(void* base, long long natoms, long long ntab) {
 // entries of the type-table accumulator (LJ_TYPES), else 0
 long long table_len(int mode, long long ntypes) { return mode == TFF_PAIR_LJ_TYPES ? ntypes * ntypes : 0; }
 
+// dynamic LDS above 64 KB has to be allowed per kernel and device, once
+int allow_lds(const void* kernel, size_t bytes, std::atomic<unsigned long long>& ready) {
+  if (bytes <= 65536) return TFF_OK;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  const unsigned long long bit = 1ull << (dev & 63);
+  if (e == hipSuccess && (ready.load() & bit)) return TFF_OK;
+  if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (e != hipSuccess) {
+    tff_set_error("tff_pair_energy: %s", hipGetErrorString(e));
+    return TFF_ERR_LAUNCH;
+  }
+  ready.fetch_or(bit);
+  return TFF_OK;
+}
+
 template <typename T>
 int run(int mode, const T* coords, long long natoms, const TffBox& box, const long long* pairs, long long P,
         const long long* pexcl, long long PE, const T* q, const T* sig, const T* eps, const long long* types,
@@ -562,9 +761,35 @@ int run(int mode, const T* coords, long long natoms, const TffBox& box, const lo
   // per-pair gradients (LJ_PAIRS) are written only for the pairs that contribute
   if (gsp) hipLaunchKernelGGL(k_zero_t<T>, dim3(1024), dim3(256), 0, st, gsp, P);
   if (gep) hipLaunchKernelGGL(k_zero_t<T>, dim3(1024), dim3(256), 0, st, gep, P);
+  // the table kernel where only coordinate / charge gradients (or none) are asked for
+  const bool table = !(chmask & 48u) && !tmask && !gsp && !gep && natoms <= 0x7fffffffLL;
+  // rows per chunk: as many steps as leave every workgroup two chunks (small lists spread over the device)
+  int steps = (int)((P + PE) / (2LL * XBLOCKS * XB));
+  steps = steps < 1 ? 1 : (steps > CHUNK_STEPS ? CHUNK_STEPS : steps);
+  if (table) {
+    blocks = (P + PE + (long long)steps * XB - 1) / ((long long)steps * XB);
+    blocks = blocks > XBLOCKS ? XBLOCKS : (blocks < 1 ? 1 : blocks);
+  }
+  const int nc = chmask & 8u ? 4 : (chmask ? 3 : 0);
+  const size_t lds = nc ? 8 * (size_t)(2 * nc) * XSTRIDE + 4 * (size_t)XSLOTS : 0;
+#define TFF_LAUNCH_TABLE(M, NC)                                                                                  \
+  do {                                                                                                           \
+    static std::atomic<unsigned long long> ready{0};                                                             \
+    const int rc = allow_lds(reinterpret_cast<const void*>(&k_pair_xyzq<T, M, NC>), lds, ready);                 \
+    if (rc) return rc;                                                                                           \
+    hipLaunchKernelGGL((k_pair_xyzq<T, M, NC>), dim3((unsigned)blocks), dim3(XB), lds, st, coords, pairs, P, pexcl, \
+                       PE, box, pa, q, sig, eps, types, natoms, w.e_part, w.atoms, steps);                       \
+  } while (0)
 #define TFF_LAUNCH_PAIR(M)                                                                                       \
-  hipLaunchKernelGGL((k_pair_terms<T, M>), grid, blk, 0, st, coords, pairs, P, pexcl, PE, box, pa, q, sig, eps,   \
-                     types, natoms, w.e_part, chmask, w.atoms, tmask, w.tab_part, w.tab_ovf, gsp, gep)
+  if (table && nc == 0)                                                                                          \
+    TFF_LAUNCH_TABLE(M, 0);                                                                                      \
+  else if (table && nc == 3)                                                                                     \
+    TFF_LAUNCH_TABLE(M, 3);                                                                                      \
+  else if (table)                                                                                                \
+    TFF_LAUNCH_TABLE(M, 4);                                                                                      \
+  else                                                                                                           \
+    hipLaunchKernelGGL((k_pair_terms<T, M>), grid, blk, 0, st, coords, pairs, P, pexcl, PE, box, pa, q, sig, eps, \
+                       types, natoms, w.e_part, chmask, w.atoms, tmask, w.tab_part, w.tab_ovf, gsp, gep)
   void* tok = tff_prof_begin("pair_terms", st);
   switch (mode) {
     case TFF_PAIR_NONBONDED: TFF_LAUNCH_PAIR(TFF_PAIR_NONBONDED); break;
@@ -576,6 +801,7 @@ int run(int mode, const T* coords, long long natoms, const TffBox& box, const lo
     default: tff_set_error("tff_pair_energy: unknown mode %d", mode); return TFF_ERR_ARG;
   }
 #undef TFF_LAUNCH_PAIR
+#undef TFF_LAUNCH_TABLE
   tff_prof_end(tok, st);
   TFF_CHECK_LAUNCH("k_pair_terms");
   if (energy) hipLaunchKernelGGL(k_sum_parts<T>, dim3(1), dim3(256), 0, st, w.e_part, (int)blocks, scale, energy);
