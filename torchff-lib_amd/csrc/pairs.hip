@@ -44,6 +44,7 @@
 
 #include <atomic>
 
+#include "pair_math.h"
 #include "tff_common.h"
 #include "torchff_hip.h"
 
@@ -291,7 +292,7 @@ __device__ __forceinline__ PairEval<T> eval_pair(T r2, long long i, long long j,
                                                  bool is_excl, const PairArgs& a, const T* __restrict__ q,
                                                  const T* __restrict__ sig, const T* __restrict__ eps) {
   PairEval<T> o{};
-  const T rinv = (T)1 / sqrt(r2);
+  const T rinv = rsqrt_full(r2);
   const T rinv2 = rinv * rinv;
   // ---- Coulomb part
   if (MODE == TFF_PAIR_NONBONDED) {
@@ -308,8 +309,9 @@ __device__ __forceinline__ PairEval<T> eval_pair(T r2, long long i, long long j,
     if (a.alpha >= 0) {
       const T r = r2 * rinv;
       const T u = (T)a.alpha * r;
-      const T ec = erfc(u);
-      const T ex = exp(-u * u) * two_over_sqrt_pi * u;
+      T ec, em;
+      erfc_exp_full(u, ec, em);
+      const T ex = em * two_over_sqrt_pi * u;
       d0 = ec;
       d1 = ec + ex;
       if (is_excl) {
