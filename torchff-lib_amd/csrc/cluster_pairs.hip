@@ -33,6 +33,9 @@
 // lane l holds atom i of slot 32x + l and atom j of column l, and walks the 32 columns by
 // shuffles.  Pairs come out in entry, lane, column order at offsets from a count pass and a scan.
 
+#include <cmath>
+
+#include "pair_math.h"
 #include "tff_common.h"
 #include "torchff_hip.h"
 
@@ -441,137 +444,253 @@ __global__ void k_cp_npairs(const long long* __restrict__ off, long long total, 
   }
 }
 
-// nonbonded energy and gradients on the cluster pairs: k q_i q_j (1/r - [1/rc]) + 4 eps s^6 (s^6 - 1),
-// sigma and eps by Lorentz-Berthelot, the same pair term as compute_nonbonded_energy_from_atom_pairs
-template <typename T>
-__global__ __launch_bounds__(CPB) void k_cp_nonbonded(const T* __restrict__ coords, CpGeom g, Entries en,
-                                                      const T* __restrict__ q, const T* __restrict__ sig,
-                                                      const T* __restrict__ eps, double coul, int do_shift,
-                                                      double* __restrict__ e_part, double* __restrict__ g_xyz,
-                                                      double* __restrict__ g_q, double* __restrict__ g_sig,
-                                                      double* __restrict__ g_eps) {
+// ---------------------------------------------------------------- nonbonded terms
+// 16-lane row rotation: lane l takes the value of lane l - 1 of its row
+__device__ __forceinline__ int ror1(int v) { return __builtin_amdgcn_mov_dpp(v, 0x121, 0xf, 0xf, true); }
+__device__ __forceinline__ float ror1(float v) { return __int_as_float(ror1(__float_as_int(v))); }
+__device__ __forceinline__ double ror1(double v) {
+  return __hiloint2double(ror1(__double2hiint(v)), ror1(__double2loint(v)));
+}
+__device__ __forceinline__ void half_sync() {  // the wave's own LDS writes before its reads
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// 1 / sqrt(x), sqrt(x) and a / b to within an ulp (float: the hardware's, corrected by one step whose
+// residual is exact; zero, infinite and denormal x as the hardware gives them)
+__device__ __forceinline__ float cp_rsqrt(float x) {
+  const float y = __builtin_amdgcn_rsqf(x), h = x * y;
+  const float e = fmaf(-h, y, 1.0f) - fmaf(x, y, -h) * y;
+  return fabsf(e) < 1.0f ? fmaf(0.5f * y, e, y) : y;
+}
+__device__ __forceinline__ double cp_rsqrt(double x) { return rsqrt_t(x); }
+__device__ __forceinline__ float cp_sqrt(float x) {
+  const float s = __builtin_amdgcn_sqrtf(x), h = 0.5f * __builtin_amdgcn_rsqf(x);
+  float f = fmaf(fmaf(-s, s, x), h, s);
+  const bool mid = x > 1e-30f && x < 1e30f;
+  if (__builtin_amdgcn_ballot_w64(!mid && x != 0.0f)) {  // rare
+    asm volatile("");                                    // (kept a branch)
+    f = mid ? f : sqrtf(x);
+  }
+  return x == 0.0f ? x : f;
+}
+__device__ __forceinline__ double cp_sqrt(double x) { return sqrt(x); }
+__device__ __forceinline__ float cp_div(float a, float b) {
+  const float y = __builtin_amdgcn_rcpf(b), d = a * y;
+  return fabsf(d) < INFINITY ? fmaf(fmaf(-b, d, a), y, d) : d;
+}
+__device__ __forceinline__ double cp_div(double a, double b) { return a / b; }
+
+// Accumulators: CH doubles per atom (x, y, z, q and, with the Lennard-Jones gradients, sigma, eps, -, -),
+// one 32 or 64 byte piece of a line each.
+template <bool LJG>
+struct CpCh {
+  static constexpr int ST = LJG ? 8 : 4;  // doubles per atom
+  static constexpr int N = LJG ? 6 : 4;   // of them in use
+};
+
+// The atoms `a` (one per lane of the half-wave, -1 for none) with N channels each, added to the
+// accumulators: through LDS, so that the lanes of one instruction hold the channels of few atoms.  An
+// atomic costs a memory-side operation per line it touches: one per atom here, one per atom and
+// channel when each lane adds its own atom's.
+template <bool LJG>
+__device__ __forceinline__ void cp_flush(int a, const double (&v)[CpCh<LJG>::N], double* __restrict__ s,
+                                         double* __restrict__ acc) {
+  constexpr int ST = CpCh<LJG>::ST, N = CpCh<LJG>::N, PAD = ST + 1;
   const int l = half_lane();
-  const long long total = en.E + en.M;
-  const T inv_rc = (T)(1.0 / g.rc);
-  double e_acc = 0.0;
-  for (long long e = half_index(); e < total; e += half_count()) {
-    int i = -1, j = -1;
-    unsigned skip = 0xffffffffu;
-    const bool live = entry_atoms(en, e, g.natoms, g.nclusters, l, i, j, skip);
-    T xi = 0, yi = 0, zi = 0, qi = 0, si = 0, ei = 0;
-    T xj = 0, yj = 0, zj = 0, qj = 0, sj = 0, ej = 0;
-    if (live && i >= 0) {
-      xi = coords[3 * i]; yi = coords[3 * i + 1]; zi = coords[3 * i + 2];
-      qi = q[i]; si = sig[i]; ei = eps[i];
-    }
-    if (live && j >= 0) {
-      xj = coords[3 * j]; yj = coords[3 * j + 1]; zj = coords[3 * j + 2];
-      qj = q[j]; sj = sig[j]; ej = eps[j];
-    }
-    double fi[3] = {0, 0, 0}, gqi = 0, gsi = 0, gei = 0;
-    for (int c = 0; c < CPW; ++c) {
-      const int jc = __shfl(j, c, 32);
-      const T xc = __shfl(xj, c, 32), yc = __shfl(yj, c, 32), zc = __shfl(zj, c, 32);
-      const T qc = __shfl(qj, c, 32), sc = __shfl(sj, c, 32), ec = __shfl(ej, c, 32);
-      // the pair predicate in float64, as the decoded list
-      double ddx = (double)xi - (double)xc, ddy = (double)yi - (double)yc, ddz = (double)zi - (double)zc;
-      tff_min_image_d(g.box, ddx, ddy, ddz);
-      const bool ok = live && i >= 0 && jc >= 0 && !((skip >> c) & 1u) && ddx * ddx + ddy * ddy + ddz * ddz <= g.rc2;
-      T dedr_over_r = 0, gqc = 0, gsc = 0, gec = 0;
-      T dx = 0, dy = 0, dz = 0;
-      if (ok) {
-        dx = xi - xc;
-        dy = yi - yc;
-        dz = zi - zc;
-        tff_min_image<T>(g.box, dx, dy, dz);
-        const T r2 = dx * dx + dy * dy + dz * dz;
-        const T rinv = (T)1 / sqrt(r2);
-        const T rinv2 = rinv * rinv;
-        const T qq = qi * qc * (T)coul;
-        const T shift = do_shift ? inv_rc : (T)0;
-        T en_ = qq * (rinv - shift);
-        dedr_over_r = -qq * rinv * rinv2;
-        const T tmp = (rinv - shift) * (T)coul;
-        gqi += (double)(qc * tmp);
-        gqc = qi * tmp;
-        const T sij = (si + sc) * (T)0.5;
-        const T eij = sqrt(ei * ec);
-        const T sr2 = sij * sij * rinv2;
-        const T s6 = sr2 * sr2 * sr2;
-        en_ += (T)4 * eij * s6 * (s6 - (T)1);
-        dedr_over_r += -(T)24 * eij * s6 * ((T)2 * s6 - (T)1) * rinv2;
-        const T dsig = (T)24 * eij * s6 * ((T)2 * s6 - (T)1) / sij;
-        const T deps = (T)4 * s6 * (s6 - (T)1);
-        gsi += (double)(dsig * (T)0.5);
-        gsc = dsig * (T)0.5;
-        if (eij > (T)0) {
-          const T de = deps * (T)0.5 / eij;
-          gei += (double)(de * ec);
-          gec = de * ei;
-        }
-        e_acc += (double)en_;
-        fi[0] += (double)(dedr_over_r * dx);
-        fi[1] += (double)(dedr_over_r * dy);
-        fi[2] += (double)(dedr_over_r * dz);
-      }
-      // the column atom's share: summed over the half-wave in the input precision (only the
-      // requested gradients), one atomic per column
-      const unsigned any = half_ballot(ok);
-      if (any) {
-        if (g_xyz) {
-          T cx = ok ? -(dedr_over_r * dx) : (T)0, cy = ok ? -(dedr_over_r * dy) : (T)0,
-            cz = ok ? -(dedr_over_r * dz) : (T)0;
-          for (int o = 16; o > 0; o >>= 1) {
-            cx += __shfl_xor(cx, o, 32);
-            cy += __shfl_xor(cy, o, 32);
-            cz += __shfl_xor(cz, o, 32);
-          }
-          if (l == c) {
-            atomicAdd(&g_xyz[3 * jc], (double)cx);
-            atomicAdd(&g_xyz[3 * jc + 1], (double)cy);
-            atomicAdd(&g_xyz[3 * jc + 2], (double)cz);
-          }
-        }
-        if (g_q || g_sig || g_eps) {
-          T cq = ok ? gqc : (T)0, cs = ok ? gsc : (T)0, ce = ok ? gec : (T)0;
-          for (int o = 16; o > 0; o >>= 1) {
-            cq += __shfl_xor(cq, o, 32);
-            cs += __shfl_xor(cs, o, 32);
-            ce += __shfl_xor(ce, o, 32);
-          }
-          if (l == c) {
-            if (g_q) atomicAdd(&g_q[jc], (double)cq);
-            if (g_sig) atomicAdd(&g_sig[jc], (double)cs);
-            if (g_eps) atomicAdd(&g_eps[jc], (double)ce);
-          }
-        }
-      }
-    }
-    if (live && i >= 0) {
-      if (g_xyz && (fi[0] != 0.0 || fi[1] != 0.0 || fi[2] != 0.0)) {
-        atomicAdd(&g_xyz[3 * i], fi[0]);
-        atomicAdd(&g_xyz[3 * i + 1], fi[1]);
-        atomicAdd(&g_xyz[3 * i + 2], fi[2]);
-      }
-      if (g_q && gqi != 0.0) atomicAdd(&g_q[i], gqi);
-      if (g_sig && gsi != 0.0) atomicAdd(&g_sig[i], gsi);
-      if (g_eps && gei != 0.0) atomicAdd(&g_eps[i], gei);
+  half_sync();
+#pragma unroll
+  for (int k = 0; k < N; ++k) s[l * PAD + k] = v[k];
+  half_sync();
+  const int k = l % ST;
+#pragma unroll
+  for (int r = 0; r < ST; ++r) {
+    const int m = r * (CPW / ST) + l / ST;
+    const int am = __shfl(a, m, 32);
+    if (k < N && am >= 0) {
+      const double x = s[m * PAD + k];
+      if (x != 0.0) atomicAdd(&acc[(size_t)am * ST + k], x);
     }
   }
-  const double s = tff_block_sum(e_acc);
-  if (threadIdx.x == 0) e_part[blockIdx.x] = s;
 }
 
-template <typename T>
-__global__ void k_cp_energy_final(const double* __restrict__ part, int n, double scale, T* __restrict__ out) {
-  const double s = tff_sum_partials(part, n);
-  if (threadIdx.x == 0) out[0] = (T)(s * scale);
+// nonbonded energy and gradients on the cluster pairs: k q_i q_j (1/r - [1/rc]) + 4 eps s^6 (s^6 - 1),
+// sigma and eps by Lorentz-Berthelot, the same pair term as compute_nonbonded_energy_from_atom_pairs.
+// GRAD: 0 energy only, 1 with coordinates and charges, 2 with sigma and epsilon too.
+//
+// A half-wave takes a run of consecutive entries (they mostly share their cluster x, whose atoms' sums
+// stay in registers, float64, until x changes).  Its two rows of 16 lanes take 16 of the column atoms
+// each, which then go round the row by DPP together with their sums (T, at most 32 terms, as the
+// sums of a column by butterfly would be), 16 steps, twice: no shuffle and no reduction per column.
+// The pair predicate is that of the decoded list, in float64: T = float decides by its own r^2
+// unless that is within its error bound `tol_k` (|d| + box) of rc^2.
+// Bound by the arithmetic of the candidate pairs (of 32 x 32 per entry about one in five is within the
+// cutoff).  96k water atoms, float, all gradients: 315 us; one column per step by shuffles, a
+// butterfly per gradient and an atomic per atom and channel took 683.
+template <typename T, int GRAD>
+__global__ __launch_bounds__(CPB) void k_cp_nonbonded(const T* __restrict__ coords, CpGeom g, Entries en, int run,
+                                                      const T* __restrict__ q, const T* __restrict__ sig,
+                                                      const T* __restrict__ eps, double coul, int do_shift, T tol_k,
+                                                      T tol_l, double* __restrict__ e_part,
+                                                      double* __restrict__ acc) {
+  constexpr bool LJG = GRAD == 2;
+  constexpr int N = GRAD ? CpCh<LJG>::N : 1;
+  __shared__ double s_fl[GRAD ? (CPB / 32) * CPW * (CpCh<LJG>::ST + 1) : 1];
+  double* s = s_fl + (GRAD ? (threadIdx.x >> 5) * CPW * (CpCh<LJG>::ST + 1) : 0);
+  const int l = half_lane(), l16 = l & 15;
+  const long long total = en.E + en.M;
+  const T shift = do_shift ? (T)(1.0 / g.rc) : (T)0, kc = (T)coul, rc2 = (T)g.rc2;
+  double e_acc = 0.0;
+  const long long runs = (total + run - 1) / run;
+  for (long long r0 = half_index() & ~1; r0 < runs; r0 += half_count()) {  // both halves of a wave together
+    const long long e0 = (r0 + (half_index() & 1)) * run;
+    double fi[N];
+    for (int k = 0; k < N; ++k) fi[k] = 0.0;
+    int i = -1, x_of = -1;
+    T xi = 0, yi = 0, zi = 0, qi = 0, si = 0, ei = 0;
+    for (int n = 0; n < run; ++n) {
+      const long long e = e0 + n;
+      int in = -1, j = -1, x = -1;
+      unsigned skip = 0xffffffffu;
+      if (e < total && entry_atoms(en, e, g.natoms, g.nclusters, l, in, j, skip))
+        x = e < en.E ? en.coo[e] : en.ic[e - en.E];
+      if (x < 0) {  // past the end or padding
+        in = i;
+        x = x_of;
+        j = -1;
+      }
+      if (x != x_of) {
+        if constexpr (GRAD != 0) {
+          if (x_of >= 0) cp_flush<LJG>(i, fi, s, acc);
+          for (int k = 0; k < N; ++k) fi[k] = 0.0;
+        }
+        x_of = x;
+        i = in;
+        if (i >= 0) {
+          xi = coords[3 * i]; yi = coords[3 * i + 1]; zi = coords[3 * i + 2];
+          qi = q[i]; si = sig[i]; ei = eps[i];
+        }
+      }
+      T xj = 0, yj = 0, zj = 0, qj = 0, sj = 0, ej = 0;
+      if (j >= 0) {
+        xj = coords[3 * j]; yj = coords[3 * j + 1]; zj = coords[3 * j + 2];
+        qj = q[j]; sj = sig[j]; ej = eps[j];
+      }
+      skip |= half_ballot(j < 0);
+      if (i < 0) skip = 0xffffffffu;
+      T gj[N];
+      for (int k = 0; k < N; ++k) gj[k] = 0;
+      for (int h = 0; h < 2; ++h) {
+        // bit 16 - k of `todo`: the pair of step k (column (l16 - k) & 15 of the row's block)
+        const unsigned m16 = ((l >> 4) ^ h ? skip >> 16 : skip) & 0xffffu;
+        unsigned todo = ~((m16 | m16 << 16) >> l16);
+        for (int c = 0; c < 16; ++c) {
+          T dx = xi - xj, dy = yi - yj, dz = zi - zj;
+          const T raw = fabs(dx) + fabs(dy) + fabs(dz);
+          tff_min_image<T>(g.box, dx, dy, dz);
+          T r2 = dx * dx + dy * dy + dz * dz;
+          bool ok = (todo & 0x10000u) != 0;
+          if constexpr (sizeof(T) == 8) {
+            double ax = (double)xi - (double)xj, ay = (double)yi - (double)yj, az = (double)zi - (double)zj;
+            tff_min_image_d(g.box, ax, ay, az);
+            ok = ok && ax * ax + ay * ay + az * az <= g.rc2;
+          } else {
+            const T gap = r2 - rc2, tol = tol_k * (raw + tol_l);
+            if (ok && !(gap < -tol || gap > tol)) {
+              double ax = (double)xi - (double)xj, ay = (double)yi - (double)yj, az = (double)zi - (double)zj;
+              tff_min_image_d(g.box, ax, ay, az);
+              ok = ax * ax + ay * ay + az * az <= g.rc2;
+            } else {
+              ok = ok && gap < 0;
+            }
+          }
+          if (ok) {
+            const T rinv = cp_rsqrt(r2), rinv2 = rinv * rinv;
+            const T qq = qi * qj * kc;
+            T en_ = qq * (rinv - shift);
+            T dr = -qq * rinv * rinv2;
+            const T sij = (si + sj) * (T)0.5, eij = cp_sqrt(ei * ej);
+            const T sr2 = sij * sij * rinv2, s6 = sr2 * sr2 * sr2;
+            en_ += (T)4 * eij * s6 * (s6 - (T)1);
+            const T w = (T)24 * eij * s6 * ((T)2 * s6 - (T)1);
+            dr -= w * rinv2;
+            e_acc += (double)en_;
+            if constexpr (GRAD != 0) {
+              const T gq = (rinv - shift) * kc;
+              fi[0] += (double)(dr * dx);
+              fi[1] += (double)(dr * dy);
+              fi[2] += (double)(dr * dz);
+              fi[3] += (double)(qj * gq);
+              gj[0] -= dr * dx;
+              gj[1] -= dr * dy;
+              gj[2] -= dr * dz;
+              gj[3] += qi * gq;
+            }
+            if constexpr (LJG) {
+              const T ds = cp_div(w, sij) * (T)0.5;
+              const T de = eij > (T)0 ? cp_div((T)4 * s6 * (s6 - (T)1) * (T)0.5, eij) : (T)0;
+              fi[4] += (double)ds;
+              fi[5] += (double)(de * ej);
+              gj[4] += ds;
+              gj[5] += de * ei;
+            }
+          }
+          if constexpr (GRAD != 0)
+            for (int k = 0; k < N; ++k) gj[k] = ror1(gj[k]);
+          sj = ror1(sj);
+          ej = ror1(ej);
+          xj = ror1(xj);
+          yj = ror1(yj);
+          zj = ror1(zj);
+          qj = ror1(qj);
+          todo <<= 1;
+        }
+        // the other row's columns and their sums (twice: every lane ends with its own column)
+        xj = __shfl_xor(xj, 16, 32);
+        yj = __shfl_xor(yj, 16, 32);
+        zj = __shfl_xor(zj, 16, 32);
+        qj = __shfl_xor(qj, 16, 32);
+        sj = __shfl_xor(sj, 16, 32);
+        ej = __shfl_xor(ej, 16, 32);
+        if constexpr (GRAD != 0)
+          for (int k = 0; k < N; ++k) gj[k] = __shfl_xor(gj[k], 16, 32);
+      }
+      if constexpr (GRAD != 0) {
+        double gd[N];
+        for (int k = 0; k < N; ++k) gd[k] = (double)gj[k];
+        cp_flush<LJG>(j, gd, s, acc);
+      }
+    }
+    if constexpr (GRAD != 0)
+      if (x_of >= 0) cp_flush<LJG>(i, fi, s, acc);
+  }
+  const double sum = tff_block_sum(e_acc);
+  if (threadIdx.x == 0) e_part[blockIdx.x] = sum;
 }
 
+// energy (block 0) and the requested gradients from the accumulators (st doubles per atom)
 template <typename T>
-__global__ void k_cp_cast(const double* __restrict__ s, long long n, double scale, int accumulate, T* __restrict__ d) {
-  for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n; k += (long long)gridDim.x * blockDim.x)
-    d[k] = accumulate ? d[k] + (T)(s[k] * scale) : (T)(s[k] * scale);
+struct CpOut {
+  T *energy, *g_xyz, *g_q, *g_sig, *g_eps, *forces;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void k_cp_finish(const double* __restrict__ part, int nparts,
+                                                   const double* __restrict__ acc, int st, long long n, double scale,
+                                                   CpOut<T> o) {
+  for (long long k = blockIdx.x * 256LL + threadIdx.x; k < n; k += (long long)gridDim.x * 256) {
+    const double* a = acc + k * st;
+    if (o.g_xyz)
+      for (int c = 0; c < 3; ++c) o.g_xyz[3 * k + c] = (T)(a[c] * scale);
+    if (o.forces)
+      for (int c = 0; c < 3; ++c) o.forces[3 * k + c] += (T)(a[c] * -scale);
+    if (o.g_q) o.g_q[k] = (T)(a[3] * scale);
+    if (o.g_sig) o.g_sig[k] = (T)(a[4] * scale);
+    if (o.g_eps) o.g_eps[k] = (T)(a[5] * scale);
+  }
+  if (o.energy && blockIdx.x == 0) {
+    const double s = tff_sum_partials(part, nparts);
+    if (threadIdx.x == 0) o.energy[0] = (T)(s * scale);
+  }
 }
 
 __global__ void k_cp_zero_d(double* p, long long n) {
@@ -741,10 +860,7 @@ struct TravWs {
   int* cnt;
   long long* off;
   double* e_part;
-  double* g_xyz;
-  double* g_q;
-  double* g_sig;
-  double* g_eps;
+  double* acc;  // 8 doubles per atom
   size_t bytes;
 };
 
@@ -760,10 +876,7 @@ TravWs carve_trav(void* base, long long natoms, long long entries) {
   w.cnt = (int*)take(4 * (size_t)entries);
   w.off = (long long*)take(8 * ((size_t)entries + 1));
   w.e_part = (double*)take(8 * (size_t)CP_MAXBLK);
-  w.g_xyz = (double*)take(24 * (size_t)natoms);
-  w.g_q = (double*)take(8 * (size_t)natoms);
-  w.g_sig = (double*)take(8 * (size_t)natoms);
-  w.g_eps = (double*)take(8 * (size_t)natoms);
+  w.acc = (double*)take(64 * (size_t)natoms);
   w.bytes = off;
   return w;
 }
@@ -925,51 +1038,54 @@ extern "C" int tff_cluster_pairs_nonbonded(int dtype, const void* coords, long l
     tff_set_error("tff_cluster_pairs_nonbonded: workspace too small (%zu < %zu)", workspace_bytes, w.bytes);
     return TFF_ERR_WORKSPACE;
   }
-  const bool need_xyz = grad_coords || forces_accum;
-  auto zero = [&](double* p, long long n) {
-    long long b = (n + 255) / 256;
-    if (b > 4096) b = 4096;
-    if (b < 1) b = 1;
-    hipLaunchKernelGGL(k_cp_zero_d, dim3((unsigned)b), dim3(256), 0, stream, p, n);
+  const int grad = grad_sigma || grad_epsilon ? 2 : (grad_coords || forces_accum || grad_charges ? 1 : 0);
+  const int stride = grad == 2 ? 8 : 4;
+  auto blocks = [](long long n) {
+    const long long b = (n + 255) / 256;
+    return dim3((unsigned)(b < 1 ? 1 : b > 4096 ? 4096 : b));
   };
-  if (need_xyz) zero(w.g_xyz, 3 * natoms);
-  if (grad_charges) zero(w.g_q, natoms);
-  if (grad_sigma) zero(w.g_sig, natoms);
-  if (grad_epsilon) zero(w.g_eps, natoms);
-  const unsigned gt = grid_for(1, total);
-  double* gx = need_xyz ? w.g_xyz : nullptr;
-  double* gq = grad_charges ? w.g_q : nullptr;
-  double* gs = grad_sigma ? w.g_sig : nullptr;
-  double* ge = grad_epsilon ? w.g_eps : nullptr;
-  auto cast = [&](auto tag, const double* s, long long n, double sc, int acc, void* d) {
-    using TT = decltype(tag);
-    long long b = (n + 255) / 256;
-    if (b > 4096) b = 4096;
-    if (b < 1) b = 1;
-    hipLaunchKernelGGL(k_cp_cast<TT>, dim3((unsigned)b), dim3(256), 0, stream, s, n, sc, acc, (TT*)d);
-  };
-  auto finish = [&](auto tag) {
-    using TT = decltype(tag);
-    if (energy_out)
-      hipLaunchKernelGGL(k_cp_energy_final<TT>, dim3(1), dim3(256), 0, stream, (const double*)w.e_part, (int)gt,
-                         scale, (TT*)energy_out);
-    if (grad_coords) cast(tag, w.g_xyz, 3 * natoms, scale, 0, grad_coords);
-    if (forces_accum) cast(tag, w.g_xyz, 3 * natoms, -scale, 1, forces_accum);
-    if (grad_charges) cast(tag, w.g_q, natoms, scale, 0, grad_charges);
-    if (grad_sigma) cast(tag, w.g_sig, natoms, scale, 0, grad_sigma);
-    if (grad_epsilon) cast(tag, w.g_eps, natoms, scale, 0, grad_epsilon);
-  };
-  if (dtype == TFF_F64) {
-    hipLaunchKernelGGL(k_cp_nonbonded<double>, dim3(gt), dim3(CPB), 0, stream, (const double*)coords, g, en,
-                       (const double*)charges, (const double*)sigma, (const double*)epsilon, coul_constant, do_shift,
-                       w.e_part, gx, gq, gs, ge);
-    finish(double{});
-  } else {
-    hipLaunchKernelGGL(k_cp_nonbonded<float>, dim3(gt), dim3(CPB), 0, stream, (const float*)coords, g, en,
-                       (const float*)charges, (const float*)sigma, (const float*)epsilon, coul_constant, do_shift,
-                       w.e_part, gx, gq, gs, ge);
-    finish(float{});
+  if (grad) hipLaunchKernelGGL(k_cp_zero_d, blocks(stride * natoms), dim3(256), 0, stream, w.acc, stride * natoms);
+  // runs of up to 16 entries, shorter ones while there are fewer than 8192 half-waves of them
+  int run = (int)(total / 8192);
+  run = run < 1 ? 1 : run > 16 ? 16 : run;
+  const unsigned gt = grid_for(1, (total + run - 1) / run);
+  // float r^2 against the exact one: each component is off by at most 8 2^-24 (|d| + box) times the
+  // condition of the change to fractional coordinates; where the cutoff is half the box, two images
+  // are equally far and only the exact test is taken
+  double box_l = 0, cond = 1;
+  for (int a = 0; a < 3; ++a) {
+    double s = 0;
+    for (int b = 0; b < 3; ++b) {
+      s += fabs(g.box.b[3 * a + b]);
+      double c = 0;
+      for (int k = 0; k < 3; ++k) c += fabs(g.box.inv[3 * a + k]) * (fabs(g.box.b[3 * k]) + fabs(g.box.b[3 * k + 1]) + fabs(g.box.b[3 * k + 2]));
+      if (c > cond) cond = c;
+    }
+    if (s > box_l) box_l = s;
   }
-  TFF_CHECK_LAUNCH("cluster pairs nonbonded");
+  const double tol_k = g.rc > 0.998 * g.half_h ? INFINITY : 64.0 / 16777216.0 * g.rc * cond;
+  auto go = [&](auto tag) {
+    using TT = decltype(tag);
+    const TT *c = (const TT*)coords, *q = (const TT*)charges, *sg = (const TT*)sigma, *ep = (const TT*)epsilon;
+    auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(gt), dim3(CPB), 0, stream, c, g, en, run, q, sg, ep, coul_constant, do_shift,
+                         (TT)tol_k, (TT)box_l, w.e_part, w.acc);
+    };
+    if (grad == 2)
+      launch(k_cp_nonbonded<TT, 2>);
+    else if (grad == 1)
+      launch(k_cp_nonbonded<TT, 1>);
+    else
+      launch(k_cp_nonbonded<TT, 0>);
+    const CpOut<TT> o{(TT*)energy_out, (TT*)grad_coords, (TT*)grad_charges, (TT*)grad_sigma, (TT*)grad_epsilon,
+                      (TT*)forces_accum};
+    hipLaunchKernelGGL(k_cp_finish<TT>, blocks(grad ? natoms : 1), dim3(256), 0, stream, (const double*)w.e_part,
+                       (int)gt, (const double*)w.acc, stride, grad ? natoms : 0LL, scale, o);
+  };
+  if (dtype == TFF_F64)
+    go(double{});
+  else
+    go(float{});
+  TFF_CHECK_LAUNCH("nonbonded from cluster pairs");
   return TFF_OK;
 }
