@@ -45,6 +45,8 @@ _SIGNATURES = {
                                       _vp, _vp, _vp, _sz, _vp]),
     "tff_pme_gather_multipole": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _ll, _vp, _i, _i, _i, _i, _d, _d, _vp, _vp, _vp,
                                       _vp, _vp]),
+    "tff_exclusions_csr_workspace_bytes": (_sz, [_ll]),
+    "tff_exclusions_csr": (_i, [_vp, _ll, _i, _ll, _vp, _vp, _vp, _vp, _sz, _vp]),
     "tff_cluster_pairs_workspace_bytes": (_sz, [_ll, _vp, _d, _d]),
     "tff_cluster_pairs_build": (_i, [_i, _vp, _ll, _vp, _d, _d, _vp, _vp, _vp, _vp, _sz, _vp]),
     "tff_cluster_pairs_emit": (_i, [_i, _vp, _ll, _vp, _d, _d, _vp, _vp, _vp, _vp, _vp, _ll, _vp, _vp, _ll, _vp, _sz,

@@ -53,13 +53,26 @@ _def.define("compute_nonbonded_forces_from_cluster_pairs(Tensor coords, Tensor b
             "Tensor interacting_atoms, Tensor(a!) forces) -> ()")
 
 
-def _exclusions_csr(exclusions, n, device):
-    """Symmetric int64 CSR of a (2, E) (or (E, 2)) COO exclusion list, as NeighborList builds it."""
+def _exclusions_csr(exclusions, n, device, status=None):
+    """Symmetric int64 CSR of a (2, E) (or (E, 2)) COO exclusion list, as NeighborList builds it (on the GPU a row's
+    partners are unordered and padded with -1; an index past the atoms sets `status`)."""
     if exclusions is None or exclusions.numel() == 0:
         return None, None
     e = exclusions.detach().to(torch.int64)
     if e.ndim != 2 or 2 not in e.shape:
         raise ValueError(f"build_cluster_pairs: exclusions must be (2, E) or (E, 2), got {tuple(e.shape)}")
+    if e.is_cuda:
+        lib = L.load()
+        e = e.contiguous()
+        two_rows = e.shape[0] == 2
+        E = e.shape[1] if two_rows else e.shape[0]
+        row_ptr = torch.empty(n + 1, dtype=torch.long, device=device)
+        col = torch.empty(2 * E, dtype=torch.long, device=device)
+        ws = L.workspace(lib.tff_exclusions_csr_workspace_bytes(n), device)
+        rc = lib.tff_exclusions_csr(L.ptr(e), E, int(two_rows), n, L.ptr(row_ptr), L.ptr(col), L.ptr(status),
+                                    L.ptr(ws), ws.numel(), L.stream_of(e))
+        L.check(rc, "build_cluster_pairs")
+        return row_ptr, col
     pairs = e.t() if e.shape[0] == 2 else e
     pairs = pairs[(pairs[:, 0] >= 0) & (pairs[:, 1] >= 0)]
     allp = torch.cat([pairs, pairs.flip(1)], dim=0)
@@ -81,17 +94,19 @@ def _build_cluster_pairs(coords, box, cutoff, exclusions, cell_size, max_num_int
     c = coords.detach().contiguous()
     n = c.shape[0]
     bh = L.box_host(box)
-    rp, col = _exclusions_csr(exclusions, n, c.device)
+    counts = torch.zeros(4, dtype=torch.int64, device=c.device)
+    rp, col = _exclusions_csr(exclusions, n, c.device, counts[3:])
     nbytes = lib.tff_cluster_pairs_workspace_bytes(n, bh, float(cutoff), float(cell_size))
     if nbytes == 0:
         L.check(lib.tff_cluster_pairs_build(L.dtype_code(c), L.ptr(c), n, bh, float(cutoff), float(cell_size), None,
                                             None, None, None, 0, L.stream_of(c)), "build_cluster_pairs")
     ws = L.workspace(nbytes, c.device)
-    counts = torch.zeros(3, dtype=torch.int64, device=c.device)
     rc = lib.tff_cluster_pairs_build(L.dtype_code(c), L.ptr(c), n, bh, float(cutoff), float(cell_size), L.ptr(rp),
                                      L.ptr(col), L.ptr(counts), L.ptr(ws), ws.numel(), L.stream_of(c))
     L.check(rc, "build_cluster_pairs")
-    E, M, flags = (int(v) for v in counts.cpu())
+    E, M, flags, outside = counts.tolist()
+    if outside:
+        raise RuntimeError("build_cluster_pairs: an exclusion index is past the atoms")
     if flags & 1:
         raise RuntimeError("build_cluster_pairs: an atom has more than 16 exclusion partners")
     if flags & 2:
