@@ -34,6 +34,7 @@
 // shuffles.  Pairs come out in entry, lane, column order at offsets from a count pass and a scan.
 
 #include <cmath>
+#include <type_traits>
 
 #include "pair_math.h"
 #include "tff_common.h"
@@ -703,12 +704,15 @@ __device__ __forceinline__ void cp_flush(int a, const double (&v)[CpCh<LJG>::N],
 // each, which then go round the row by DPP together with their sums (T, at most 32 terms, as the
 // sums of a column by butterfly would be), 16 steps, twice: no shuffle and no reduction per column.
 // The pair predicate is that of the decoded list, in float64: T = float decides by its own r^2
-// unless that is within its error bound `tol_k` (|d| + box) of rc^2.
+// unless that is within its error bound `tol_k` (|x_i| + |x_j| + box) of rc^2.
 // Bound by the arithmetic of the candidate pairs (of 32 x 32 per entry about one in five is within the
-// cutoff).  96k water atoms, float, all gradients: 315 us; one column per step by shuffles, a
-// butterfly per gradient and an atomic per atom and channel took 683.
-template <typename T, int GRAD>
-__global__ __launch_bounds__(CPB) void k_cp_nonbonded(const T* __restrict__ coords, CpGeom g, Entries en, int run,
+// cutoff; some 150 instructions a step).  96k water atoms, float, all gradients: 275 us (energy alone
+// 150); one column per step by shuffles, a butterfly per gradient and an atomic per atom and channel
+// took 683.  Testing all pairs first and working off each lane's hits, with the column sums in LDS, took
+// 828: the fullest lane of 64 has nearly all 32 columns.
+// BOX: 0 no box, 1 orthorhombic, 2 general.
+template <typename T, int GRAD, int BOX>
+__global__ __launch_bounds__(CPB) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 3))) void k_cp_nonbonded(const T* __restrict__ coords, CpGeom g, Entries en, int run,
                                                       const T* __restrict__ q, const T* __restrict__ sig,
                                                       const T* __restrict__ eps, double coul, int do_shift, T tol_k,
                                                       T tol_l, double* __restrict__ e_part,
@@ -720,6 +724,8 @@ __global__ __launch_bounds__(CPB) void k_cp_nonbonded(const T* __restrict__ coor
   const int l = half_lane(), l16 = l & 15;
   const long long total = en.E + en.M;
   const T shift = do_shift ? (T)(1.0 / g.rc) : (T)0, kc = (T)coul, rc2 = (T)g.rc2;
+  const T b0 = (T)g.box.b[0], b1 = (T)g.box.b[4], b2 = (T)g.box.b[8];
+  const T v0 = (T)g.box.inv[0], v1 = (T)g.box.inv[4], v2 = (T)g.box.inv[8];
   double e_acc = 0.0;
   const long long runs = (total + run - 1) / run;
   for (long long r0 = half_index() & ~1; r0 < runs; r0 += half_count()) {  // both halves of a wave together
@@ -741,70 +747,84 @@ __global__ __launch_bounds__(CPB) void k_cp_nonbonded(const T* __restrict__ coor
       }
       if (x != x_of) {
         if constexpr (GRAD != 0) {
-          if (x_of >= 0) cp_flush<LJG>(i, fi, s, acc);
+          if (x_of >= 0) {
+            fi[3] *= coul;
+            cp_flush<LJG>(i, fi, s, acc);
+          }
           for (int k = 0; k < N; ++k) fi[k] = 0.0;
         }
         x_of = x;
         i = in;
         if (i >= 0) {
           xi = coords[3 * i]; yi = coords[3 * i + 1]; zi = coords[3 * i + 2];
-          qi = q[i]; si = sig[i]; ei = eps[i];
+          qi = q[i]; si = (T)0.5 * sig[i]; ei = eps[i];
         }
       }
       T xj = 0, yj = 0, zj = 0, qj = 0, sj = 0, ej = 0;
       if (j >= 0) {
         xj = coords[3 * j]; yj = coords[3 * j + 1]; zj = coords[3 * j + 2];
-        qj = q[j]; sj = sig[j]; ej = eps[j];
+        qj = q[j]; sj = (T)0.5 * sig[j]; ej = eps[j];
       }
       skip |= half_ballot(j < 0);
       if (i < 0) skip = 0xffffffffu;
+      // r^2 (T) below r2_in is within the cutoff, above r2_out it is not
+      T r2_in = rc2, r2_out = rc2;
+      if constexpr (sizeof(T) == 4) {
+        T m = fabs(xj) + fabs(yj) + fabs(zj);
+        for (int o = 16; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 32));  // (a NaN fails its own tests)
+        const T tol = tol_k * (fabs(xi) + fabs(yi) + fabs(zi) + m + tol_l);
+        r2_in = rc2 - tol;
+        r2_out = rc2 + tol;
+      }
       T gj[N];
       for (int k = 0; k < N; ++k) gj[k] = 0;
       for (int h = 0; h < 2; ++h) {
-        // bit 16 - k of `todo`: the pair of step k (column (l16 - k) & 15 of the row's block)
+        // bit 31 - k of `todo`: the pair of step k (column (l16 - k) & 15 of the row's block)
         const unsigned m16 = ((l >> 4) ^ h ? skip >> 16 : skip) & 0xffffu;
-        unsigned todo = ~((m16 | m16 << 16) >> l16);
+        int todo = (int)(~((m16 | m16 << 16) >> l16) << 15);
         for (int c = 0; c < 16; ++c) {
           T dx = xi - xj, dy = yi - yj, dz = zi - zj;
-          const T raw = fabs(dx) + fabs(dy) + fabs(dz);
-          tff_min_image<T>(g.box, dx, dy, dz);
+          if constexpr (BOX == 1) {  // tff_min_image, its branches taken
+            dx *= v0; dy *= v1; dz *= v2;
+            dx = (dx - rint(dx)) * b0; dy = (dy - rint(dy)) * b1; dz = (dz - rint(dz)) * b2;
+          } else if constexpr (BOX == 2) {
+            tff_min_image<T>(g.box, dx, dy, dz);
+          }
           T r2 = dx * dx + dy * dy + dz * dz;
-          bool ok = (todo & 0x10000u) != 0;
+          bool ok = todo < 0;
           if constexpr (sizeof(T) == 8) {
             double ax = (double)xi - (double)xj, ay = (double)yi - (double)yj, az = (double)zi - (double)zj;
             tff_min_image_d(g.box, ax, ay, az);
             ok = ok && ax * ax + ay * ay + az * az <= g.rc2;
           } else {
-            const T gap = r2 - rc2, tol = tol_k * (raw + tol_l);
-            if (ok && !(gap < -tol || gap > tol)) {
+            if (ok && !(r2 < r2_in || r2 > r2_out)) {
               double ax = (double)xi - (double)xj, ay = (double)yi - (double)yj, az = (double)zi - (double)zj;
               tff_min_image_d(g.box, ax, ay, az);
               ok = ax * ax + ay * ay + az * az <= g.rc2;
             } else {
-              ok = ok && gap < 0;
+              ok = ok && r2 < r2_in;
             }
           }
           if (ok) {
             const T rinv = cp_rsqrt(r2), rinv2 = rinv * rinv;
-            const T qq = qi * qj * kc;
-            T en_ = qq * (rinv - shift);
+            const T qq = qi * qj * kc, ph = rinv - shift;
+            T en_ = qq * ph;
             T dr = -qq * rinv * rinv2;
-            const T sij = (si + sj) * (T)0.5, eij = cp_sqrt(ei * ej);
+            const T sij = si + sj, eij = cp_sqrt(ei * ej);
             const T sr2 = sij * sij * rinv2, s6 = sr2 * sr2 * sr2;
             en_ += (T)4 * eij * s6 * (s6 - (T)1);
             const T w = (T)24 * eij * s6 * ((T)2 * s6 - (T)1);
             dr -= w * rinv2;
             e_acc += (double)en_;
             if constexpr (GRAD != 0) {
-              const T gq = (rinv - shift) * kc;
               fi[0] += (double)(dr * dx);
               fi[1] += (double)(dr * dy);
               fi[2] += (double)(dr * dz);
-              fi[3] += (double)(qj * gq);
+              fi[3] += (double)(qj * ph);  // times k at the end
               gj[0] -= dr * dx;
               gj[1] -= dr * dy;
               gj[2] -= dr * dz;
-              gj[3] += qi * gq;
+              gj[3] += qi * ph;
             }
             if constexpr (LJG) {
               const T ds = cp_div(w, sij) * (T)0.5;
@@ -837,12 +857,15 @@ __global__ __launch_bounds__(CPB) void k_cp_nonbonded(const T* __restrict__ coor
       }
       if constexpr (GRAD != 0) {
         double gd[N];
-        for (int k = 0; k < N; ++k) gd[k] = (double)gj[k];
+        for (int k = 0; k < N; ++k) gd[k] = k == 3 ? (double)gj[k] * coul : (double)gj[k];
         cp_flush<LJG>(j, gd, s, acc);
       }
     }
     if constexpr (GRAD != 0)
-      if (x_of >= 0) cp_flush<LJG>(i, fi, s, acc);
+      if (x_of >= 0) {
+        fi[3] *= coul;
+        cp_flush<LJG>(i, fi, s, acc);
+      }
   }
   const double sum = tff_block_sum(e_acc);
   if (threadIdx.x == 0) e_part[blockIdx.x] = sum;
@@ -1286,12 +1309,21 @@ extern "C" int tff_cluster_pairs_nonbonded(int dtype, const void* coords, long l
       hipLaunchKernelGGL(kern, dim3(gt), dim3(CPB), 0, stream, c, g, en, run, q, sg, ep, coul_constant, do_shift,
                          (TT)tol_k, (TT)box_l, w.e_part, w.acc);
     };
-    if (grad == 2)
-      launch(k_cp_nonbonded<TT, 2>);
-    else if (grad == 1)
-      launch(k_cp_nonbonded<TT, 1>);
+    auto pick = [&](auto box) {
+      constexpr int B = decltype(box)::value;
+      if (grad == 2)
+        launch(k_cp_nonbonded<TT, 2, B>);
+      else if (grad == 1)
+        launch(k_cp_nonbonded<TT, 1, B>);
+      else
+        launch(k_cp_nonbonded<TT, 0, B>);
+    };
+    if (!g.box.periodic)
+      pick(std::integral_constant<int, 0>{});
+    else if (g.box.ortho)
+      pick(std::integral_constant<int, 1>{});
     else
-      launch(k_cp_nonbonded<TT, 0>);
+      pick(std::integral_constant<int, 2>{});
     const CpOut<TT> o{(TT*)energy_out, (TT*)grad_coords, (TT*)grad_charges, (TT*)grad_sigma, (TT*)grad_epsilon,
                       (TT*)forces_accum};
     hipLaunchKernelGGL(k_cp_finish<TT>, blocks(grad ? natoms : 1), dim3(256), 0, stream, (const double*)w.e_part,
