@@ -1655,14 +1655,25 @@ __global__ __launch_bounds__(FB) void k_slot_splines(const int* __restrict__ ncl
 // brick in LDS with int64 fixed-point atomics.  Integer sums do not depend on the order, so the grid
 // equals k_spread_bricks' bit for bit; the brick is stored once, so the grid needs neither clearing
 // nor global atomics.
+// DIPOLE: the dipoles q_i v_i . grad_r theta_i(m) of the force-matching backward instead of the charges
+// (per-slot vectors vsl, Cartesian-to-grid scale jsc = K / L), from the lists that the charge spread
+// left.  A point gets (X1 Y1 + X2 Y2) Z1 + X2 Y1 Z2 with X1 = w_x M'_x, X2 = M_x, Y1 = M_y, Y2 = w_y M'_y,
+// Z1 = M_z, Z2 = w_z M'_z; weights and derivatives are evaluated again per brick that a stencil meets
+// (some 4 times; a table of both would be read as often).  Charges: wts holds the weights.
+// 96k water atoms, order 5, 96^3: the dipoles 44 us; k_spread_bricks (a search over clusters per brick, one lane
+// per slot, a general double-to-int64 conversion per point) took 251 beside the pair kernel.
 constexpr int LIST_ROUND = 256;
-template <int P>
+template <int P, bool DIPOLE>
 __global__ __launch_bounds__(LIST_ROUND) void k_spread_lists(const float* __restrict__ wts,
                                                              const int* __restrict__ bcount,
                                                              const int2* __restrict__ blist, BrickGrid bg,
-                                                             PmeGeom pg, unsigned long long* __restrict__ grid) {
+                                                             PmeGeom pg, unsigned long long* __restrict__ grid,
+                                                             const V4<float>* __restrict__ xyzq,
+                                                             const V4<float>* __restrict__ vsl, V4<float> jsc) {
   constexpr int NT = LIST_ROUND;
-  constexpr int REC = spline_stride<P>();  // per compacted slot: the weights of its runs, then the runs
+  constexpr int NW = DIPOLE ? 6 * P : 3 * P;  // weights per compacted slot: of its runs, then the runs
+  constexpr int REC = (NW + 1 + 3) & ~3;
+  constexpr int NC = DIPOLE ? 1 : 2;          // candidates per thread and pass
   __shared__ unsigned long long s_q[SQ_Z * BR];
   __shared__ __align__(16) float s_w[NT][REC];
   __shared__ int s_hoff[28], s_hid[27], s_cnt[27];
@@ -1727,15 +1738,15 @@ __global__ __launch_bounds__(LIST_ROUND) void k_spread_lists(const float* __rest
     __syncthreads();
   }
   const int nh = s_nh, total = s_hoff[nh];
-  // candidates in passes of 2 NT: each thread loads and tests its two (k and k + NT) and loads the
+  // candidates in passes of NC NT: each thread loads and tests its two (k and k + NT) and loads the
   // spline tables of those that hit before the first is spread, so the global loads of both rounds
   // overlap
-  for (int p0 = 0; p0 < total; p0 += 2 * NT) {
-    float rec2[2][REC];
-    bool hit2[2] = {false, false};
-    int2 e2[2];
+  for (int p0 = 0; p0 < total; p0 += NC * NT) {
+    float rec2[NC][REC];
+    bool hit2[NC] = {};
+    int2 e2[NC];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < NC; ++c) {
       const int k = p0 + c * NT + threadIdx.x;
       e2[c] = make_int2(0, 0);
       if (k < total) {
@@ -1745,13 +1756,14 @@ __global__ __launch_bounds__(LIST_ROUND) void k_spread_lists(const float* __rest
       }
     }
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < NC; ++c) {
       const int k = p0 + c * NT + threadIdx.x;
       if (k >= total) continue;
       const int2 e = e2[c];
       const int bs[3] = {e.y & 1023, (e.y >> 10) & 1023, (e.y >> 20) & 1023};
       bool hit = true;
       int q0[3], l0[3], nr[3];
+      bool small = true;
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
         // the stencil [bs, bs + P) and the brick [B0, B0 + Bn) as arcs of Z_K: one common run
@@ -1772,28 +1784,58 @@ __global__ __launch_bounds__(LIST_ROUND) void k_spread_lists(const float* __rest
       }
       if (!hit) continue;
       hit2[c] = true;
-      const float* src = wts + (size_t)e.x * LIST_WST;
-      float tb[3 * P + 1];
+      if constexpr (DIPOLE) {
+        const V4<float> p = xyzq[e.x], vv = vsl[e.x];
+        const double rr[3] = {(double)p.x, (double)p.y, (double)p.z};
+        // d theta / d r_a = -K_a / L_a M'_a ... (the weights fall as the scaled coordinate grows)
+        const float wv[3] = {-p.w * vv.x * jsc.x, -p.w * vv.y * jsc.y, -p.w * vv.z * jsc.z};
+        // contributions below 2^10 (weights and derivatives are at most 1) convert by mantissa
+        small = fabsf(wv[0]) + fabsf(wv[1]) + fabsf(wv[2]) < 1024.0f;
 #pragma unroll
-      for (int i = 0; i <= 3 * P; ++i) tb[i] = src[i];
+        for (int a = 0; a < 3; ++a) {
+          const double sa = (rr[0] * pg.inv[a] + rr[1] * pg.inv[3 + a] + rr[2] * pg.inv[6 + a]) * (double)pg.K[a];
+          int base;
+          double t;
+          float Mv[P], dM[P];
+          anchor_axis(sa, pg.K[a], P, base, t);
+          spline_weights<float, P>((float)t, Mv, dM);
 #pragma unroll
-      for (int a = 0; a < 3; ++a)
+          for (int i = 0; i < P; ++i) {
+            float m = 0.f, d = 0.f;
 #pragma unroll
-        for (int i = 0; i < P; ++i) {
-          float v = 0.f;
-#pragma unroll
-          for (int kk = 0; kk < P; ++kk)
-            if (i < nr[a] && q0[a] + i == kk) v = tb[a * P + kk];
-          // z weights carry the fixed-point scale (a power of two: (a b) 2^28 = a (b 2^28) exactly)
-          rec2[c][a * P + i] = a == 0 ? tb[3 * P] * v : (a == 2 ? v * (float)QF_SCALE : v);
+            for (int kk = 0; kk < P; ++kk)
+              if (i < nr[a] && q0[a] + i == kk) {
+                m = Mv[kk];
+                d = wv[a] * dM[kk];
+              }
+            rec2[c][2 * a * P + i] = m;
+            rec2[c][(2 * a + 1) * P + i] = d;
+          }
         }
-      rec2[c][3 * P] = __int_as_float(l0[0] | (l0[1] << 3) | (l0[2] << 6) | (nr[0] << 9) | (nr[1] << 13) |
-                                      (nr[2] << 17));
+      } else {
+        const float* src = wts + (size_t)e.x * LIST_WST;
+        float tb[3 * P + 1];
 #pragma unroll
-      for (int i = 3 * P + 1; i < REC; ++i) rec2[c][i] = 0.f;
+        for (int i = 0; i <= 3 * P; ++i) tb[i] = src[i];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+          for (int i = 0; i < P; ++i) {
+            float v = 0.f;
+#pragma unroll
+            for (int kk = 0; kk < P; ++kk)
+              if (i < nr[a] && q0[a] + i == kk) v = tb[a * P + kk];
+            // z weights carry the fixed-point scale (a power of two: (a b) 2^28 = a (b 2^28) exactly)
+            rec2[c][a * P + i] = a == 0 ? tb[3 * P] * v : (a == 2 ? v * (float)QF_SCALE : v);
+          }
+      }
+      rec2[c][NW] = __int_as_float(l0[0] | (l0[1] << 3) | (l0[2] << 6) | (nr[0] << 9) | (nr[1] << 13) |
+                                   (nr[2] << 17) | (small ? 1 << 21 : 0));
+#pragma unroll
+      for (int i = NW + 1; i < REC; ++i) rec2[c][i] = 0.f;
     }
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < NC; ++c) {
       if (p0 + c * NT >= total) break;
       if (threadIdx.x == 0) s_na = 0;
       __syncthreads();
@@ -1811,9 +1853,39 @@ __global__ __launch_bounds__(LIST_ROUND) void k_spread_lists(const float* __rest
       for (int k = threadIdx.x; k < nlanes; k += NT) {
         const int t = k / P, ix = k - t * P;
         const float* w = s_w[t];
-        const int meta = __float_as_int(w[3 * P]);
+        const int meta = __float_as_int(w[NW]);
         const int nx = (meta >> 9) & 15, ny = (meta >> 13) & 15, nz = (meta >> 17) & 15;
         if (ix >= nx) continue;
+        const int lx = (meta & 7) + ix, ly0 = (meta >> 3) & 7, lz0 = (meta >> 6) & 7;
+        if constexpr (DIPOLE) {
+          const float x2 = w[ix], x1 = w[P + ix];
+          float z1[P], z2[P];
+#pragma unroll
+          for (int i = 0; i < P; ++i) {
+            z1[i] = w[4 * P + i];
+            z2[i] = w[5 * P + i];
+          }
+          const bool by_mantissa = (meta >> 21) & 1;
+#pragma unroll
+          for (int iy = 0; iy < P; ++iy) {
+            if (iy >= ny) break;
+            const float y1 = w[2 * P + iy], y2 = w[3 * P + iy];
+            const float cxy = fmaf(x1, y1, x2 * y2), dxy = x2 * y1;
+            unsigned long long* row = s_q + lz0 * SQ_Z + (ly0 + iy) * SQ_Y + lx;
+#pragma unroll
+            for (int iz = 0; iz < P; ++iz) {
+              const double v = (double)fmaf(cxy, z1[iz], dxy * z2[iz]);
+              unsigned long long b;
+              if (__builtin_expect(by_mantissa, 1))
+                b = (unsigned long long)(__double_as_longlong(fma(v, Q_SCALE, 6755399441055744.0)) -
+                                         0x4338000000000000LL);
+              else
+                b = (unsigned long long)to_fx(v, Q_SCALE);
+              if (iz < nz) atomicAdd(&row[iz * SQ_Z], b);
+            }
+          }
+          continue;
+        }
         const float wx = w[ix];
         float wy[P], wz[P];
 #pragma unroll
@@ -1821,7 +1893,6 @@ __global__ __launch_bounds__(LIST_ROUND) void k_spread_lists(const float* __rest
           wy[i] = w[P + i];
           wz[i] = w[2 * P + i];
         }
-        const int lx = (meta & 7) + ix, ly0 = (meta >> 3) & 7, lz0 = (meta >> 6) & 7;
 #pragma unroll
         for (int iy = 0; iy < P; ++iy) {
           if (iy >= ny) break;
@@ -2250,9 +2321,10 @@ int launch_pme_slots(int order, const FusedWs& w, const Geo& g, const PmeGeom& p
   if (spread && sizeof(TC) == 4 && spread_from_lists(P, pg.K)) {                                                \
     hipLaunchKernelGGL((k_slot_splines<P < 7 ? P : 6>), dim3(nb), dim3(FB), 0, st, w.ncl,                      \
                        (const V4<float>*)w.xyzq, w.slot_orig, pg, w.bg, w.wts, w.bcount, w.blist, status);      \
-    hipLaunchKernelGGL((k_spread_lists<P < 7 ? P : 6>), dim3(nbricks), dim3(LIST_ROUND), 0, st,              \
+    hipLaunchKernelGGL((k_spread_lists<P < 7 ? P : 6, false>), dim3(nbricks), dim3(LIST_ROUND), 0, st,       \
                        (const float*)w.wts,                                                                      \
-                       (const int*)w.bcount, (const int2*)w.blist, w.bg, pg, w.grid);                         \
+                       (const int*)w.bcount, (const int2*)w.blist, w.bg, pg, w.grid,                          \
+                       (const V4<float>*)nullptr, (const V4<float>*)nullptr, V4<float>{});                    \
   } else if (spread)                                                                                            \
     hipLaunchKernelGGL((k_spread_bricks<TC, P, false>), dim3(nbricks), dim3(256), 0, st, w.ncl,               \
                        (const V4<TC>*)w.xyzq, w.slot_orig, w.bb_c, w.bb_h, w.col_cl_start, g, pg, w.grid, status, \
@@ -2616,16 +2688,30 @@ int run_fused_grad(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
   TC* phi = (TC*)w.grid;
   TC* psi = (TC*)w.grid_d;
   const unsigned nb = (unsigned)((nslots + FB - 1) / FB);
-#define TFF_GRAD_PME(P)                                                                                          \
-  {                                                                                                              \
-    hipLaunchKernelGGL((k_spread_bricks<TC, P, true>), dim3(nbricks), dim3(256), 0, sp, w.ncl,                   \
-                       (const V4<TC>*)w.xyzq, w.slot_orig, w.bb_c, w.bb_h, w.col_cl_start, g, pg, w.grid_d,       \
-                       status, (const V4<TC>*)w.vsl, jsc);                                                       \
-    run_recip_fft<TC>(w, K, box, alpha, pl, mx, my, mz, w.grid_d, 1.0 / Q_SCALE, psi, w.kparts,                 \
-                      "fused_grad_fft", sp);                                                                     \
-    hipLaunchKernelGGL((k_gather_grad<TC, P>), dim3(nb), dim3(FB), 0, sp, w.ncl, phi, psi, (const V4<TC>*)w.xyzq, \
-                       (const V4<TC>*)w.vsl, w.slot_orig, pg, coul, gE, w.gpme);                                 \
-  }
+  auto spread_dipoles = [&] {
+    auto go = [&](auto order_c) {
+      constexpr int P = decltype(order_c)::value;
+      if constexpr (sizeof(TC) == 4 && P < 7) {
+        if (spread_from_lists(P, K)) {
+          hipLaunchKernelGGL((k_spread_lists<P, true>), dim3(nbricks), dim3(LIST_ROUND), 0, sp, (const float*)w.wts,
+                             (const int*)w.bcount, (const int2*)w.blist, w.bg, pg, w.grid_d,
+                             (const V4<float>*)w.xyzq, (const V4<float>*)w.vsl, jsc);
+          return;
+        }
+      }
+      hipLaunchKernelGGL((k_spread_bricks<TC, P, true>), dim3(nbricks), dim3(256), 0, sp, w.ncl,
+                         (const V4<TC>*)w.xyzq, w.slot_orig, w.bb_c, w.bb_h, w.col_cl_start, g, pg, w.grid_d, status,
+                         (const V4<TC>*)w.vsl, jsc);
+    };
+    switch (order) {
+      case 3: go(std::integral_constant<int, 3>{}); break;
+      case 4: go(std::integral_constant<int, 4>{}); break;
+      case 5: go(std::integral_constant<int, 5>{}); break;
+      case 6: go(std::integral_constant<int, 6>{}); break;
+      case 7: go(std::integral_constant<int, 7>{}); break;
+      default: go(std::integral_constant<int, 8>{}); break;
+    }
+  };
   // the potential grid phi of the charges: the forward call's, left in place (reuse), or made
   // again by the forward's own spread and transforms, so that both give the same bits
   if (!reuse) {
@@ -2637,15 +2723,20 @@ int run_fused_grad(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
     run_recip_fft<TC>(w, K, box, alpha, pl, mx, my, mz, w.grid, 1.0 / grid_scale<TC>(), phi, w.kparts,
                       "fused_grad_fft", sp);
   }
+  spread_dipoles();
+  run_recip_fft<TC>(w, K, box, alpha, pl, mx, my, mz, w.grid_d, 1.0 / Q_SCALE, psi, w.kparts, "fused_grad_fft", sp);
+#define TFF_GRAD_GATHER(P)                                                                                       \
+  hipLaunchKernelGGL((k_gather_grad<TC, P>), dim3(nb), dim3(FB), 0, sp, w.ncl, phi, psi, (const V4<TC>*)w.xyzq, \
+                     (const V4<TC>*)w.vsl, w.slot_orig, pg, coul, gE, w.gpme)
   switch (order) {
-    case 3: TFF_GRAD_PME(3); break;
-    case 4: TFF_GRAD_PME(4); break;
-    case 5: TFF_GRAD_PME(5); break;
-    case 6: TFF_GRAD_PME(6); break;
-    case 7: TFF_GRAD_PME(7); break;
-    default: TFF_GRAD_PME(8); break;
+    case 3: TFF_GRAD_GATHER(3); break;
+    case 4: TFF_GRAD_GATHER(4); break;
+    case 5: TFF_GRAD_GATHER(5); break;
+    case 6: TFF_GRAD_GATHER(6); break;
+    case 7: TFF_GRAD_GATHER(7); break;
+    default: TFF_GRAD_GATHER(8); break;
   }
-#undef TFF_GRAD_PME
+#undef TFF_GRAD_GATHER
   aux_stream_join(st, sp);
   hipLaunchKernelGGL(k_finalize_grad<TI>, dim3(nbS), dim3(FB), 0, st, w.ncl, w.slot_orig, w.gacc, w.gpme, q, coul,
                      alpha, gE, dr, dq, dsig, deps, w.es, status, status_host);
