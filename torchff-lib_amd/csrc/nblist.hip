@@ -211,35 +211,42 @@ __global__ void k_scatter(const double4* __restrict__ xyz, long long n, TffBox b
   }
 }
 
-// One workgroup of CP_WAVES waves per home cell.  The home cell's atoms (in chunks of 64) and their
-// exclusion partners (up to CP_EX each; more are looked up in the CSR arrays) are staged in LDS
-// once; each wave takes every CP_WAVES-th cell of the half shell (the cells' starts and sizes loaded
-// at once, one lane per cell), stages that cell's atoms (first 64 prefetched into registers while
-// the previous cell is walked) in its own LDS area and walks the ni x nj candidate block 64 at a
-// time, the lane's (a, b) advanced incrementally (one division per cell).  WRITE = false: each
-// wave's accepted-pair count into wcount[home * CP_WAVES + wave]; WRITE = true: the pairs from
-// woff[home * CP_WAVES + wave] on, in ballot order (rows at or past max_npairs are not stored).
+// One workgroup of CP_WAVES waves per home cell.  The home cell's atoms (in chunks of 64) with their
+// exclusion partners (up to CP_EX each; more are looked up in the CSR arrays) and the atoms of the half
+// shell (home cell first, in batches of CP_JB, with their cell pair's periodic shift) are staged in
+// LDS.  Each wave takes every CP_WAVES-th 64 of the batch, one atom per lane in registers, and walks the
+// home atoms, which all lanes read at one LDS address.  WRITE = false: each wave's accepted-pair count
+// into wcount[home * CP_WAVES + wave]; WRITE = true: the pairs from woff[home * CP_WAVES + wave] on, in
+// ballot order (rows at or past max_npairs are not stored).
+// Bound by the instructions per 64 candidates (some 25; the write pass also by its 16 bytes per pair).  96k
+// water atoms, 1 nm: 150 and 176 us for the two passes; with each lane taking its own pair of a cell pair's
+// ni x nj block (three 16-byte LDS reads per candidate, four passes per cell pair of 14 x 14 with a
+// quarter of the lanes idle, a staging step per cell) 238 + 262.
 constexpr int CP_WAVES = 4;
-constexpr int CP_HOME = 64;  // home atoms per chunk
-constexpr int CP_EX = 4;     // exclusion partners per home atom kept in LDS
+constexpr int CP_HOME = 64;   // home atoms per chunk
+constexpr int CP_EX = 4;      // exclusion partners per home atom kept in LDS
+constexpr int CP_JB = 1024;   // half-shell atoms per batch
 
-template <bool WRITE>
+// PF: the float32 prefilter (g.pf)
+template <bool WRITE, bool PF>
 __global__ __launch_bounds__(CP_WAVES * TFF_WAVE) void k_cell_pairs(
     const int* __restrict__ start, const int* __restrict__ sorted_idx, const double4* __restrict__ sxyz,
     const float4* __restrict__ sf, CellGrid g, TffBox box, double cutoff2, int include_self,
     const int64_t* __restrict__ row_ptr, const int64_t* __restrict__ col, int* __restrict__ wcount,
     const int* __restrict__ woff, long long* __restrict__ pairs, long long max_npairs, int* __restrict__ npairs) {
-  // staged atoms: x, y, z and the atom index (exact in a double) in w
+  // home atoms: x, y, z and the atom index (exact in a double) in w; the prefilter's copies (wrapped float32
+  // coordinates, atom index bits in w)
   __shared__ double4 s_h[CP_HOME];
+  __shared__ float4 s_hf[CP_HOME];
   // the home atoms' exclusion partners, -1 padded; all -2: more than CP_EX (CSR lookup)
   __shared__ int4 s_hx[CP_HOME];
-  __shared__ double4 s_n[CP_WAVES][TFF_WAVE];
-  // prefilter copies (wrapped float32 coordinates, atom index bits in w); the neighbour copies carry
-  // their cell pair's periodic shift
-  __shared__ float4 s_hf[CP_HOME];
-  __shared__ float4 s_nf[CP_WAVES][TFF_WAVE];
+  // half-shell atoms: prefilter copy (atom index in w) and place in the sorted arrays
+  __shared__ float4 s_nf[CP_JB];
+  __shared__ int s_np[CP_JB];
+  __shared__ int s_off[TFF_WAVE + 1], s_js[TFF_WAVE];  // the half shell's cells (at most 63)
+  __shared__ float s_sh[3][TFF_WAVE];
   const int lane = threadIdx.x & (TFF_WAVE - 1);
-  const int wv = threadIdx.x / TFF_WAVE;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / TFF_WAVE);
   const int home = blockIdx.x;
   if (home >= g.ncell) return;
   // WRITE: the next row of this wave; else its count
@@ -247,12 +254,43 @@ __global__ __launch_bounds__(CP_WAVES * TFF_WAVE) void k_cell_pairs(
   if (WRITE && home == 0 && threadIdx.x == 0) *npairs = woff[g.ncell * CP_WAVES];
   const int hs = start[home];
   const int ni_all = start[home + 1] - hs;
-  const int hz = home % g.nc[2];
-  const int hy = (home / g.nc[2]) % g.nc[1];
-  const int hx = home / (g.nc[2] * g.nc[1]);
   const int R = g.reach;
   const int side = 2 * R + 1;
-  const int noff = side * side * side;
+  const int noff = side * side * side, ncells = noff - noff / 2;
+  if (threadIdx.x < TFF_WAVE) {
+    // lane c: the half shell's cell c (offsets with linear index >= centre, the centre first)
+    int js = 0, nj = 0;
+    float sx = 0.f, sy = 0.f, sz = 0.f;
+    if (lane < ncells && ni_all > 0) {
+      const int hz = home % g.nc[2];
+      const int hy = (home / g.nc[2]) % g.nc[1];
+      const int hx = home / (g.nc[2] * g.nc[1]);
+      const int o = noff / 2 + lane;
+      int nx = hx + o / (side * side) - R, ny = hy + (o / side) % side - R, nz = hz + o % side - R;
+      sx = nx < 0 ? -g.L[0] : (nx >= g.nc[0] ? g.L[0] : 0.f);
+      sy = ny < 0 ? -g.L[1] : (ny >= g.nc[1] ? g.L[1] : 0.f);
+      sz = nz < 0 ? -g.L[2] : (nz >= g.nc[2] ? g.L[2] : 0.f);
+      nx += nx < 0 ? g.nc[0] : (nx >= g.nc[0] ? -g.nc[0] : 0);
+      ny += ny < 0 ? g.nc[1] : (ny >= g.nc[1] ? -g.nc[1] : 0);
+      nz += nz < 0 ? g.nc[2] : (nz >= g.nc[2] ? -g.nc[2] : 0);
+      const int nb = (nx * g.nc[1] + ny) * g.nc[2] + nz;
+      js = start[nb];
+      nj = start[nb + 1] - js;
+    }
+    int incl = nj;
+    for (int o = 1; o < TFF_WAVE; o <<= 1) {
+      const int v = __shfl_up(incl, o, TFF_WAVE);
+      if (lane >= o) incl += v;
+    }
+    s_off[lane] = incl - nj;
+    if (lane == TFF_WAVE - 1) s_off[TFF_WAVE] = incl;
+    s_js[lane] = js;
+    s_sh[0][lane] = sx;
+    s_sh[1][lane] = sy;
+    s_sh[2][lane] = sz;
+  }
+  __syncthreads();
+  const int total = s_off[TFF_WAVE];
   for (int h0 = 0; h0 < ni_all; h0 += CP_HOME) {
     const int ni = ni_all - h0 < CP_HOME ? ni_all - h0 : CP_HOME;
     __syncthreads();  // the previous chunk's readers are done
@@ -262,7 +300,7 @@ __global__ __launch_bounds__(CP_WAVES * TFF_WAVE) void k_cell_pairs(
       double4 r = sxyz[pa];
       r.w = (double)ai;
       s_h[threadIdx.x] = r;
-      if (g.pf) s_hf[threadIdx.x] = sf[pa];
+      s_hf[threadIdx.x] = PF ? sf[pa] : make_float4(0.f, 0.f, 0.f, __int_as_float(ai));
       int ex[CP_EX] = {-1, -1, -1, -1};
       if (col) {
         const int64_t e0 = row_ptr[ai], e1 = row_ptr[ai + 1];
@@ -275,113 +313,74 @@ __global__ __launch_bounds__(CP_WAVES * TFF_WAVE) void k_cell_pairs(
       }
       s_hx[threadIdx.x] = make_int4(ex[0], ex[1], ex[2], ex[3]);
     }
-    __syncthreads();
-    // this wave's cells of the half shell (offsets with linear index >= centre, the centre first
-    // being the home cell): o = noff / 2 + wv + CP_WAVES c; lane c holds cell c's start and size
-    const int ncw = (noff - noff / 2 - wv + CP_WAVES - 1) / CP_WAVES;
-    int my_js = 0, my_nj = 0;
-    float my_sx = 0.f, my_sy = 0.f, my_sz = 0.f;  // the cell's periodic shift (prefilter)
-    if (lane < ncw) {
-      const int o = noff / 2 + wv + CP_WAVES * lane;
-      const int ox = o / (side * side) - R, oy = (o / side) % side - R, oz = o % side - R;
-      int nx = hx + ox, ny = hy + oy, nz = hz + oz;
-      my_sx = nx < 0 ? -g.L[0] : (nx >= g.nc[0] ? g.L[0] : 0.f);
-      my_sy = ny < 0 ? -g.L[1] : (ny >= g.nc[1] ? g.L[1] : 0.f);
-      my_sz = nz < 0 ? -g.L[2] : (nz >= g.nc[2] ? g.L[2] : 0.f);
-      nx += nx < 0 ? g.nc[0] : (nx >= g.nc[0] ? -g.nc[0] : 0);
-      ny += ny < 0 ? g.nc[1] : (ny >= g.nc[1] ? -g.nc[1] : 0);
-      nz += nz < 0 ? g.nc[2] : (nz >= g.nc[2] ? -g.nc[2] : 0);
-      const int nb = (nx * g.nc[1] + ny) * g.nc[2] + nz;
-      my_js = start[nb];
-      my_nj = start[nb + 1] - my_js;
-    }
-    // the first 64 atoms of the next cell are loaded into registers while the current one is walked
-    double4 pre_x = make_double4(0, 0, 0, 0);
-    float4 pre_f = make_float4(0, 0, 0, 0);
-    int pre_i = 0;
-    if (ncw > 0) {
-      const int js = __shfl(my_js, 0, TFF_WAVE), nj = __shfl(my_nj, 0, TFF_WAVE);
-      if (lane < nj) {
-        pre_x = sxyz[js + lane];
-        pre_i = sorted_idx[js + lane];
-        if (g.pf) pre_f = sf[js + lane];
-      }
-    }
-    for (int c = 0; c < ncw; ++c) {
-      const int js = __shfl(my_js, c, TFF_WAVE);
-      const int nj_all = __shfl(my_nj, c, TFF_WAVE);
-      const bool self_cell = wv == 0 && c == 0;
-      const float shx = __shfl(my_sx, c, TFF_WAVE), shy = __shfl(my_sy, c, TFF_WAVE),
-                  shz = __shfl(my_sz, c, TFF_WAVE);
-      // this cell's first 64 atoms from the registers, then the next cell's load is issued (also
-      // when this cell is empty)
-      if (lane < nj_all) {
-        s_n[wv][lane] = make_double4(pre_x.x, pre_x.y, pre_x.z, (double)pre_i);
-        s_nf[wv][lane] = make_float4(pre_f.x + shx, pre_f.y + shy, pre_f.z + shz, pre_f.w);
-      }
-      tff_wave_sync_lds();
-      if (c + 1 < ncw) {
-        const int jsn = __shfl(my_js, c + 1, TFF_WAVE), njn = __shfl(my_nj, c + 1, TFF_WAVE);
-        if (lane < njn) {
-          pre_x = sxyz[jsn + lane];
-          pre_i = sorted_idx[jsn + lane];
-          if (g.pf) pre_f = sf[jsn + lane];
+    for (int f0 = 0; f0 < total; f0 += CP_JB) {
+      const int nb = total - f0 < CP_JB ? total - f0 : CP_JB;
+      __syncthreads();  // the previous batch's readers are done
+      for (int k = threadIdx.x; k < nb; k += CP_WAVES * TFF_WAVE) {
+        int c = 0;  // the last cell that starts at or before this atom
+        for (int step = TFF_WAVE / 2; step > 0; step >>= 1)
+          if (s_off[c + step] <= f0 + k) c += step;
+        const int p = s_js[c] + f0 + k - s_off[c];
+        s_np[k] = p;
+        if (PF) {
+          const float4 v = sf[p];
+          s_nf[k] = make_float4(v.x + s_sh[0][c], v.y + s_sh[1][c], v.z + s_sh[2][c], v.w);
+        } else {
+          s_nf[k] = make_float4(0.f, 0.f, 0.f, __int_as_float(sorted_idx[p]));
         }
       }
-      for (int j0 = 0; j0 < nj_all; j0 += TFF_WAVE) {
-        const int nj = nj_all - j0 < TFF_WAVE ? nj_all - j0 : TFF_WAVE;
-        if (j0 > 0) {
-          if (lane < nj) {
-            const double4 r = sxyz[js + j0 + lane];
-            s_n[wv][lane] = make_double4(r.x, r.y, r.z, (double)sorted_idx[js + j0 + lane]);
-            if (g.pf) {
-              const float4 f = sf[js + j0 + lane];
-              s_nf[wv][lane] = make_float4(f.x + shx, f.y + shy, f.z + shz, f.w);
+      __syncthreads();
+      for (int k0 = wv * TFF_WAVE; k0 < nb; k0 += CP_WAVES * TFF_WAVE) {
+        const int k = k0 + lane;
+        const bool live = k < nb;
+        const float4 fb = s_nf[live ? k : 0];
+        const int p = s_np[live ? k : 0], bj = __float_as_int(fb.w);
+        double4 rb = make_double4(0, 0, 0, 0);
+        if (!PF) rb = sxyz[p];
+        const unsigned long long lm = __builtin_amdgcn_ballot_w64(live);
+#pragma unroll 2
+        for (int a = 0; a < ni; ++a) {
+          const float4 fa = s_hf[a];
+          const int4 hx = s_hx[a];
+          // the masks stay in scalar registers.  A pair within the home cell counts once: this atom against
+          // the later ones of the shell's order (the home cell leads it), itself on request
+          unsigned long long in = 0, near = lm;
+          if (PF) {
+            const float ex = fa.x - fb.x, ey = fa.y - fb.y, ez = fa.z - fb.z;
+            const float d2f = ex * ex + ey * ey + ez * ez;
+            in = __builtin_amdgcn_ballot_w64(d2f < g.lo) & lm;
+            near = __builtin_amdgcn_ballot_w64(!(d2f > g.hi)) & lm & ~in;
+          }
+          const int d = h0 + a - (f0 + k0);
+          const unsigned long long later = d < 0 ? ~0ull : d < 63 ? ~0ull << (d + 1) : 0ull;
+          in &= later;
+          near &= later;
+          if (near) {
+            bool ok = false;
+            if ((near >> lane) & 1ull) {
+              const double4 ra = s_h[a];
+              if (PF) rb = sxyz[p];
+              ok = tff_dist2_d(box, ra.x - rb.x, ra.y - rb.y, ra.z - rb.z) <= cutoff2;
+            }
+            in |= __builtin_amdgcn_ballot_w64(ok);
+          }
+          if (include_self && d >= 0 && d < 64) in |= 1ull << d;
+          const int ai = __builtin_amdgcn_readfirstlane(__float_as_int(fa.w));
+          if (col) {
+            const unsigned long long out =
+                __builtin_amdgcn_ballot_w64(hx.x == bj) | __builtin_amdgcn_ballot_w64(hx.y == bj) |
+                __builtin_amdgcn_ballot_w64(hx.z == bj) | __builtin_amdgcn_ballot_w64(hx.w == bj);
+            in &= ~out;
+            if (__builtin_amdgcn_readfirstlane(hx.x) == -2) {
+              const bool ex = ((in >> lane) & 1ull) && tff_is_excluded(ai, bj, row_ptr, col);
+              in &= ~__builtin_amdgcn_ballot_w64(ex);
             }
           }
-          tff_wave_sync_lds();
-        }
-        const int total = ni * nj;
-        int a = lane / nj, b = lane - a * nj;
-        const int da = TFF_WAVE / nj, db = TFF_WAVE - da * nj;
-        for (int t0 = 0; t0 < total; t0 += TFF_WAVE) {
-          bool ok = false;
-          int ai = 0, bj = 0;
-          if (a < ni) {
-            const int pa = h0 + a, pb = j0 + b;  // positions within their cells
-            if (!self_cell || pa <= pb) {
-              const int4 hx = s_hx[a];
-              bool exact = true;
-              if (g.pf) {
-                const float4 fa = s_hf[a], fb = s_nf[wv][b];
-                ai = __float_as_int(fa.w);
-                bj = __float_as_int(fb.w);
-                const float ex = fa.x - fb.x, ey = fa.y - fb.y, ez = fa.z - fb.z;
-                const float d2f = ex * ex + ey * ey + ez * ez;
-                ok = d2f < g.lo;
-                exact = !(d2f < g.lo) && !(d2f > g.hi);
-              }
-              if (self_cell && pa == pb) {
-                const double4 ra = s_h[a];
-                ai = bj = (int)ra.w;
-                ok = include_self != 0;
-              } else if (exact) {
-                const double4 ra = s_h[a], rb = s_n[wv][b];
-                ai = (int)ra.w;
-                bj = (int)rb.w;
-                const double d2 = tff_dist2_d(box, ra.x - rb.x, ra.y - rb.y, ra.z - rb.z);
-                ok = d2 <= cutoff2;
-              }
-              if (ok && col) {
-                bool ex = (hx.x == bj) | (hx.y == bj) | (hx.z == bj) | (hx.w == bj);
-                if (hx.x == -2) ex = tff_is_excluded(ai, bj, row_ptr, col);
-                ok = !ex;
-              }
-            }
-          }
-          const unsigned long long m = __ballot(ok);
+          const unsigned long long m = in;
+          const bool ok = (m >> lane) & 1ull;
           if (WRITE && ok) {
-            const long long row = pos + __popcll(m & ((1ull << lane) - 1ull));
+            const long long row = pos + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
             if (row < max_npairs) {
               longlong2 v;
               v.x = ai > bj ? ai : bj;
@@ -390,14 +389,7 @@ __global__ __launch_bounds__(CP_WAVES * TFF_WAVE) void k_cell_pairs(
             }
           }
           pos += __popcll(m);
-          a += da;
-          b += db;
-          if (b >= nj) {
-            b -= nj;
-            ++a;
-          }
         }
-        tff_wave_sync_lds();  // before the next chunk restages s_n
       }
     }
   }
@@ -589,13 +581,14 @@ extern "C" int tff_build_neighbor_list(int dtype, const void* coords, long long 
   hipLaunchKernelGGL(k_scatter, dim3(nbk), dim3(256), 0, stream, ws.xyz, natoms, box, ws.cell_of, ws.start,
                      ws.cursor, ws.sidx, ws.sxyz, ws.sf);
   void* tok = tff_prof_begin("nblist_cell_pairs", stream);
-  hipLaunchKernelGGL(k_cell_pairs<false>, dim3(m), dim3(CP_WAVES * TFF_WAVE), 0, stream, ws.start, ws.sidx,
-                     ws.sxyz, (const float4*)ws.sf, g, box, cutoff2, include_self, excl_row_ptr, excl_col,
-                     ws.wcount, (const int*)ws.woff, P, max_npairs, NP);
+  auto walk = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(m), dim3(CP_WAVES * TFF_WAVE), 0, stream, ws.start, ws.sidx, ws.sxyz,
+                       (const float4*)ws.sf, g, box, cutoff2, include_self, excl_row_ptr, excl_col, ws.wcount,
+                       (const int*)ws.woff, P, max_npairs, NP);
+  };
+  walk(g.pf ? k_cell_pairs<false, true> : k_cell_pairs<false, false>);
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, stream, ws.wcount, m * CP_WAVES, ws.woff);
-  hipLaunchKernelGGL(k_cell_pairs<true>, dim3(m), dim3(CP_WAVES * TFF_WAVE), 0, stream, ws.start, ws.sidx,
-                     ws.sxyz, (const float4*)ws.sf, g, box, cutoff2, include_self, excl_row_ptr, excl_col,
-                     ws.wcount, (const int*)ws.woff, P, max_npairs, NP);
+  walk(g.pf ? k_cell_pairs<true, true> : k_cell_pairs<true, false>);
   tff_prof_end(tok, stream);
   TFF_CHECK_LAUNCH("k_cell_pairs");
   return fill_tail();
