@@ -217,37 +217,49 @@ __global__ __launch_bounds__(256) void k_spread(const T* __restrict__ coords, Mu
   }
   for (int k = threadIdx.x; k < SB_Z * SB; k += blockDim.x) s_b[k] = 0.0;
   // source bricks: per axis those holding a stencil base in [B0 - P + 1, B0 + Bn - 1] (periodic);
-  // their atom ranges are concatenated so that every thread takes atoms of the whole set
-  __shared__ int s_a0[SB_SRC * SB_SRC * SB_SRC], s_pref[SB_SRC * SB_SRC * SB_SRC + 1], s_nc;
-  if (threadIdx.x == 0) {
-    int src[3][SB_SRC], ns[3];
-    for (int a = 0; a < 3; ++a) {
-      ns[a] = 0;
-      for (int v = B0[a] - (P - 1); v <= B0[a] + Bn[a] - 1; ++v) {
-        int w = v % g.K[a];
-        w = w < 0 ? w + g.K[a] : w;
-        const int sb = w / SB;
-        bool seen = false;
-        for (int k = 0; k < ns[a]; ++k) seen |= src[a][k] == sb;
-        if (!seen && ns[a] < SB_SRC) src[a][ns[a]++] = sb;
-      }
+  // their atom ranges are concatenated so that every thread takes atoms of the whole set.  One lane per
+  // axis steps from brick to brick, one lane per combination loads its range: done by one thread,
+  // grid point by grid point, it cost 5 us of 23.5 for 300 waters on 24^3 and 15 us of 90 for
+  // 96k atoms with quadrupoles on 96^3
+  constexpr int NSRC = SB_SRC * SB_SRC * SB_SRC;
+  __shared__ int s_a0[NSRC], s_pref[NSRC + 1], s_src[3][SB_SRC], s_ns[3];
+  static_assert(NSRC == TFF_WAVE, "one wave holds the source bricks");
+  if (threadIdx.x < 3) {
+    const int a = threadIdx.x, K = a == 0 ? K0 : a == 1 ? K1 : K2, b0 = B[a] * SB, last = b0 + (K - b0 < SB ? K - b0 : SB) - 1;
+    int n = 0;
+    for (int v = b0 - (P - 1); v <= last;) {
+      int w = v % K;
+      w = w < 0 ? w + K : w;
+      const int sb = w / SB;
+      bool seen = false;
+      for (int k = 0; k < n; ++k) seen |= s_src[a][k] == sb;
+      if (!seen && n < SB_SRC) s_src[a][n++] = sb;
+      v += ((sb + 1) * SB < K ? (sb + 1) * SB : K) - w;
     }
-    int nc = 0, tot = 0;
-    for (int sx = 0; sx < ns[0]; ++sx)
-      for (int sy = 0; sy < ns[1]; ++sy)
-        for (int sz = 0; sz < ns[2]; ++sz) {
-          const int sb = (src[0][sx] * nb[1] + src[1][sy]) * nb[2] + src[2][sz];
-          s_a0[nc] = start[sb];
-          s_pref[nc] = tot;
-          tot += start[sb + 1] - start[sb];
-          ++nc;
-        }
-    s_pref[nc] = tot;
-    s_nc = nc;
+    s_ns[a] = n;
+  }
+  __syncthreads();
+  const int ncomb = s_ns[0] * s_ns[1] * s_ns[2];
+  if (threadIdx.x < TFF_WAVE) {
+    const int t = threadIdx.x, ny = s_ns[1], nz = s_ns[2];
+    int a0 = 0, len = 0;
+    if (t < ncomb) {
+      const int sb = (s_src[0][t / (ny * nz)] * nb[1] + s_src[1][t / nz % ny]) * nb[2] + s_src[2][t % nz];
+      a0 = start[sb];
+      len = start[sb + 1] - a0;
+    }
+    int incl = len;
+    for (int o = 1; o < TFF_WAVE; o <<= 1) {
+      const int v = __shfl_up(incl, o, TFF_WAVE);
+      if (t >= o) incl += v;
+    }
+    s_a0[t] = a0;
+    s_pref[t + 1] = incl;
+    if (t == 0) s_pref[0] = 0;
   }
   __syncthreads();
   constexpr int PD = LVL >= 2 ? P : 1;
-  const int ncomb = s_nc, total = s_pref[ncomb];
+  const int total = s_pref[ncomb];
   {
         for (int k = (int)threadIdx.x; k < total; k += blockDim.x) {
           int c = 0;
@@ -618,10 +630,11 @@ int launch_spread(int order, const T* coords, const Multipoles& mp, long long n,
   void* tok = tff_prof_begin("pme_spread", st);
   const int nbk = w.nbricks;
   {
-    int zb = (nbk + 255) / 256;
+    // counts, starts and cursors lie in a row: one launch clears them
+    const int words = (int)(w.bcursor - w.bcount) + nbk;
+    int zb = (words + 255) / 256;
     zb = zb > 4096 ? 4096 : (zb < 1 ? 1 : zb);
-    hipLaunchKernelGGL(k_zero_ints, dim3((unsigned)zb), dim3(256), 0, st, w.bcount, nbk);
-    hipLaunchKernelGGL(k_zero_ints, dim3((unsigned)zb), dim3(256), 0, st, w.bcursor, nbk);
+    hipLaunchKernelGGL(k_zero_ints, dim3((unsigned)zb), dim3(256), 0, st, w.bcount, words);
   }
   if (n > 0) {
     const unsigned nb = (unsigned)((n + 255) / 256);
