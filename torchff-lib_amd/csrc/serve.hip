@@ -129,46 +129,57 @@ __device__ __forceinline__ long long grid_term(double wab, double mc) {
   return __double2ll_rn(wab * mc * SQ_SCALE);
 }
 
-// spread of one task's atoms (a workgroup: lane = atom, the RW waves share the P^2 (a, b) stencil
-// columns): order-P B-spline weights, int64 fixed-point atomics
+// LDS of a spread task: the order-P weights of its 64 atoms by axis, their charges and stencil bases
+template <typename TC, int P>
+struct SpreadLds {
+  TC M[3][P][TFF_WAVE];
+  double q[TFF_WAVE];
+  int base[3][TFF_WAVE];  // base[0]: -1 without an atom
+};
+// Spread of one task's atoms (a workgroup): one thread per atom and axis evaluates the order-P B-spline weights,
+// then eight lanes take the z points of one atom's (a, b) stencil column, eight atoms per instruction,
+// with int64 fixed-point atomics.  A memory-side atomic costs one operation per 64-byte line that an
+// instruction touches (20 to 24 G/s): a column's P points lie on one or two lines and go together.
+// With one lane per atom every point was an operation of its own, some 2.5 M for 24 systems at order 5
+// (k_serve_real_spread 123 us, 88 this way; 16 boxes of an MD step 45 and 41: the real-space items now
+// set its time).
 template <typename TC, int P>
 __device__ __forceinline__ void spread_task(const BatchHead* __restrict__ hd, const SysDesc* __restrict__ d,
                                             const double* __restrict__ atoms, unsigned long long* __restrict__ grid,
-                                            int task, int lane, int wv) {
+                                            int task, SpreadLds<TC, P>& w) {
+  static_assert(P <= 8 && RW >= 3, "eight lanes a column, a wave per axis");
+  const int lane = threadIdx.x & (TFF_WAVE - 1), wv = threadIdx.x / TFF_WAVE;
   int s = 0;
   const int i = task_atom(hd, d, task, lane, s);
-  if (i < 0) return;
   const SysDesc& sd = d[s];
-  const int K0 = sd.cv.K[0], K1 = sd.cv.K[1], K2 = sd.cv.K[2];
-  const double* rec = atoms + (size_t)REC * i;
-  TC Mv[3][P], dM[3][P];
-  int base[3];
-  for (int a = 0; a < 3; ++a) {
-    double t;
-    anchor_axis(rec[a] * sd.invL[a] * (double)sd.cv.K[a], sd.cv.K[a], P, base[a], t);
-    spline_weights<TC, P>((TC)t, Mv[a], dM[a]);
+  if (wv < 3) {
+    int base = -1;
+    if (i >= 0) {
+      const double* rec = atoms + (size_t)REC * i;
+      TC Mv[P], dM[P];
+      double t;
+      anchor_axis(rec[wv] * sd.invL[wv] * (double)sd.cv.K[wv], sd.cv.K[wv], P, base, t);
+      spline_weights<TC, P>((TC)t, Mv, dM);
+#pragma unroll
+      for (int k = 0; k < P; ++k) w.M[wv][k][lane] = Mv[k];
+      if (wv == 0) w.q[lane] = rec[3];
+    }
+    w.base[wv][lane] = base;
   }
-  const double qi = rec[3];
+  __syncthreads();
+  const int K0 = sd.cv.K[0], K1 = sd.cv.K[1], K2 = sd.cv.K[2];
   unsigned long long* g = grid + sd.grid_off;
-  for (int ab = wv; ab < P * P; ab += RW) {
-    const int a = ab / P, b = ab - a * P;
-    int gx = base[0] + a, gy = base[1] + b;
-    while (gx >= K0) gx -= K0;  // a, b < P: a few steps even when K < P
+  const int c = lane & 7;
+  for (int u = wv; u < 8 * P * P; u += RW) {
+    const int ab = u >> 3, a = ab / P, b = ab - a * P;
+    const int m = (u & 7) * 8 + (lane >> 3);
+    if (c >= P || w.base[0][m] < 0) continue;
+    int gx = w.base[0][m] + a, gy = w.base[1][m] + b, gz = w.base[2][m] + c;
+    while (gx >= K0) gx -= K0;  // a, b, c < P: a few steps even when K < P
     while (gy >= K1) gy -= K1;
-    TC ma = Mv[0][0], mb = Mv[1][0];
-#pragma unroll
-    for (int k = 1; k < P; ++k) {
-      ma = a == k ? Mv[0][k] : ma;
-      mb = b == k ? Mv[1][k] : mb;
-    }
-    const double wab = qi * (double)ma * (double)mb;
-    unsigned long long* row = g + ((long long)gx * K1 + gy) * K2;
-    int gz = base[2];
-#pragma unroll
-    for (int c = 0; c < P; ++c) {
-      atomicAdd(&row[gz], (unsigned long long)grid_term(wab, Mv[2][c]));
-      gz = gz + 1 == K2 ? 0 : gz + 1;
-    }
+    while (gz >= K2) gz -= K2;
+    const double wab = w.q[m] * (double)w.M[0][a][m] * (double)w.M[1][b][m];
+    atomicAdd(&g[((long long)gx * K1 + gy) * K2 + gz], (unsigned long long)grid_term(wab, w.M[2][c][m]));
   }
 }
 
@@ -319,11 +330,12 @@ __global__ __launch_bounds__(RW * TFF_WAVE) void k_serve_real_spread(const Batch
   constexpr int STAGE = TFF_WAVE * (sizeof(P4<TC>) + sizeof(L4<TC>));
   constexpr int RED = RW / 2 * 4 * TFF_WAVE * sizeof(double);
   __shared__ __align__(16) unsigned char lds[RW * STAGE > RED ? RW * STAGE : RED];
+  static_assert(sizeof(SpreadLds<TC, P>) <= sizeof(lds), "a spread task fits the staging area");
   const int nsp = hd->ntask;
   const int nitems = nsp + hd->nwork;
   for (int it = blockIdx.x; it < nitems; it += gridDim.x) {  // uniform over the workgroup
     if (it < nsp) {
-      spread_task<TC, P>(hd, d, atoms, grid, it, threadIdx.x & (TFF_WAVE - 1), threadIdx.x / TFF_WAVE);
+      spread_task<TC, P>(hd, d, atoms, grid, it, *reinterpret_cast<SpreadLds<TC, P>*>(lds));
     } else {
       real_item<TC>(hd, d, atoms, coul, it - nsp, lds, STAGE, freal, epart);
     }
