@@ -28,16 +28,21 @@ __device__ __forceinline__ void erfc_exp(float u, float& ec, float& em) {
   em = __builtin_amdgcn_exp2f(u * u * -1.44269502f);
   ec = erfc_scaled(u) * em;
 }
-// double: both from one argument, without a branch.  -u^2 = n ln 2 + r with the rounding of u^2 taken
-// into r (the library call on the rounded square is off by up to u^2 ulp), exp(r) a degree-11
-// polynomial; erfc(u) exp(u^2) a degree-21 polynomial in t = (1.28125 u - 3.75) / (u + 3.75), which
-// maps [0, 26.67] onto [-1, 1]: both are Chebyshev interpolants computed in 60 digits, 3e-18 and 4e-18
-// off in exact arithmetic.  u is cut at 27.5, where both results are 0 already (a padding pair at 1e15
-// stays exactly 0).  Measured against 25-digit values for u in [0, 3.6], rms and largest: erfc 9.7e-17
-// and 3.2e-16 (library 9.8e-17, 3.4e-16), exp(-u^2) 5.0e-17 and 1.4e-16 (library 2.8e-16, 1.0e-15);
-// over r in [0.9, 9] A at alpha 0.3 A^-1 the pair energies are off by 5.8e-16 rms and their forces by
-// 5.2e-16 (library 6.2e-16, 5.7e-16).  Bound by the FP64 rate: erfc, exp and 1 / sqrt of a million
-// pairs took 5.4 us with the library's, 3.2 us with these (k_tiles_f64 of 60k water atoms 256 -> 190 us).
+// double: both from one argument, without a branch.  -u^2 = n ln 2 + r with u^2 unrounded (the library call
+// on the rounded square is off by up to u^2 ulp), exp(r) a degree-11 polynomial; (u + K) erfc(u) exp(u^2) a
+// degree-23 polynomial in t = (A u - K) / (u + K) = A - K (A + 1) / (u + K), which maps [0, 27.9] onto
+// [-1, 1]: both are Chebyshev interpolants computed in 60 digits, 3e-18 and 3e-17 off in exact
+// arithmetic.  The factor u + K leaves the polynomial to run from 2.4 to 0.6; erfc(u) exp(u^2) alone
+// runs from 1 to 0.02, where its even and odd parts cancel (3.7e-15 off for u in [10, 20]).  It is the
+// factor 1 + 2 u of Shepherd and Laframboise, Math. Comp. 36, 1981, in a form whose reciprocal t needs
+// anyway; K = 151 / 64 and A were chosen among short numbers so that the constant term is a double to
+// 3e-20.  The reciprocal, the constant and linear terms and exp(r) carry their roundings along.  u is
+// cut at 27.5, where both results are 0 already (a padding pair at 1e15 stays exactly 0).
+// Relative errors against 28 digits (this arithmetic on the host), rms and largest: erfc 5.8e-17 and 2.1e-16
+// for u in [0, 3.6] (C library 8.4e-17, 4.7e-16), at most 7.8e-17 and 3.0e-16 on [3.6, 26] (library
+// 8.8e-17, 3.2e-16); exp(-u^2) 5.0e-17 and 1.6e-16 throughout (library call 2.8e-16, 1.0e-15 on [0, 3.6]).
+// Bound by the FP64 rate: one evaluation of 60k water atoms takes 392 us with the library's functions, 374 us
+// with these (372 us with the polynomial for erfc(u) exp(u^2) alone).
 // Each coefficient is the scalar addend of a v_fma: left to itself the compiler moves it into a
 // vector register first, one move per fma (3.7 us instead of 2.75 before the last corrections).
 __device__ __forceinline__ double fma_coef(double a, double b, double c) {
@@ -49,39 +54,43 @@ static __device__ constexpr double EXP_C[12] = {
     0x1.0000000000000p+0, 0x1.0000000000000p+0, 0x1.0000000000011p-1, 0x1.5555555555562p-3,
     0x1.555555554f0ccp-5, 0x1.111111110db75p-7, 0x1.6c16c187fc3e6p-10, 0x1.a01a01b802660p-13,
     0x1.a01991aba6f13p-16, 0x1.71dde76a2f6d2p-19, 0x1.28b40639f7187p-22, 0x1.af785e0a5dff9p-26};
-static __device__ constexpr double ERFCX_C[22] = {
-    0x1.76eb8a31072c7p-3, -0x1.2ef15ea35aa48p-2, 0x1.d37d59145d1aep-3, -0x1.34696a5469df1p-3,
-    0x1.58bb04227d1b5p-4, -0x1.403d71bd5537ap-5, 0x1.dc2a28605774fp-7, -0x1.04408f6e53ca3p-8,
-    0x1.396ede3f17fbcp-11, 0x1.009e30e82b512p-14, -0x1.d97c3d57c13bbp-15, 0x1.1413239c0c019p-17,
-    0x1.80d1790065794p-19, -0x1.30947befef2fcp-20, -0x1.d8805c68c88f3p-24, 0x1.f05ff1829a28ep-24,
-    0x1.56ec6dfa80deep-29, -0x1.8e2cfdf20744fp-27, 0x1.35ce6dd1300acp-35, 0x1.358385ec92ffdp-30,
-    -0x1.40d78682a7ecfp-39, -0x1.52433b61b276dp-34};
+static __device__ constexpr double ERFCX_K = 2.359375, ERFCX_A = 1.16888427734375;
+static __device__ constexpr double ERFCX_C[24] = {
+    0x1.1c08996a7f535p+0, -0x1.8db9f04495585p-1, 0x1.7eece391e3014p-2, -0x1.acfb97a3f0883p-4,
+    0x1.8d76d6840b2f1p-9, 0x1.114fd1049d386p-7, -0x1.3d0b470d9a8cap-10, -0x1.ca64e770e7228p-11,
+    0x1.1aaaa78517553p-13, 0x1.04979d2286077p-13, -0x1.5866a7aae1bb6p-18, -0x1.44959b93d7645p-16,
+    -0x1.832bd42588626p-19, 0x1.535dc11cf178ep-19, 0x1.3398120a23249p-20, -0x1.031b85d7f71edp-23,
+    -0x1.0f910b0826991p-22, -0x1.0a2409b18687fp-24, 0x1.13cf99d0fa925p-25, 0x1.92ccb01864b9bp-26,
+    -0x1.8023504096768p-31, -0x1.214244ff06bf4p-28, -0x1.5bdc4714cdf1ap-32, 0x1.7c0b3c7a2ada2p-32};
 __device__ __forceinline__ void erfc_exp(double u, double& ec, double& em) {
-  u = u > 27.5 ? 27.5 : u;  // (a NaN stays one)
-  const double u2 = u * u, lo = fma(u, u, -u2);
-  const double n = rint(u2 * -1.4426950408889634);
-  const double r = fma(n, -0x1.abc9e3b39803fp-56, fma(n, -0x1.62e42fefa39efp-1, -u2)) - lo;
-  double p = EXP_C[11];
+  u = __hiloint2double(u > 27.5 ? 0x403b8000 : __double2hiint(u), __double2loint(u));  // high word only; a NaN stays one
+  // n = rint(-u^2 log2 e): the integer is the low word of its sum with 1.5 2^52; ln 2 in two parts, the first of
+  // 42 bits, so that n times it is exact
+  const double nm = fma(u * u, -1.4426950408889634, 6755399441055744.0), n = nm - 6755399441055744.0;
+  const int ni = __double2loint(nm);
+  const double r = fma(n, -0x1.ef35793c7673p-45, fma(-u, u, n * -0x1.62e42fefa38p-1));
+  double g = EXP_C[11];
 #pragma unroll
-  for (int k = 10; k >= 0; --k) p = fma_coef(p, r, EXP_C[k]);
-  em = ldexp(p, (int)n);
-  const double d = u + 3.75;
-  double w = __builtin_amdgcn_rcp(d);  // off by at most 5e-8
-  const double e = fma(-d, w, 1.0);
-  w = fma(w * e, e + 1.0, w);
-  // t = (1.28125 u - 3.75) / (u + 3.75), corrected by the roundings of numerator, denominator and quotient
-  const double num = fma(u, 1.28125, -3.75), dlo = u - (d - 3.75), nlo = fma(u, 1.28125, -(num + 3.75));
-  double t = num * w;
-  t = fma(fma(-t, d, num) + fma(-t, dlo, nlo), w, t);
+  for (int k = 10; k >= 1; --k) g = fma_coef(g, r, EXP_C[k]);
+  const double p = fma(g, r, 1.0), h = g * r;  // exp(r), exp(r) - 1
+  em = ldexp(p, ni);
+  // w + wl = 1 / (u + K): w the float reciprocal, off by e (at most 2e-7), wl = w (e + e^2); w's 24 bits
+  // make its product with K and the subtraction from 1 exact
+  const double w = (double)__builtin_amdgcn_rcpf((float)(u + ERFCX_K));
+  const double e = fma(-w, u, fma(-w, ERFCX_K, 1.0)), wl = fma(e, e, e) * w;
+  const double t = fma(-ERFCX_K * (ERFCX_A + 1.0), wl, fma(-ERFCX_K * (ERFCX_A + 1.0), w, ERFCX_A));
   const double t2 = t * t;
-  double a = ERFCX_C[20], b = ERFCX_C[21];  // even and odd powers: two chains
+  double a = ERFCX_C[22], b = ERFCX_C[23];  // even and odd powers: two chains
 #pragma unroll
-  for (int k = 18; k >= 0; k -= 2) {
+  for (int k = 20; k >= 2; k -= 2) {
     a = fma_coef(a, t2, ERFCX_C[k]);
     b = fma_coef(b, t2, ERFCX_C[k + 1]);
   }
-  const double f = fma(b, t, a);
-  ec = fma(f, em, fma(b, t, a - f) * em);
+  // f + fl = (u + K) erfc(u) exp(u^2), constant and linear terms last
+  const double c1t = ERFCX_C[1] * t, s = fma(fma(b, t, a), t2, c1t), f = ERFCX_C[0] + s;
+  const double fl = ((ERFCX_C[0] - f) + s) + fma(ERFCX_C[1], t, -c1t);
+  const double q = f * w, ql = fma(fl, w, fma(f, wl, fma(f, w, -q)));
+  ec = ldexp(q + fma(q, h, ql * p), ni);
 }
 // the same with 1 subtracted from erfc where excl is set (float: in one rounding)
 __device__ __forceinline__ void erfc_exp_excl(float u, bool excl, float& ec, float& em) {
