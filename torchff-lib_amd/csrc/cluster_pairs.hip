@@ -626,11 +626,14 @@ __global__ void k_cp_npairs(const long long* __restrict__ off, long long total, 
 }
 
 // ---------------------------------------------------------------- nonbonded terms
-// 16-lane row rotation: lane l takes the value of lane l - 1 of its row
-__device__ __forceinline__ int ror1(int v) { return __builtin_amdgcn_mov_dpp(v, 0x121, 0xf, 0xf, true); }
-__device__ __forceinline__ float ror1(float v) { return __int_as_float(ror1(__float_as_int(v))); }
-__device__ __forceinline__ double ror1(double v) {
-  return __hiloint2double(ror1(__double2hiint(v)), ror1(__double2loint(v)));
+// 16-lane row rotation: lane l takes the value of lane l - K of its row
+template <int K>
+__device__ __forceinline__ int ror(int v) { return __builtin_amdgcn_mov_dpp(v, 0x120 + K, 0xf, 0xf, true); }
+template <int K>
+__device__ __forceinline__ float ror(float v) { return __int_as_float(ror<K>(__float_as_int(v))); }
+template <int K>
+__device__ __forceinline__ double ror(double v) {
+  return __hiloint2double(ror<K>(__double2hiint(v)), ror<K>(__double2loint(v)));
 }
 __device__ __forceinline__ void half_sync() {  // the wave's own LDS writes before its reads
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -701,16 +704,20 @@ __device__ __forceinline__ void cp_flush(int a, const double (&v)[CpCh<LJG>::N],
 //
 // A half-wave takes a run of consecutive entries (they mostly share their cluster x, whose atoms' sums
 // stay in registers, float64, until x changes).  Its two rows of 16 lanes take 16 of the column atoms
-// each, which then go round the row by DPP together with their sums (T, at most 32 terms, as the
-// sums of a column by butterfly would be), 16 steps, twice: no shuffle and no reduction per column.
+// each, which then go round the row by DPP together with their sums, 16 steps, twice: no shuffle and no
+// reduction per column.  A column's sums are T for CP_CHAIN steps and float64 from there on: for 32 terms of
+// like size their squared rounding error is 140 (in units of a rounding of one term), where a butterfly over
+// the rows has 160 and one sum over all steps 527.  (List and terms of the call below: 463 us with one sum,
+// 470 with chains of 8, 474 of 4, which spill.)
 // The pair predicate is that of the decoded list, in float64: T = float decides by its own r^2
 // unless that is within its error bound `tol_k` (|x_i| + |x_j| + box) of rc^2.
 // Bound by the arithmetic of the candidate pairs (of 32 x 32 per entry about one in five is within the
-// cutoff; some 150 instructions a step).  96k water atoms, float, all gradients: 275 us (energy alone
+// cutoff; some 150 instructions a step).  96k water atoms, float, all gradients: 283 us (energy alone
 // 150); one column per step by shuffles, a butterfly per gradient and an atomic per atom and channel
 // took 683.  Testing all pairs first and working off each lane's hits, with the column sums in LDS, took
 // 828: the fullest lane of 64 has nearly all 32 columns.
 // BOX: 0 no box, 1 orthorhombic, 2 general.
+constexpr int CP_CHAIN = 8;
 template <typename T, int GRAD, int BOX>
 __global__ __launch_bounds__(CPB) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 3))) void k_cp_nonbonded(const T* __restrict__ coords, CpGeom g, Entries en, int run,
                                                       const T* __restrict__ q, const T* __restrict__ sig,
@@ -776,74 +783,80 @@ __global__ __launch_bounds__(CPB) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
         r2_in = rc2 - tol;
         r2_out = rc2 + tol;
       }
-      T gj[N];
-      for (int k = 0; k < N; ++k) gj[k] = 0;
+      double gd[N];  // the column's sums, float64 over chains of CP_CHAIN steps
+      for (int k = 0; k < N; ++k) gd[k] = 0.0;
       for (int h = 0; h < 2; ++h) {
         // bit 31 - k of `todo`: the pair of step k (column (l16 - k) & 15 of the row's block)
         const unsigned m16 = ((l >> 4) ^ h ? skip >> 16 : skip) & 0xffffu;
         int todo = (int)(~((m16 | m16 << 16) >> l16) << 15);
-        for (int c = 0; c < 16; ++c) {
-          T dx = xi - xj, dy = yi - yj, dz = zi - zj;
-          if constexpr (BOX == 1) {  // tff_min_image, its branches taken
-            dx *= v0; dy *= v1; dz *= v2;
-            dx = (dx - rint(dx)) * b0; dy = (dy - rint(dy)) * b1; dz = (dz - rint(dz)) * b2;
-          } else if constexpr (BOX == 2) {
-            tff_min_image<T>(g.box, dx, dy, dz);
-          }
-          T r2 = dx * dx + dy * dy + dz * dz;
-          bool ok = todo < 0;
-          if constexpr (sizeof(T) == 8) {
-            double ax = (double)xi - (double)xj, ay = (double)yi - (double)yj, az = (double)zi - (double)zj;
-            tff_min_image_d(g.box, ax, ay, az);
-            ok = ok && ax * ax + ay * ay + az * az <= g.rc2;
-          } else {
-            if (ok && !(r2 < r2_in || r2 > r2_out)) {
+        for (int c0 = 0; c0 < 16; c0 += CP_CHAIN) {
+          T gj[N];
+          for (int k = 0; k < N; ++k) gj[k] = 0;
+          for (int c = 0; c < CP_CHAIN; ++c) {
+            T dx = xi - xj, dy = yi - yj, dz = zi - zj;
+            if constexpr (BOX == 1) {  // tff_min_image, its branches taken
+              dx *= v0; dy *= v1; dz *= v2;
+              dx = (dx - rint(dx)) * b0; dy = (dy - rint(dy)) * b1; dz = (dz - rint(dz)) * b2;
+            } else if constexpr (BOX == 2) {
+              tff_min_image<T>(g.box, dx, dy, dz);
+            }
+            T r2 = dx * dx + dy * dy + dz * dz;
+            bool ok = todo < 0;
+            if constexpr (sizeof(T) == 8) {
               double ax = (double)xi - (double)xj, ay = (double)yi - (double)yj, az = (double)zi - (double)zj;
               tff_min_image_d(g.box, ax, ay, az);
-              ok = ax * ax + ay * ay + az * az <= g.rc2;
+              ok = ok && ax * ax + ay * ay + az * az <= g.rc2;
             } else {
-              ok = ok && r2 < r2_in;
+              if (ok && !(r2 < r2_in || r2 > r2_out)) {
+                double ax = (double)xi - (double)xj, ay = (double)yi - (double)yj, az = (double)zi - (double)zj;
+                tff_min_image_d(g.box, ax, ay, az);
+                ok = ax * ax + ay * ay + az * az <= g.rc2;
+              } else {
+                ok = ok && r2 < r2_in;
+              }
             }
-          }
-          if (ok) {
-            const T rinv = cp_rsqrt(r2), rinv2 = rinv * rinv;
-            const T qq = qi * qj * kc, ph = rinv - shift;
-            T en_ = qq * ph;
-            T dr = -qq * rinv * rinv2;
-            const T sij = si + sj, eij = cp_sqrt(ei * ej);
-            const T sr2 = sij * sij * rinv2, s6 = sr2 * sr2 * sr2;
-            en_ += (T)4 * eij * s6 * (s6 - (T)1);
-            const T w = (T)24 * eij * s6 * ((T)2 * s6 - (T)1);
-            dr -= w * rinv2;
-            e_acc += (double)en_;
-            if constexpr (GRAD != 0) {
-              fi[0] += (double)(dr * dx);
-              fi[1] += (double)(dr * dy);
-              fi[2] += (double)(dr * dz);
-              fi[3] += (double)(qj * ph);  // times k at the end
-              gj[0] -= dr * dx;
-              gj[1] -= dr * dy;
-              gj[2] -= dr * dz;
-              gj[3] += qi * ph;
+            if (ok) {
+              const T rinv = cp_rsqrt(r2), rinv2 = rinv * rinv;
+              const T qq = qi * qj * kc, ph = rinv - shift;
+              T en_ = qq * ph;
+              T dr = -qq * rinv * rinv2;
+              const T sij = si + sj, eij = cp_sqrt(ei * ej);
+              const T sr2 = sij * sij * rinv2, s6 = sr2 * sr2 * sr2;
+              en_ += (T)4 * eij * s6 * (s6 - (T)1);
+              const T w = (T)24 * eij * s6 * ((T)2 * s6 - (T)1);
+              dr -= w * rinv2;
+              e_acc += (double)en_;
+              if constexpr (GRAD != 0) {
+                fi[0] += (double)(dr * dx);
+                fi[1] += (double)(dr * dy);
+                fi[2] += (double)(dr * dz);
+                fi[3] += (double)(qj * ph);  // times k at the end
+                gj[0] -= dr * dx;
+                gj[1] -= dr * dy;
+                gj[2] -= dr * dz;
+                gj[3] += qi * ph;
+              }
+              if constexpr (LJG) {
+                const T ds = cp_div(w, sij) * (T)0.5;
+                const T de = eij > (T)0 ? cp_div((T)4 * s6 * (s6 - (T)1) * (T)0.5, eij) : (T)0;
+                fi[4] += (double)ds;
+                fi[5] += (double)(de * ej);
+                gj[4] += ds;
+                gj[5] += de * ei;
+              }
             }
-            if constexpr (LJG) {
-              const T ds = cp_div(w, sij) * (T)0.5;
-              const T de = eij > (T)0 ? cp_div((T)4 * s6 * (s6 - (T)1) * (T)0.5, eij) : (T)0;
-              fi[4] += (double)ds;
-              fi[5] += (double)(de * ej);
-              gj[4] += ds;
-              gj[5] += de * ei;
-            }
+            if constexpr (GRAD != 0)
+              for (int k = 0; k < N; ++k) gj[k] = ror<1>(gj[k]);
+            sj = ror<1>(sj);
+            ej = ror<1>(ej);
+            xj = ror<1>(xj);
+            yj = ror<1>(yj);
+            zj = ror<1>(zj);
+            qj = ror<1>(qj);
+            todo <<= 1;
           }
           if constexpr (GRAD != 0)
-            for (int k = 0; k < N; ++k) gj[k] = ror1(gj[k]);
-          sj = ror1(sj);
-          ej = ror1(ej);
-          xj = ror1(xj);
-          yj = ror1(yj);
-          zj = ror1(zj);
-          qj = ror1(qj);
-          todo <<= 1;
+            for (int k = 0; k < N; ++k) gd[k] = ror<CP_CHAIN>(gd[k]) + (double)gj[k];
         }
         // the other row's columns and their sums (twice: every lane ends with its own column)
         xj = __shfl_xor(xj, 16, 32);
@@ -853,11 +866,10 @@ __global__ __launch_bounds__(CPB) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
         sj = __shfl_xor(sj, 16, 32);
         ej = __shfl_xor(ej, 16, 32);
         if constexpr (GRAD != 0)
-          for (int k = 0; k < N; ++k) gj[k] = __shfl_xor(gj[k], 16, 32);
+          for (int k = 0; k < N; ++k) gd[k] = __shfl_xor(gd[k], 16, 32);
       }
       if constexpr (GRAD != 0) {
-        double gd[N];
-        for (int k = 0; k < N; ++k) gd[k] = k == 3 ? (double)gj[k] * coul : (double)gj[k];
+        gd[3] *= coul;
         cp_flush<LJG>(j, gd, s, acc);
       }
     }
