@@ -489,7 +489,9 @@ __global__ __launch_bounds__(PB) void k_pair_terms(const T* __restrict__ coords,
 // four rows per distinct atom in 2048 rows); adding per wave step instead cost 22 M memory-side line
 // operations at 96k atoms (26.6 M rows), which at about 20 G/s bounded the kernel (1389 us in float64
 // against 602 us this way, 2.5 M operations, bound by vector issue).  A row whose atom finds no slot in
-// PROBES steps (a list in random order) goes to the line directly.  Measured: 1024 threads and 2048
+// PROBES steps (a list in random order) goes to the line directly, eight lanes per line: the list above with
+// its rows shuffled takes 2.10 ms a call (2.04 by k_pair_terms, both bound by the line operations; 10.2 when each
+// lane added its atom's words itself).  Measured: 1024 threads and 2048
 // slots 637 us, 256 and 512 609 us, twice the slots per thread 856 us (one workgroup per CU).
 constexpr int XB = 512;              // threads
 constexpr int XLOG = 10;
@@ -519,19 +521,23 @@ struct AtomTable {
   long long* w;    // word c of slot s at w[c * XSTRIDE + s]
 };
 
-template <int NC>
-__device__ __forceinline__ void table_add(const AtomTable& t, int atom, const double (&v)[NC], const Acc& acc) {
+// atom's slot, taken if need be; -1 when PROBES steps find none
+__device__ __forceinline__ int table_slot(const AtomTable& t, int atom) {
   unsigned p = ((unsigned)atom * 2654435761u) >> (32 - XLOG);
-  int slot = -1;
   for (int k = 0; k < PROBES; ++k) {
     int old = t.key[p];
     if (old != atom) old = old == -1 ? atomicCAS(&t.key[p], -1, atom) : old;
-    if (old == -1 || old == atom) {
-      slot = (int)p;
-      break;
-    }
+    if (old == -1 || old == atom) return (int)p;
     p = (p + 1) & (XSLOTS - 1);
   }
+  return -1;
+}
+
+// adds v[c] to atom's slot; false when it has none (contributions too large for the integer words, which go to the
+// float64 fallback of the atom, are added in either case)
+template <int NC>
+__device__ __forceinline__ bool table_add(const AtomTable& t, int atom, const double (&v)[NC], const Acc& acc) {
+  const int slot = table_slot(t, atom);
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     long long hi, lo;
@@ -540,10 +546,38 @@ __device__ __forceinline__ void table_add(const AtomTable& t, int atom, const do
     } else if (slot >= 0) {
       atomicAdd((unsigned long long*)(t.w + c * XSTRIDE + slot), (unsigned long long)hi);
       atomicAdd((unsigned long long*)(t.w + (NC + c) * XSTRIDE + slot), (unsigned long long)lo);
-    } else {
-      atomicAdd((unsigned long long*)(acc.a + 8LL * atom + c), (unsigned long long)hi);
-      atomicAdd((unsigned long long*)(acc.a + 8LL * atom + 4 + c), (unsigned long long)lo);
     }
+  }
+  return slot >= 0;
+}
+
+// The lanes of m add v[c] to their atom's line (what table_add left), eight adjacent lanes per line: an operation per
+// line, where a lane adding its words by itself costs one per word.  s_w: the wave's 8 lines of 8 words,
+// s_k: their atoms.  Wave-uniform control flow.
+template <int NC>
+__device__ __forceinline__ void line_add(unsigned long long m, int atom, const double (&v)[NC], const Acc& acc,
+                                         long long* s_w, int* s_k) {
+  const int lane = threadIdx.x & (TFF_WAVE - 1);
+  while (m) {  // eight atoms at a time
+    const int rank = __popcll(m & ((1ull << lane) - 1ull)), n = __popcll(m);
+    const bool mine = ((m >> lane) & 1ull) && rank < 8;
+    if (mine) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        long long hi = 0, lo = 0;
+        if (c < NC) split_fast(v[c < NC ? c : 0], hi, lo);  // (both 0 where it went to the fallback)
+        s_w[8 * rank + c] = hi;
+        s_w[8 * rank + 4 + c] = lo;
+      }
+      s_k[rank] = atom;
+    }
+    m &= ~__ballot(mine);
+    tff_wave_sync_lds();
+    if (lane >> 3 < n) {
+      const long long x = s_w[lane];
+      if (x != 0) atomicAdd((unsigned long long*)(acc.a + 8LL * s_k[lane >> 3] + (lane & 7)), (unsigned long long)x);
+    }
+    tff_wave_sync_lds();
   }
 }
 
@@ -555,10 +589,12 @@ __global__ __launch_bounds__(XB) void k_pair_xyzq(const T* __restrict__ coords, 
                                                   const T* __restrict__ sig, const T* __restrict__ eps,
                                                   const long long* __restrict__ types, long long natoms,
                                                   double* __restrict__ e_part, Acc acc, int steps) {
-  extern __shared__ __align__(16) long long s_tab[];
+  extern __shared__ __align__(16) long long s_tab[];  // table words, then keys, then the waves' lines and their atoms
   const AtomTable tab{reinterpret_cast<int*>(s_tab + 2 * NC * XSTRIDE), s_tab};
   const int t = threadIdx.x, lane = t & (TFF_WAVE - 1), wv = t / TFF_WAVE;
   const int row = (wv / XROWS) * TFF_WAVE * XROWS + lane * XROWS + wv % XROWS;
+  long long* const s_w = s_tab + 2 * NC * XSTRIDE + XSLOTS / 2 + 64 * wv;
+  int* const s_k = reinterpret_cast<int*>(s_tab + 2 * NC * XSTRIDE + XSLOTS / 2 + 64 * (XB / TFF_WAVE)) + 8 * wv;
   if (NC) {
     for (int k = t; k < XSLOTS; k += XB) {
       tab.key[k] = -1;
@@ -576,36 +612,44 @@ __global__ __launch_bounds__(XB) void k_pair_xyzq(const T* __restrict__ coords, 
     for (int s = 0; s < steps; ++s) {
       const long long idx = c0 + (long long)s * XB + row;
       const PairRow r = load_row(pairs, P, pexcl, total, idx, natoms);
-      if (!r.valid) continue;
       const long long i = r.i, j = r.j;
-      T dx = coords[3 * i] - coords[3 * j];
-      T dy = coords[3 * i + 1] - coords[3 * j + 1];
-      T dz = coords[3 * i + 2] - coords[3 * j + 2];
-      tff_min_image<T>(box, dx, dy, dz);
-      const T r2 = dx * dx + dy * dy + dz * dz;
-      bool act = r2 <= rc2;
-      long long tix = 0;
-      if (MODE == TFF_PAIR_LJ_TYPES && act) {
-        const long long ti = types[i], tj = types[j];
-        act = ti >= 0 && tj >= 0 && ti < a.ntypes && tj < a.ntypes;
-        tix = act ? ti * a.ntypes + tj : 0;
+      bool act = r.valid;  // (every lane stays to the end of the step: the adds are wave-wide)
+      double v[NC > 0 ? NC : 1], dqj = 0.0;
+      if (act) {
+        T dx = coords[3 * i] - coords[3 * j];
+        T dy = coords[3 * i + 1] - coords[3 * j + 1];
+        T dz = coords[3 * i + 2] - coords[3 * j + 2];
+        tff_min_image<T>(box, dx, dy, dz);
+        const T r2 = dx * dx + dy * dy + dz * dz;
+        act = r2 <= rc2;
+        long long tix = 0;
+        if (MODE == TFF_PAIR_LJ_TYPES && act) {
+          const long long ti = types[i], tj = types[j];
+          act = ti >= 0 && tj >= 0 && ti < a.ntypes && tj < a.ntypes;
+          tix = act ? ti * a.ntypes + tj : 0;
+        }
+        if (act) {
+          const PairEval<T> o = eval_pair<T, MODE, false>(r2, i, j, idx, tix, r.is_excl, a, q, sig, eps);
+          e_acc += (double)o.e;
+          if constexpr (NC > 0) {
+            v[0] = (double)(o.dedr_over_r * dx);
+            v[1] = (double)(o.dedr_over_r * dy);
+            v[2] = (double)(o.dedr_over_r * dz);
+            if constexpr (NC > 3) v[3] = (double)o.dq_i;
+            dqj = (double)o.dq_j;
+          }
+        }
       }
-      if (!act) continue;
-      const PairEval<T> o = eval_pair<T, MODE, false>(r2, i, j, idx, tix, r.is_excl, a, q, sig, eps);
-      e_acc += (double)o.e;
       if constexpr (NC > 0) {
-        any = true;
-        double v[NC];
-        v[0] = (double)(o.dedr_over_r * dx);
-        v[1] = (double)(o.dedr_over_r * dy);
-        v[2] = (double)(o.dedr_over_r * dz);
-        if constexpr (NC > 3) v[3] = (double)o.dq_i;
-        table_add<NC>(tab, (int)i, v, acc);
+        any |= act;
+        unsigned long long miss = __ballot(act && !table_add<NC>(tab, (int)i, v, acc));
+        if (miss) line_add<NC>(miss, (int)i, v, acc, s_w, s_k);
         v[0] = -v[0];
         v[1] = -v[1];
         v[2] = -v[2];
-        if constexpr (NC > 3) v[3] = (double)o.dq_j;
-        table_add<NC>(tab, (int)j, v, acc);
+        if constexpr (NC > 3) v[3] = dqj;
+        miss = __ballot(act && !table_add<NC>(tab, (int)j, v, acc));
+        if (miss) line_add<NC>(miss, (int)j, v, acc, s_w, s_k);
       }
     }
     if constexpr (NC > 0) {
@@ -785,7 +829,7 @@ int run(int mode, const T* coords, long long natoms, const TffBox& box, const lo
     blocks = blocks > XBLOCKS ? XBLOCKS : (blocks < 1 ? 1 : blocks);
   }
   const int nc = chmask & 8u ? 4 : (chmask ? 3 : 0);
-  const size_t lds = nc ? 8 * (size_t)(2 * nc) * XSTRIDE + 4 * (size_t)XSLOTS : 0;
+  const size_t lds = nc ? 8 * (size_t)(2 * nc) * XSTRIDE + 4 * (size_t)XSLOTS + (XB / TFF_WAVE) * (8 * 64 + 4 * 8) : 0;
 #define TFF_LAUNCH_TABLE(M, NC)                                                                                  \
   do {                                                                                                           \
     static std::atomic<unsigned long long> ready{0};                                                             \
