@@ -819,8 +819,8 @@ int run(int mode, const T* coords, long long natoms, const TffBox& box, const lo
   // per-pair gradients (LJ_PAIRS) are written only for the pairs that contribute
   if (gsp) hipLaunchKernelGGL(k_zero_t<T>, dim3(1024), dim3(256), 0, st, gsp, P);
   if (gep) hipLaunchKernelGGL(k_zero_t<T>, dim3(1024), dim3(256), 0, st, gep, P);
-  // the table kernel where only coordinate / charge gradients (or none) are asked for
-  const bool table = !(chmask & 48u) && !tmask && !gsp && !gep && natoms <= 0x7fffffffLL;
+  // the table kernel where only coordinate / charge gradients (or none) are asked for: always for the Coulomb modes
+  const bool table = !(chmask & 48u) && !tmask && !gsp && !gep;
   // rows per chunk: as many steps as leave every workgroup two chunks (small lists spread over the device)
   int steps = (int)((P + PE) / (2LL * XBLOCKS * XB));
   steps = steps < 1 ? 1 : (steps > CHUNK_STEPS ? CHUNK_STEPS : steps);
@@ -845,7 +845,7 @@ int run(int mode, const T* coords, long long natoms, const TffBox& box, const lo
     TFF_LAUNCH_TABLE(M, 3);                                                                                      \
   else if (table)                                                                                                \
     TFF_LAUNCH_TABLE(M, 4);                                                                                      \
-  else                                                                                                           \
+  else if constexpr (M != TFF_PAIR_COUL_EWALD && M != TFF_PAIR_COUL_EWALD_SYM)                                   \
     hipLaunchKernelGGL((k_pair_terms<T, M>), grid, blk, 0, st, coords, pairs, P, pexcl, PE, box, pa, q, sig, eps, \
                        types, natoms, w.e_part, chmask, w.atoms, tmask, w.tab_part, w.tab_ovf, gsp, gep)
   void* tok = tff_prof_begin("pair_terms", st);
@@ -906,6 +906,10 @@ extern "C" int tff_pair_energy(int dtype, int mode, const void* coords, long lon
                                void* forces_accum, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (natoms < 0 || npairs < 0 || npairs_excl < 0 || (npairs > 0 && !pairs) || (npairs_excl > 0 && !pairs_excl)) {
     tff_set_error("tff_pair_energy: invalid pair arguments");
+    return TFF_ERR_ARG;
+  }
+  if (natoms > 0x7fffffffLL) {  // (atom indices are 32-bit in the kernels' tables)
+    tff_set_error("tff_pair_energy: natoms exceeds int32 indexing");
     return TFF_ERR_ARG;
   }
   const bool sym = mode == TFF_PAIR_COUL_EWALD_SYM;
