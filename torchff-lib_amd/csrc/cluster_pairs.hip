@@ -533,7 +533,6 @@ struct Entries {
   long long M;
 };
 
-// lane's atom i, column atom j and skip mask for entry e; false if the entry is padding
 // the atom of a slot, -1 for a slot past the end or an index out of range
 __device__ __forceinline__ int slot_atom(const int* __restrict__ sorted, long long slot, int natoms) {
   if (slot >= natoms) return -1;
@@ -541,6 +540,7 @@ __device__ __forceinline__ int slot_atom(const int* __restrict__ sorted, long lo
   return a >= 0 && a < natoms ? a : -1;
 }
 
+// lane's atom i, column atom j and skip mask for entry e; false if the entry is padding
 __device__ __forceinline__ bool entry_atoms(const Entries& en, long long e, int natoms, int nclusters, int l, int& i,
                                             int& j, unsigned& skip) {
   if (e < en.E) {
@@ -716,14 +716,13 @@ __device__ __forceinline__ void cp_flush(int a, const double (&v)[CpCh<LJG>::N],
 // 150); one column per step by shuffles, a butterfly per gradient and an atomic per atom and channel
 // took 683.  Testing all pairs first and working off each lane's hits, with the column sums in LDS, took
 // 828: the fullest lane of 64 has nearly all 32 columns.
-// BOX: 0 no box, 1 orthorhombic, 2 general.
+// ORTHO: the box is orthorhombic.
 constexpr int CP_CHAIN = 8;
-template <typename T, int GRAD, int BOX>
-__global__ __launch_bounds__(CPB) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 3))) void k_cp_nonbonded(const T* __restrict__ coords, CpGeom g, Entries en, int run,
-                                                      const T* __restrict__ q, const T* __restrict__ sig,
-                                                      const T* __restrict__ eps, double coul, int do_shift, T tol_k,
-                                                      T tol_l, double* __restrict__ e_part,
-                                                      double* __restrict__ acc) {
+template <typename T, int GRAD, bool ORTHO>
+__global__ __launch_bounds__(CPB) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 3))) void k_cp_nonbonded(
+    const T* __restrict__ coords, CpGeom g, Entries en, int run, const T* __restrict__ q, const T* __restrict__ sig,
+    const T* __restrict__ eps, double coul, int do_shift, T tol_k, T tol_l, double* __restrict__ e_part,
+    double* __restrict__ acc) {
   constexpr bool LJG = GRAD == 2;
   constexpr int N = GRAD ? CpCh<LJG>::N : 1;
   __shared__ double s_fl[GRAD ? (CPB / 32) * CPW * (CpCh<LJG>::ST + 1) : 1];
@@ -794,10 +793,10 @@ __global__ __launch_bounds__(CPB) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
           for (int k = 0; k < N; ++k) gj[k] = 0;
           for (int c = 0; c < CP_CHAIN; ++c) {
             T dx = xi - xj, dy = yi - yj, dz = zi - zj;
-            if constexpr (BOX == 1) {  // tff_min_image, its branches taken
+            if constexpr (ORTHO) {  // tff_min_image, its branches taken
               dx *= v0; dy *= v1; dz *= v2;
               dx = (dx - rint(dx)) * b0; dy = (dy - rint(dy)) * b1; dz = (dz - rint(dz)) * b2;
-            } else if constexpr (BOX == 2) {
+            } else {
               tff_min_image<T>(g.box, dx, dy, dz);
             }
             T r2 = dx * dx + dy * dy + dz * dz;
@@ -1322,7 +1321,7 @@ extern "C" int tff_cluster_pairs_nonbonded(int dtype, const void* coords, long l
                          (TT)tol_k, (TT)box_l, w.e_part, w.acc);
     };
     auto pick = [&](auto box) {
-      constexpr int B = decltype(box)::value;
+      constexpr bool B = decltype(box)::value;
       if (grad == 2)
         launch(k_cp_nonbonded<TT, 2, B>);
       else if (grad == 1)
@@ -1330,12 +1329,10 @@ extern "C" int tff_cluster_pairs_nonbonded(int dtype, const void* coords, long l
       else
         launch(k_cp_nonbonded<TT, 0, B>);
     };
-    if (!g.box.periodic)
-      pick(std::integral_constant<int, 0>{});
-    else if (g.box.ortho)
-      pick(std::integral_constant<int, 1>{});
+    if (g.box.ortho)
+      pick(std::true_type{});
     else
-      pick(std::integral_constant<int, 2>{});
+      pick(std::false_type{});
     const CpOut<TT> o{(TT*)energy_out, (TT*)grad_coords, (TT*)grad_charges, (TT*)grad_sigma, (TT*)grad_epsilon,
                       (TT*)forces_accum};
     hipLaunchKernelGGL(k_cp_finish<TT>, blocks(grad ? natoms : 1), dim3(256), 0, stream, (const double*)w.e_part,
