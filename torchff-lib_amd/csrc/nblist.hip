@@ -17,15 +17,17 @@
 // box is too small for 5 cells), counting-sorted by cell, and one workgroup
 // of four waves per home cell walks the half shell of 62 (or 13) neighbour
 // cells plus the home cell, the home atoms and their exclusion partners staged
-// in LDS once and each neighbour cell's atoms staged by the wave that takes
-// it.  The ni x nj candidate block of a cell pair is spread over the 64 lanes,
-// so lane utilisation does not depend on cell occupancy.  Two passes: the
-// first counts each wave's accepted pairs, a scan turns the counts into
-// offsets, the second repeats the walk and writes each wave's pairs from its
-// offset in ballot order (no shared counter: one global atomic per few
-// hundred pairs on a single address cost more than the search itself), so the
-// output order is the same on every call.  The rows past the found count are
-// set to -1 after the search (each output row is written once).
+// in LDS and the shell's atoms staged in LDS in batches.  Each lane takes one
+// shell atom and walks the home atoms, so lane utilisation does not depend on
+// the occupancy of a cell.  Two passes: the first counts each wave's accepted
+// pairs, a scan turns the counts into offsets, the second repeats the walk and
+// writes each wave's pairs from its offset in ballot order (no shared counter:
+// one global atomic per few hundred pairs on a single address cost more than
+// the search itself).  The set of pairs is the same on every call; their order
+// follows that of the atoms within a cell, which the counting sort's atomics
+// set anew on each call (the all-pairs search's order follows its shared
+// counter).  The rows past the found count are set to -1 after the search
+// (each output row is written once).
 
 #include <stdarg.h>
 #include <stdio.h>
@@ -395,6 +397,7 @@ __global__ __launch_bounds__(CP_WAVES * TFF_WAVE) void k_cell_pairs(
   }
   if (!WRITE && lane == 0) wcount[home * CP_WAVES + wv] = (int)pos;
 }
+
 bool choose_grid(const TffBox& box, double cutoff, long long n, CellGrid& g) {
   if (!box.periodic || !(cutoff > 0.0)) return false;
   double w[3];
