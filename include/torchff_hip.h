@@ -193,6 +193,12 @@ int tff_ewald_multipole(int dtype, const void* coords, long long natoms, const d
                         size_t workspace_bytes, tff_stream_t stream);
 
 /* ------------------------------------------------------- cluster pairs */
+/* Symmetric CSR (row_ptr natoms + 1, col 2 num_pairs) of a COO pair list, (2, num_pairs) when two_rows else
+ * (num_pairs, 2): pairs with a negative index are left out; an index >= natoms sets *status (device) to 1.
+ * Each row holds its distinct partners (at most 17) in any order, then -1. */
+size_t tff_exclusions_csr_workspace_bytes(long long natoms);
+int tff_exclusions_csr(const int64_t* pairs, long long num_pairs, int two_rows, long long natoms, int64_t* row_ptr,
+                       int64_t* col, long long* status, void* workspace, size_t workspace_bytes, tff_stream_t stream);
 /* Cluster-pair neighbour list in the reference's format (torchff/nblist.py:260-344
  * build_cluster_pairs / decode_cluster_pairs; csrc/nblist/nblist_cluster_pairs_cuda.cu:18-720) and
  * the nonbonded terms evaluated on it (the schemas commented at
@@ -208,12 +214,6 @@ int tff_ewald_multipole(int dtype, const void* coords, long long natoms, const d
  * flags: 1 = an atom has more than 16 exclusion partners, 2 = a cluster has more than 32
  * exclusion-partner clusters; either makes the list unusable), _emit writes the tensors with the
  * given capacities (-1 padding past E and M) from the same workspace. */
-/* Symmetric CSR (row_ptr natoms + 1, col 2 num_pairs) of a COO pair list, (2, num_pairs) when two_rows else
- * (num_pairs, 2): pairs with a negative index are left out; an index >= natoms sets *status (device) to 1.
- * Each row holds its distinct partners (at most 17) in any order, then -1. */
-size_t tff_exclusions_csr_workspace_bytes(long long natoms);
-int tff_exclusions_csr(const int64_t* pairs, long long num_pairs, int two_rows, long long natoms, int64_t* row_ptr,
-                       int64_t* col, long long* status, void* workspace, size_t workspace_bytes, tff_stream_t stream);
 size_t tff_cluster_pairs_workspace_bytes(long long natoms, const double* box_host, double cutoff, double cell_size);
 int tff_cluster_pairs_build(int dtype, const void* coords, long long natoms, const double* box_host, double cutoff,
                             double cell_size, const int64_t* excl_row_ptr, const int64_t* excl_col,
