@@ -976,9 +976,10 @@ __device__ __forceinline__ V3<TC> entry_steps(unsigned info, int ci, int jg, con
 // time.  The list holds only the j-groups with a partner (2.9 of the 4 of a listed cluster on average in
 // water), so the per-entry work - loads, shift, the sums of F_j, their conversion and the atomics - is
 // not spent on the empty ones; what bounds the kernel is vector issue (about 50 instructions per 8 x 8
-// block with a pair in range, 38 % of whose lanes are).  Measured at 96k atoms, alone: float 143 -> 121 us
-// (5 waves per SIMD), float64 396 -> 256 us (216 registers instead of 310: two waves per SIMD, not one),
-// against one 32 x 32 tile at a time with all 12 F_j components of it reduced in every lane; F_i stays in registers for the whole share, F_j of a quad is summed over the 8 lanes sharing
+// block with a pair in range, 38 % of whose lanes are).  Measured alone: float, 96k atoms, 143 -> 121 us
+// (5 waves per SIMD), float64, 60k atoms, 396 -> 256 us (two waves per SIMD instead of one; 208 with the pair
+// functions of pair_math.h), against one 32 x 32 tile at a time with all 12 F_j components of it reduced in
+// every lane; F_i stays in registers for the whole share, F_j of a quad is summed over the 8 lanes sharing
 // jj and added to the int64 fixed-point accumulators (entry 2 (lane >> 5) + ((lane >> 4) & 1), slot jj;
 // bit 3 picks the components).  Integer sums do not depend on their order and each share is summed
 // in a fixed order, so the results are bitwise reproducible.  Charges are pre-multiplied by the
@@ -1068,8 +1069,8 @@ __global__ __launch_bounds__(TFF_WAVE) __attribute__((amdgpu_waves_per_eu(4))) v
     unsigned long long* __restrict__ facc, ESlots es) {
   // The body needs 89 registers, i.e. 5 waves per SIMD; naming v103 holds it at 4 (104 each) and leaves
   // 96 per SIMD free, so that the workgroups of the reciprocal-space chain find room beside the pair
-  // kernel.  Alone the kernel takes 121 us with 5 waves and 129 with 4 (96k atoms), the whole
-  // evaluation 256 and 243 us; 999k atoms 2.02 and 2.00 ms.
+  // kernel.  Alone the kernel takes 121 us with 5 waves and 129 with 4 (96k atoms); the whole evaluation
+  // 258 with 5 and 256 with 4, at 999k atoms 2.00 and 2.06 ms.
   asm volatile("" ::: "v103");
   pairs_body<float>(ncl_ptr, pl, parts, xyzq, lj, excl_part, ta, facc, es);
 }
@@ -1660,8 +1661,9 @@ __global__ __launch_bounds__(FB) void k_slot_splines(const int* __restrict__ ncl
 // left.  A point gets (X1 Y1 + X2 Y2) Z1 + X2 Y1 Z2 with X1 = w_x M'_x, X2 = M_x, Y1 = M_y, Y2 = w_y M'_y,
 // Z1 = M_z, Z2 = w_z M'_z; weights and derivatives are evaluated again per brick that a stencil meets
 // (some 4 times; a table of both would be read as often).  Charges: wts holds the weights.
-// 96k water atoms, order 5, 96^3: the dipoles 44 us; k_spread_bricks (a search over clusters per brick, one lane
-// per slot, a general double-to-int64 conversion per point) took 251 beside the pair kernel.
+// 96k water atoms, order 5, 96^3: the dipoles alone 44 us, beside the backward's pair kernel 188; k_spread_bricks (a
+// search over clusters per brick, one lane per slot, a general double-to-int64 conversion per point) took 251
+// beside it, the force-matching step 657 us instead of 644.
 constexpr int LIST_ROUND = 256;
 template <int P, bool DIPOLE>
 __global__ __launch_bounds__(LIST_ROUND) void k_spread_lists(const float* __restrict__ wts,
@@ -1884,26 +1886,26 @@ __global__ __launch_bounds__(LIST_ROUND) void k_spread_lists(const float* __rest
               if (iz < nz) atomicAdd(&row[iz * SQ_Z], b);
             }
           }
-          continue;
-        }
-        const float wx = w[ix];
-        float wy[P], wz[P];
+        } else {
+          const float wx = w[ix];
+          float wy[P], wz[P];
 #pragma unroll
-        for (int i = 0; i < P; ++i) {
-          wy[i] = w[P + i];
-          wz[i] = w[2 * P + i];
-        }
+          for (int i = 0; i < P; ++i) {
+            wy[i] = w[P + i];
+            wz[i] = w[2 * P + i];
+          }
 #pragma unroll
-        for (int iy = 0; iy < P; ++iy) {
-          if (iy >= ny) break;
-          const float wab = wx * wy[iy];
-          long long v[P];
+          for (int iy = 0; iy < P; ++iy) {
+            if (iy >= ny) break;
+            const float wab = wx * wy[iy];
+            long long v[P];
 #pragma unroll
-          for (int iz = 0; iz < P; ++iz) v[iz] = (long long)__float2int_rn(wab * wz[iz]);
-          unsigned long long* row = s_q + lz0 * SQ_Z + (ly0 + iy) * SQ_Y + lx;
+            for (int iz = 0; iz < P; ++iz) v[iz] = (long long)__float2int_rn(wab * wz[iz]);
+            unsigned long long* row = s_q + lz0 * SQ_Z + (ly0 + iy) * SQ_Y + lx;
 #pragma unroll
-          for (int iz = 0; iz < P; ++iz)
-            if (iz < nz) atomicAdd(&row[iz * SQ_Z], (unsigned long long)v[iz]);
+            for (int iz = 0; iz < P; ++iz)
+              if (iz < nz) atomicAdd(&row[iz * SQ_Z], (unsigned long long)v[iz]);
+          }
         }
       }
       __syncthreads();
@@ -2359,9 +2361,10 @@ AuxStream g_aux[64];
 // 0: the reciprocal-space chain runs on the caller's stream, in order (a timing aid); 2: the charge
 // spread runs on the caller's stream before the fork, the FFT and the gather on the auxiliary
 // stream; 3: the whole chain runs on the auxiliary stream; 1: 3 below SPREAD_FIRST_ATOMS, 2 from
-// there on.  Measured per evaluation (mixed): 96k atoms 0.309 ms as 3 against 0.312 as 2; 999k
-// atoms 2.616 ms as 3 against 2.533 as 2 (the pair kernel starves a concurrent spread, which
-// then leaves the FFT and the gather to run after it).
+// there on (beside the pair kernel a spread gets few registers and leaves the FFT and the gather to run
+// after it).  Measured per evaluation (mixed, launched one by one, as 3 and as 2): 96k atoms 0.242 and
+// 0.266 ms, 192k 0.453 and 0.433, 300k 0.583 and 0.601, 480k 0.975 and 0.878, 999k 2.06 and 2.07; replayed as a
+// graph 96k 0.260 and 0.279, 192k 0.416 and 0.442.
 constexpr long long SPREAD_FIRST_ATOMS = 300000;
 std::atomic<int> g_overlap{1};
 
@@ -2616,7 +2619,7 @@ int run_fused_grad(const TI* coords, const TI* q, const TI* sig, const TI* eps, 
     };
     if (!reuse) {
       add(w.col_count, ncols + 1);
-        add(status, 2);
+      add(status, 2);
       add(w.slot_orig, nslots);
       // the brick counters of the charge spread (float: the forward's list spread runs again)
       if (w.bcount) add(w.bcount, (long long)w.bg.nb[0] * w.bg.nb[1] * w.bg.nb[2]);
@@ -2903,9 +2906,12 @@ bool g_seen_valid[64];
 
 // a graph is captured and launched for a call on st: by the mode (0: never; 1: float32 arithmetic
 // below SPREAD_FIRST_ATOMS atoms; 2: always), no event timing requested, st not itself being
-// captured (an enclosing capture records the kernels one by one instead).  Mode 1 follows the
-// measurements per evaluation (graph against one by one): 96k atoms mixed 0.294 against 0.304 ms,
-// fp64 0.773 against 0.761, 999k atoms mixed 2.350 against 2.351.
+// captured (an enclosing capture records the kernels one by one instead).  Measured per evaluation in a
+// back-to-back loop (cutoff 0.9 nm, from 192k atoms on 1.0), graph and one by one, us: mixed 900 atoms 145 and
+// 163, 3k 147 and 165, 12k 153 and 160, 60k 194 and 182, 96k 241 and 228, 192k 416 and 453, 300k 580 and 583,
+// 999k 2050 and 2055; fp64 900 atoms 136 and 152, 3k 144 and 155, 12k 174 and 171, 60k 317 and 322, 96k 429 and
+// 449.  (The line was drawn with slower pair kernels: most fp64 boxes would gain by a graph now, mixed ones of 60k
+// to 96k atoms by going without.)
 bool graphs_usable(hipStream_t st, bool f32, long long n) {
   const int mode = g_graphs_mode.load();
   if (mode == 0 || (mode == 1 && !(f32 && n < SPREAD_FIRST_ATOMS)) || tff_prof_active()) return false;
