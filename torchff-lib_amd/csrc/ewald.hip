@@ -14,7 +14,7 @@
 // input precision); one workgroup of 16 waves per (m_x, m_y) line, the lanes of a wave taking the
 // m_z values of a few atoms and the waves a share of the atoms (fixed-order reduction), G S stored per
 // vector; one workgroup per atom for the potential and force, the lanes taking the m_z values and its
-// waves the lines (reading G S through L1 / L2), and wave sums at the end.  Every sum runs in a fixed order, in float64.
+// waves the lines (or the lanes striding over all k; reading G S through L1 / L2), and wave sums at the end.  Every sum runs in a fixed order, in float64.
 
 #include <type_traits>
 
@@ -132,8 +132,10 @@ __global__ __launch_bounds__(EW_WAVES * TFF_WAVE) void k_ewald_structure(EwMp sr
   double kx, ky, kz;
   ew_k(box, mx, my, mz, kx, ky, kz);
   double sr = 0, si = 0;
+  // quadrupoles: four atoms at once spilled (12000 atoms, kmax 16: 3.34 ms, 2.87 one by one)
+  constexpr int UNROLL = RANK < 2 ? 4 : 1;
   if (grp < G) {
-#pragma unroll 4
+#pragma unroll UNROLL
     for (long long j = wv * G + grp; j < n; j += EW_WAVES * G) {
       const CX<T> tx = tab[(0 * n + j) * W + mx + kmax];
       const CX<T> ty = tab[(1 * n + j) * W + my + kmax];
@@ -198,9 +200,14 @@ __device__ __forceinline__ EwAtom ew_atom(const EwMp& m, long long j) {
 // 35 operations per atom and k) and, for few atoms, by the waves in flight: hence several per atom below
 // 8192 atoms.  2700 atoms, dipoles, kmax 10, float64: 38 us; a wave per atom striding over all k, with two
 // integer divisions and a z phase load each, took 51.
+// FLAT: where one line leaves too many lanes idle (33 to EW_FLAT - 1 values of m_z), the lanes stride over all k
+// instead, line and m_z advanced without a division.  12000 atoms, ranks 0, 1, 2, the whole call in ms: kmax 16
+// (33 values) 1.48, 2.09, 4.07, by lines 1.66, 2.39, 4.52; kmax 25 (51) 3.67, 4.98, 9.48, by lines 3.57, 5.10, 9.76; kmax
+// 28 (57) 4.69, 6.34, 12.0, by lines 4.30, 6.12, 11.8.
 constexpr int EW_AWAVES = 8;
+constexpr int EW_FLAT = 53;
 
-template <typename T, int RANK>
+template <typename T, int RANK, bool FLAT>
 __global__ __launch_bounds__(EW_AWAVES * TFF_WAVE) void k_ewald_atoms(EwMp src, EwMp con, long long n, int kmax,
                                                                       TffBox box, double alpha, int nlines,
                                                                       const CX<T>* __restrict__ tab,
@@ -234,54 +241,74 @@ __global__ __launch_bounds__(EW_AWAVES * TFF_WAVE) void k_ewald_atoms(EwMp src, 
   const CX<T>* tx = tab + (0 * n + i) * W;
   const CX<T>* ty = tab + (1 * n + i) * W;
   double sar = 0, fa[3] = {0, 0, 0}, eg[6] = {0, 0, 0, 0, 0, 0}, fk[3] = {0, 0, 0};
-  const int grp = lane / W, h = lane - grp * W, mz = h - kmax;
-  if (grp < G) {
-    const CX<T> az_ = tab[(2 * n + i) * W + h];
-    const double zx = box.inv[2] * mz, zy = box.inv[5] * mz, zz = box.inv[8] * mz;
-    const float inv_w = 1.0f / (float)W;
+  const float inv_w = 1.0f / (float)W;
+  const double2* GS = reinterpret_cast<const double2*>(S);  // G S (0 outside the half space)
+  // vector (line, m_z): z phase az_, m_z's part of k zx, zy, zz
+  auto step = [&](int line, const CX<T>& az_, double zx, double zy, double zz, const double2& Sk) {
+    // line_of with the division by W in float (exact for fewer than 2^20 lines)
+    const int t = line - (kmax + 1), row = (int)(((float)t + 0.5f) * inv_w);
+    const int mx = t < 0 ? 0 : 1 + row, my = t < 0 ? line : t - row * W - kmax;
+    const CX<T> ax_ = tx[mx + kmax], ay_ = ty[my + kmax];
+    const double ax = (double)ax_.x * ay_.x - (double)ax_.y * ay_.y,
+                 ay = (double)ax_.x * ay_.y + (double)ax_.y * ay_.x;
+    const double c = ax * az_.x - ay * az_.y, s = ax * az_.y + ay * az_.x;
+    const double kx = box.inv[0] * mx + box.inv[1] * my + zx;
+    const double ky = box.inv[3] * mx + box.inv[4] * my + zy;
+    const double kz = box.inv[6] * mx + box.inv[7] * my + zz;
+    const double Ar = Sk.x * c + Sk.y * s, Ai = Sk.x * s - Sk.y * c;
+    sar += Ar;
+    fa[0] += kx * Ai;
+    fa[1] += ky * Ai;
+    fa[2] += kz * Ai;
+    if (fgrad) {
+      eg[0] += Ar * kx * kx;
+      eg[1] += Ar * ky * ky;
+      eg[2] += Ar * kz * kz;
+      eg[3] += Ar * kx * ky;
+      eg[4] += Ar * kx * kz;
+      eg[5] += Ar * ky * kz;
+    }
+    if (RANK >= 1 && forces) {  // (of charges alone: q times the field's sums)
+      double lr = X.q, li = 0.0;
+      if (xp) li = 2.0 * M_PI * (kx * X.p[0] + ky * X.p[1] + kz * X.p[2]);
+      if (xt) {
+        const double kv[3] = {kx, ky, kz};
+        double acc = 0.0;
+#pragma unroll
+        for (int x = 0; x < 3; ++x)
+#pragma unroll
+          for (int y = 0; y < 3; ++y) acc += kv[x] * X.th[3 * x + y] * kv[y];
+        lr -= 4.0 * M_PI * M_PI / 3.0 * acc;
+      }
+      const double im = lr * Ai + li * Ar;
+      fk[0] += kx * im;
+      fk[1] += ky * im;
+      fk[2] += kz * im;
+    }
+  };
+  if constexpr (FLAT) {
+    const CX<T>* tz = tab + (2 * n + i) * W;
+    const int stride = nw * TFF_WAVE, dl = stride / W, dh = stride - dl * W;
+    int k = wv * TFF_WAVE + lane, line = k / W, h = k - line * W;
 #pragma unroll 2
-    for (int line = wv * G + grp; line < nlines; line += nw * G) {
-      // line_of with the division by W in float (exact for fewer than 2^20 lines)
-      const int t = line - (kmax + 1), row = (int)(((float)t + 0.5f) * inv_w);
-      const int mx = t < 0 ? 0 : 1 + row, my = t < 0 ? line : t - row * W - kmax;
-      const CX<T> ax_ = tx[mx + kmax], ay_ = ty[my + kmax];
-      const double2 Sk = reinterpret_cast<const double2*>(S)[(size_t)line * W + h];  // G S (0 outside the half space)
-      const double ax = (double)ax_.x * ay_.x - (double)ax_.y * ay_.y,
-                   ay = (double)ax_.x * ay_.y + (double)ax_.y * ay_.x;
-      const double c = ax * az_.x - ay * az_.y, s = ax * az_.y + ay * az_.x;
-      const double kx = box.inv[0] * mx + box.inv[1] * my + zx;
-      const double ky = box.inv[3] * mx + box.inv[4] * my + zy;
-      const double kz = box.inv[6] * mx + box.inv[7] * my + zz;
-      const double Ar = Sk.x * c + Sk.y * s, Ai = Sk.x * s - Sk.y * c;
-      sar += Ar;
-      fa[0] += kx * Ai;
-      fa[1] += ky * Ai;
-      fa[2] += kz * Ai;
-      if (fgrad) {
-        eg[0] += Ar * kx * kx;
-        eg[1] += Ar * ky * ky;
-        eg[2] += Ar * kz * kz;
-        eg[3] += Ar * kx * ky;
-        eg[4] += Ar * kx * kz;
-        eg[5] += Ar * ky * kz;
+    for (; k < nlines * W; k += stride) {
+      const int mz = h - kmax;
+      step(line, tz[h], box.inv[2] * mz, box.inv[5] * mz, box.inv[8] * mz, GS[k]);
+      line += dl;
+      h += dh;
+      if (h >= W) {
+        h -= W;
+        ++line;
       }
-      if (RANK >= 1 && forces) {  // (of charges alone: q times the field's sums)
-        double lr = X.q, li = 0.0;
-        if (xp) li = 2.0 * M_PI * (kx * X.p[0] + ky * X.p[1] + kz * X.p[2]);
-        if (xt) {
-          const double kv[3] = {kx, ky, kz};
-          double acc = 0.0;
-#pragma unroll
-          for (int x = 0; x < 3; ++x)
-#pragma unroll
-            for (int y = 0; y < 3; ++y) acc += kv[x] * X.th[3 * x + y] * kv[y];
-          lr -= 4.0 * M_PI * M_PI / 3.0 * acc;
-        }
-        const double im = lr * Ai + li * Ar;
-        fk[0] += kx * im;
-        fk[1] += ky * im;
-        fk[2] += kz * im;
-      }
+    }
+  } else {
+    const int grp = lane / W, h = lane - grp * W, mz = h - kmax;
+    if (grp < G) {
+      const CX<T> az = tab[(2 * n + i) * W + h];
+      const double zx = box.inv[2] * mz, zy = box.inv[5] * mz, zz = box.inv[8] * mz;
+#pragma unroll 2
+      for (int line = wv * G + grp; line < nlines; line += nw * G)
+        step(line, az, zx, zy, zz, GS[(size_t)line * W + h]);
     }
   }
   auto put = [&](int k, double v) {
@@ -358,9 +385,12 @@ int run_ewald(const T* coords, const EwMp& src, const EwMp& con, long long n, co
     constexpr int R = decltype(rank)::value;
     hipLaunchKernelGGL((k_ewald_structure<T, R>), dim3(nlines), dim3(EW_WAVES * TFF_WAVE), 0, st, src, n, kmax, box,
                        alpha, (const CX<T>*)w.tab, w.S, w.eline);
-    hipLaunchKernelGGL((k_ewald_atoms<T, R>), dim3(g3), dim3(nw * TFF_WAVE), 0, st, src, con, n, kmax, box, alpha,
-                       nlines, (const CX<T>*)w.tab, (const double*)w.S, (const double*)w.eline, energy, pot, field,
-                       fgrad, forces);
+    auto atoms = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(g3), dim3(nw * TFF_WAVE), 0, st, src, con, n, kmax, box, alpha, nlines,
+                         (const CX<T>*)w.tab, (const double*)w.S, (const double*)w.eline, energy, pot, field, fgrad,
+                         forces);
+    };
+    atoms(2 * W > TFF_WAVE && W < EW_FLAT ? k_ewald_atoms<T, R, true> : k_ewald_atoms<T, R, false>);
   };
   if (src.th || con.th)
     go(std::integral_constant<int, 2>{});
