@@ -501,6 +501,9 @@ constexpr int CHUNK_STEPS = 4;       // rows per thread and chunk
 constexpr int XROWS = 8;             // the lanes of a wave take rows this far apart: a run of rows of one atom then
                                      // falls to several waves instead of colliding in one instruction (685 us at 1)
 constexpr int XBLOCKS = 512;
+// energy alone: no table, so as many workgroups as the device holds, each wave on consecutive rows (96k atoms, float64,
+// 27M rows: 227 us, as with gradients 293; float32 195 and 245)
+constexpr int XBLOCKS_E = 2048;
 constexpr int PROBES = 12;
 
 // v -> words as split_words, by adding 1.5 2^52 (the integer is then the low mantissa bits): three fma and an
@@ -592,7 +595,7 @@ __global__ __launch_bounds__(XB) void k_pair_xyzq(const T* __restrict__ coords, 
   extern __shared__ __align__(16) long long s_tab[];  // table words, then keys, then the waves' lines and their atoms
   const AtomTable tab{reinterpret_cast<int*>(s_tab + 2 * NC * XSTRIDE), s_tab};
   const int t = threadIdx.x, lane = t & (TFF_WAVE - 1), wv = t / TFF_WAVE;
-  const int row = (wv / XROWS) * TFF_WAVE * XROWS + lane * XROWS + wv % XROWS;
+  const int row = NC ? (wv / XROWS) * TFF_WAVE * XROWS + lane * XROWS + wv % XROWS : t;
   long long* const s_w = s_tab + 2 * NC * XSTRIDE + XSLOTS / 2 + 64 * wv;
   int* const s_k = reinterpret_cast<int*>(s_tab + 2 * NC * XSTRIDE + XSLOTS / 2 + 64 * (XB / TFF_WAVE)) + 8 * wv;
   if (NC) {
@@ -821,14 +824,15 @@ int run(int mode, const T* coords, long long natoms, const TffBox& box, const lo
   if (gep) hipLaunchKernelGGL(k_zero_t<T>, dim3(1024), dim3(256), 0, st, gep, P);
   // the table kernel where only coordinate / charge gradients (or none) are asked for: always for the Coulomb modes
   const bool table = !(chmask & 48u) && !tmask && !gsp && !gep;
+  const int nc = chmask & 8u ? 4 : (chmask ? 3 : 0);
+  const long long max_blocks = nc ? XBLOCKS : XBLOCKS_E;
   // rows per chunk: as many steps as leave every workgroup two chunks (small lists spread over the device)
-  int steps = (int)((P + PE) / (2LL * XBLOCKS * XB));
+  int steps = (int)((P + PE) / (2LL * max_blocks * XB));
   steps = steps < 1 ? 1 : (steps > CHUNK_STEPS ? CHUNK_STEPS : steps);
   if (table) {
     blocks = (P + PE + (long long)steps * XB - 1) / ((long long)steps * XB);
-    blocks = blocks > XBLOCKS ? XBLOCKS : (blocks < 1 ? 1 : blocks);
+    blocks = blocks > max_blocks ? max_blocks : (blocks < 1 ? 1 : blocks);
   }
-  const int nc = chmask & 8u ? 4 : (chmask ? 3 : 0);
   const size_t lds = nc ? 8 * (size_t)(2 * nc) * XSTRIDE + 4 * (size_t)XSLOTS + (XB / TFF_WAVE) * (8 * 64 + 4 * 8) : 0;
 #define TFF_LAUNCH_TABLE(M, NC)                                                                                  \
   do {                                                                                                           \
